@@ -46,7 +46,7 @@ _lib = None
 
 def build() -> None:
     subprocess.run(["make", "-s", "-C", HERE, "libasohf_oracle.so"], check=True)
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/grids.f"):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True,
                        stdout=subprocess.DEVNULL)
 
