@@ -152,19 +152,12 @@ struct PipeArgs {
   unsigned long long* cursor;
   unsigned long long* bsum;
   unsigned* nitems;
-  unsigned* nsplit;
   unsigned long long* item_off;
-  unsigned long long* split_off;
-  int* split;
-  unsigned* is_split;
-  unsigned long long* split_rank;
-  int* split_tiles;
   double* grid_mass;
   long long nblk;
   long long nkeys;
-  unsigned long long cap_entries;   // entries, items and split-tile slots the buffers hold
+  unsigned long long cap_entries;   // entries and items the buffers hold
   unsigned long long cap_items;
-  unsigned long long cap_split;
   int ntiles, chunk, chunk_wide, red, grid, block, cus, elem;
   // TSC binning along the hierarchy
   unsigned* item_pairs;
@@ -182,8 +175,8 @@ struct asohf_ctx {
   asohf_tune tune{{16, 8, 8}, 256, 4096, 16};
   HostPlan plan;
   DBuf plan_blob;
-  DBuf cnt, start, cursor, bsum, counters, stiles, isplit, srank, nitems, split, tmass, entries, items, scratch;
-  DBuf flags, idx, pool, pool_off, pool_nk, blk_pairs, blk_mmax, nsplit, item_off, split_off;
+  DBuf cnt, start, cursor, bsum, counters, nitems, tmass, entries, items, scratch;
+  DBuf flags, idx, pool, pool_off, pool_nk, blk_pairs, blk_mmax, item_off;
   DBuf elist, eoff, ecount;
   DBuf ipairs;                             // members found per work item (TSC hierarchy binning)
   void* noalloc = nullptr;                 // this device's scratch array of order.hip (device address)
@@ -201,7 +194,6 @@ struct asohf_ctx {
   uint64_t hier_key = 0;
   long long hier_items[kNLevels + 2] = {};
   long long hier_nitems = 0;
-  unsigned long long hier_nsplit = 0;
   hipGraphExec_t gexec = nullptr;   // the captured batched build and the arguments it holds
   PipeArgs gkey;
   DBuf h_in[4], h_out[2], h_mass;    // device copies for the host entry point
@@ -209,7 +201,7 @@ struct asohf_ctx {
   Counters* hcount = nullptr;          // pinned
   unsigned long long* hscalar = nullptr;
   hipEvent_t ev[9] = {};   // 0 start, 1 count pass, 2 scatter start, 3 scatter end, 4 deposit start,
-                           // 8 deposit end, 5 split tiles summed, 6 end, 7 the caller's stream
+                           // 8 deposit end, 5 output cells written, 6 end, 7 the caller's stream
                            // before a graph launch
   asohf_stats stats{};
   bool stats_pending = false;
@@ -802,15 +794,11 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   HIPCHK(ctx->cursor.ensure(sizeof(unsigned long long) * std::max<long long>(nkeys, 1)), "allocating cursors");
   HIPCHK(ctx->bsum.ensure(sizeof(unsigned long long) * scan_scratch_elems(nkeys)), "allocating scan");
   HIPCHK(ctx->counters.ensure(sizeof(Counters)), "allocating counters");
-  HIPCHK(ctx->stiles.ensure(sizeof(int) * std::max(ntiles, 1)), "allocating tile state");
-  HIPCHK(ctx->isplit.ensure(sizeof(unsigned) * std::max(ntiles, 1)), "allocating tile state");
-  HIPCHK(ctx->srank.ensure(sizeof(unsigned long long) * (ntiles + 1)), "allocating tile state");
   HIPCHK(ctx->nitems.ensure(sizeof(unsigned) * std::max(ntiles, 1)), "allocating tile state");
-  HIPCHK(ctx->nsplit.ensure(sizeof(unsigned) * std::max(ntiles, 1)), "allocating tile state");
   HIPCHK(ctx->item_off.ensure(sizeof(unsigned long long) * (ntiles + 1)), "allocating tile state");
-  HIPCHK(ctx->split_off.ensure(sizeof(unsigned long long) * (ntiles + 1)), "allocating tile state");
-  HIPCHK(ctx->split.ensure(sizeof(int) * std::max(ntiles, 1)), "allocating tile state");
   HIPCHK(ctx->tmass.ensure(sizeof(double) * std::max(ntiles, 1)), "allocating tile sums");
+  HIPCHK(ctx->scratch.ensure((size_t)std::max(ntiles, 1) * exchange_cells(a.P.tile) * a.elem),
+         "allocating exchange cells");
   // saved per-block tables: sized from the previous call (a block whose table
   // does not fit its sub-pool recounts in the scatter pass)
   const long long pool_cap = std::max<long long>(ctx->pool_want + ctx->pool_want / 8, 256 * nblk);
@@ -843,13 +831,7 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   a.cursor = ctx->cursor.as<unsigned long long>();
   a.bsum = ctx->bsum.as<unsigned long long>();
   a.nitems = ctx->nitems.as<unsigned>();
-  a.nsplit = ctx->nsplit.as<unsigned>();
   a.item_off = ctx->item_off.as<unsigned long long>();
-  a.split_off = ctx->split_off.as<unsigned long long>();
-  a.split = ctx->split.as<int>();
-  a.is_split = ctx->isplit.as<unsigned>();
-  a.split_rank = ctx->srank.as<unsigned long long>();
-  a.split_tiles = ctx->stiles.as<int>();
   a.grid_mass = grid_mass;
   a.chunk = std::max(ctx->tune.chunk, 64);
   // wide table-mode entries: a tile's classes are deposited in the
@@ -862,9 +844,8 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   a.block = ctx->tune.block;
   a.grid = std::max(1, ctx->cus * waves / std::max(a.block / 64, 1));
   a.D.nitems_tile = ctx->nitems.as<int>();
-  a.D.split_slot = ctx->split.as<int>();
-  a.D.split_tiles = ctx->stiles.as<int>();
-  a.D.n_split_tiles = ctx->srank.as<unsigned long long>() + ntiles;
+  a.D.start = a.start;
+  a.D.scratch = ctx->scratch.p;
   a.D.C = a.C;
   a.D.u1 = u1;
   a.D.u11 = u11;
@@ -876,13 +857,10 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
 
 // the buffers sized by the planning totals, as they are now
 static void bind_sized(asohf_ctx* ctx, PipeArgs& a) {
-  const int T = a.P.tile[0] * a.P.tile[1] * a.P.tile[2];
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
-  a.D.scratch = ctx->scratch.p;
   a.cap_entries = ctx->entries.cap / sizeof(int4);
   a.cap_items = ctx->items.cap / sizeof(Item);
-  a.cap_split = ctx->scratch.cap / ((size_t)T * a.elem);
 }
 
 // count pass: per-(tile, kind) counts, block sums, offsets and the item plan
@@ -892,30 +870,26 @@ static asohf_status enqueue_count(asohf_ctx* ctx, const PipeArgs& a, hipStream_t
   HIPCHK(launch_count(a.P, a.A, a.cnt, a.C, a.BT, a.cus, s), "count kernel");
   if (a.A.n > 0) HIPCHK(launch_reduce_blocks(a.BT, bin_blocks(a.A.n), a.C, a.cus, s), "block sums");
   HIPCHK(launch_scan(a.cnt, a.nkeys, a.bsum, a.start, a.cursor, s), "scan");
-  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, a.chunk_wide, a.nitems, a.nsplit, a.is_split, s),
+  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, a.chunk_wide, a.nitems, s),
          "planning items");
   HIPCHK(launch_scan(a.nitems, a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
-  HIPCHK(launch_scan(a.nsplit, a.ntiles, a.bsum, a.split_off, nullptr, s), "split offsets");
-  HIPCHK(launch_scan(a.is_split, a.ntiles, a.bsum, a.split_rank, nullptr, s), "split tiles");
   return ASOHF_OK;
 }
 
 // gate, scatter, item plan, persistent deposit, grid sums; events between the
 // phases unless the sequence is being captured
 static asohf_status enqueue_deposit(asohf_ctx* ctx, const PipeArgs& a, hipStream_t s, bool events) {
-  HIPCHK(launch_gate(a.start + a.nkeys, a.item_off + a.ntiles, a.split_off + a.ntiles, a.cap_entries,
-                     a.cap_items, a.cap_split, a.C, s), "gate");
+  HIPCHK(launch_gate(a.start + a.nkeys, a.item_off + a.ntiles, a.cap_entries, a.cap_items, a.C, s), "gate");
   if (events) HIPCHK(hipEventRecord(ctx->ev[2], s), "event");
   HIPCHK(launch_scatter(a.P, a.A, a.cursor, const_cast<int4*>(a.D.entries), a.cap_entries, a.BT, a.C, a.cus, s), "scatter kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[3], s), "event");
-  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.chunk_wide, a.item_off, a.split_off, a.split_rank,
-                           const_cast<Item*>(a.D.items), a.split, a.split_tiles, a.D.tile_mass_i, a.C, s),
+  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.chunk_wide, a.item_off, const_cast<Item*>(a.D.items), a.C, s),
          "writing items");
   HIPCHK(launch_zero_split(a.P, a.D, a.red, a.cus, s), "clearing split tiles");
   if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
   HIPCHK(launch_deposit(a.P, a.D, a.red, a.grid, a.block, s), "deposit kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[8], s), "event");
-  HIPCHK(launch_split_reduce(a.P, a.D, a.red, a.cus, s), "split tiles");
+  HIPCHK(launch_combine(a.P, a.D, a.red, a.cus, s), "output cells");
   if (events) HIPCHK(hipEventRecord(ctx->ev[5], s), "event");
   if (a.grid_mass) HIPCHK(launch_grid_sums(a.P, a.D, a.red, a.grid_mass, s), "grid sums");
   return ASOHF_OK;
@@ -959,22 +933,16 @@ static asohf_status run_exact(asohf_ctx* ctx, const asohf_opts& o, const Parts& 
          "reading totals");
   HIPCHK(hipMemcpyAsync(ctx->hscalar + 1, a.item_off + a.ntiles, sizeof(unsigned long long),
                         hipMemcpyDeviceToHost, s), "reading totals");
-  HIPCHK(hipMemcpyAsync(ctx->hscalar + 2, a.split_off + a.ntiles, sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, s), "reading totals");
   HIPCHK(hipStreamSynchronize(s), "count pass");
   Counters hc = *ctx->hcount;
   hc.n_entries = ctx->hscalar[0];
   hc.n_items = ctx->hscalar[1];
-  hc.n_split = ctx->hscalar[2];
   st = decode_err(ctx, hc.err);
   if (st != ASOHF_OK) return st;
   if (hc.n_items >= (1ull << 31)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^31 work items");
   note_pool(ctx, hc);
-  const int T = a.P.tile[0] * a.P.tile[1] * a.P.tile[2];
   HIPCHK(ctx->entries.ensure(sizeof(int4) * std::max<unsigned long long>(hc.n_entries, 1)), "allocating entries");
   HIPCHK(ctx->items.ensure(sizeof(Item) * std::max<unsigned long long>(hc.n_items, 1)), "allocating work items");
-  HIPCHK(ctx->scratch.ensure((size_t)std::max<unsigned long long>(hc.n_split, 1) * T * a.elem),
-         "allocating split-tile scratch");
   bind_sized(ctx, a);
   a.grid = (int)std::min<long long>(a.grid, std::max<unsigned long long>(hc.n_items, 1));
   a.D.n_queues = std::min(kQueues, a.grid);
@@ -1003,49 +971,35 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   HostPlan& H = ctx->plan;
   HIPCHK(launch_fill_u32((unsigned*)a.C, 0u, sizeof(Counters) / 4, s), "clearing counters");
   HIPCHK(launch_fill_u32(a.cnt, 0u, a.nkeys, s), "clearing counts");
-  // a member's home-tile entry counts under key 2t, its others under 2t + 1
-  Plan pc = a.P;
-  pc.home_split = 1;
-  HIPCHK(launch_count(pc, a.A, a.cnt, a.C, a.BT, a.cus, s), "count kernel");
+  HIPCHK(launch_count(a.P, a.A, a.cnt, a.C, a.BT, a.cus, s), "count kernel");
   HIPCHK(launch_count_to_capacity(a.cnt, a.nkeys, a.cus, s), "capacities");
   HIPCHK(launch_scan(a.cnt, a.nkeys, a.bsum, a.start, a.cursor, s), "scan");
-  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, 0, a.nitems, a.nsplit, a.is_split, s),
+  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, 0, a.nitems, s),
          "planning items");
   HIPCHK(launch_scan(a.nitems, a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
-  HIPCHK(launch_scan(a.nsplit, a.ntiles, a.bsum, a.split_off, nullptr, s), "split offsets");
-  HIPCHK(launch_scan(a.is_split, a.ntiles, a.bsum, a.split_rank, nullptr, s), "split tiles");
   const int nl = a.P.nl;
   HIPCHK(hipMemcpyAsync(ctx->hcount, a.C, sizeof(Counters), hipMemcpyDeviceToHost, s), "reading counters");
   HIPCHK(hipMemcpyAsync(ctx->hscalar, a.start + a.nkeys, sizeof(unsigned long long), hipMemcpyDeviceToHost, s),
          "reading totals");
-  HIPCHK(hipMemcpyAsync(ctx->hscalar + 1, a.split_off + a.ntiles, sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, s), "reading totals");
   for (int l = 0; l <= nl + 1; ++l)
-    HIPCHK(hipMemcpyAsync(ctx->hscalar + 2 + l, a.item_off + H.level_tile0[l], sizeof(unsigned long long),
+    HIPCHK(hipMemcpyAsync(ctx->hscalar + 1 + l, a.item_off + H.level_tile0[l], sizeof(unsigned long long),
                           hipMemcpyDeviceToHost, s), "reading item offsets");
   HIPCHK(hipStreamSynchronize(s), "count pass");
   asohf_status st = decode_err(ctx, ctx->hcount->err);
   if (st != ASOHF_OK) return st;
   const unsigned long long cap_entries = ctx->hscalar[0];
-  const unsigned long long nsplit = ctx->hscalar[1];
-  const long long n_items = (long long)ctx->hscalar[2 + nl + 1];
+  const long long n_items = (long long)ctx->hscalar[1 + nl + 1];
   if (n_items >= (1ll << 31)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^31 work items");
   if (cap_entries >= (1ull << 40)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^40 tile entries");
-  for (int l = 0; l <= nl + 1; ++l) ctx->hier_items[l] = (long long)ctx->hscalar[2 + l];
-  const int T = a.P.tile[0] * a.P.tile[1] * a.P.tile[2];
+  for (int l = 0; l <= nl + 1; ++l) ctx->hier_items[l] = (long long)ctx->hscalar[1 + l];
   HIPCHK(ctx->entries.ensure(sizeof(int4) * std::max<unsigned long long>(cap_entries, 1)), "allocating entries");
   HIPCHK(ctx->items.ensure(sizeof(Item) * std::max<long long>(n_items, 1)), "allocating work items");
-  HIPCHK(ctx->scratch.ensure((size_t)std::max<unsigned long long>(nsplit, 1) * T * a.elem),
-         "allocating split-tile scratch");
   HIPCHK(ctx->ipairs.ensure(sizeof(unsigned) * std::max<long long>(n_items, 1)), "allocating item sums");
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
-  a.D.scratch = ctx->scratch.p;
-  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, 0, a.item_off, a.split_off, a.split_rank,
-                           const_cast<Item*>(a.D.items), a.split, a.split_tiles, a.D.tile_mass_i, a.C, s),
+  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, 0, a.item_off, const_cast<Item*>(a.D.items), a.C, s),
          "writing items");
   ctx->hier_nitems = n_items;
-  ctx->hier_nsplit = nsplit;
   return ASOHF_OK;
 }
 
@@ -1053,9 +1007,7 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
 static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
-  a.D.scratch = ctx->scratch.p;
   a.D.cursor = a.cursor;
-  a.D.start = a.start;
   a.item_pairs = ctx->ipairs.as<unsigned>();
   a.n_items = ctx->hier_nitems;
   for (int l = 0; l <= kNLevels + 1; ++l) a.lvl_items[l] = ctx->hier_items[std::min(l, a.P.nl + 1)];
@@ -1066,7 +1018,7 @@ static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
 }
 
 // One call on the planned capacities: base-grid binning, one emission pass
-// per level, the persistent deposit over every item, the split tiles, the
+// per level, the persistent deposit over every item, the output cells, the
 // grid sums and the call's statistics; no host round trip (graph-capturable).
 static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t s, bool events) {
   HIPCHK(launch_fill_u32((unsigned*)a.C, 0u, sizeof(Counters) / 4, s), "clearing counters");
@@ -1091,7 +1043,7 @@ static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t 
   if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
   HIPCHK(launch_deposit(a.P, a.D, a.red, a.grid, a.block, s), "deposit kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[8], s), "event");
-  HIPCHK(launch_split_reduce(a.P, a.D, a.red, a.cus, s), "split tiles");
+  HIPCHK(launch_combine(a.P, a.D, a.red, a.cus, s), "output cells");
   if (events) HIPCHK(hipEventRecord(ctx->ev[5], s), "event");
   if (a.grid_mass) HIPCHK(launch_grid_sums(a.P, a.D, a.red, a.grid_mass, s), "grid sums");
   HIPCHK(launch_hier_stats(a.item_pairs, a.n_items, a.start, a.cursor, a.nkeys, a.C, a.cus, s), "statistics");
@@ -1347,9 +1299,9 @@ void asohf_hip_destroy(asohf_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
-  DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax, &ctx->nsplit,
-                  &ctx->item_off, &ctx->split_off, &ctx->plan_blob, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum, &ctx->counters,
-                  &ctx->stiles, &ctx->isplit, &ctx->srank, &ctx->nitems, &ctx->split, &ctx->tmass, &ctx->entries, &ctx->items,
+  DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
+                  &ctx->item_off, &ctx->plan_blob, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum, &ctx->counters,
+                  &ctx->nitems, &ctx->tmass, &ctx->entries, &ctx->items,
                   &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1], &ctx->h_in[2],
                   &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0], &ctx->ord[1],
                   &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount, &ctx->sp_k[0],
@@ -2302,9 +2254,9 @@ asohf_status asohf_hip_release_workspaces(asohf_ctx* ctx) {
   HIPCHK(hipStreamSynchronize(ctx->stream), "waiting for the context's stream");
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   ctx->gexec = nullptr;
-  DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax, &ctx->nsplit,
-                  &ctx->item_off, &ctx->split_off, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum,
-                  &ctx->stiles, &ctx->isplit, &ctx->srank, &ctx->nitems, &ctx->split, &ctx->tmass, &ctx->entries,
+  DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
+                  &ctx->item_off, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum,
+                  &ctx->nitems, &ctx->tmass, &ctx->entries,
                   &ctx->items, &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1],
                   &ctx->h_in[2], &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0],
                   &ctx->ord[1], &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount,

@@ -1,24 +1,23 @@
 // hier.hip -- TSC binning along the patch hierarchy (gfx950).
 //
-// The batched TSC build bins each (particle, grid) member into the tiles its
-// 27-cell stencil touches.  Instead of testing every particle against a hash
-// of every level's patch boxes, the binning follows the hierarchy:
+// The batched TSC build bins each (particle, grid) member into the tile that
+// holds its centre cell (clamped into the grid); what its 27-cell stencil
+// spills over the tile's border is exchanged between tiles after the deposit.
+// Instead of testing every particle against a hash of every level's patch
+// boxes, the binning follows the hierarchy:
 //
 //   bin_base_tsc  particles -> base-grid tile entries (16 B: x, y, z, m);
 //                 every particle is a member of the base grid
-//                 (grids.f:1159-1246), one entry per base tile its stencil
-//                 touches (1 to 8)
-//   emit_tsc      for one level at a time: the entries of a level-l tile whose
-//                 particle has its home cell in that tile (its clamped cell
-//                 index lies there, so each member of a grid is visited once)
-//                 are tested against the patch boxes of the tile's target
+//                 (grids.f:1159-1246)
+//   emit_tsc      for one level at a time: the entries of a level-l tile are
+//                 tested against the patch boxes of the tile's target
 //                 list: the patches whose membership box lies inside this
 //                 grid's box (found on the host in FP32, the values the
 //                 device compares), so every member of such a patch is a
-//                 member of this grid and has exactly one home entry here.
-//                 A member gets entries in the tiles of its stencil in that
-//                 patch, exactly as the reference's strict box test and index
-//                 expressions give them (grids.f:1294-1323).
+//                 member of this grid and has exactly one entry here.
+//                 A member gets its entry in that patch, exactly as the
+//                 reference's strict box test and index expressions give it
+//                 (grids.f:1294-1323).
 //
 // Entries go to per-tile ranges whose capacities come from an exact count
 // pass (the first call on a geometry, or after an overflow): every workgroup
@@ -38,7 +37,6 @@ constexpr int kHbThreads = 256;
 constexpr int kHbPer = 2;                        // particles per thread
 constexpr int kHbChunk = kHbThreads * kHbPer;    // particles per bin_base workgroup (< 2^16)
 constexpr int kHbCap = 1024;                     // LDS key slots (power of two, < 2^16)
-constexpr int kHbWList = 384;                    // list words per wave
 constexpr int kHbProbe = 32;
 constexpr int kEmThreads = 256;
 constexpr int kEmPer = 2;                        // entries per thread and round
@@ -75,13 +73,6 @@ __device__ __forceinline__ int slot_insert(int* keys, int k) {
   return -1;
 }
 
-// c / e for 0 <= c <= 26 and e in {1, 2, 3} (the tiles of a 3-cell stencil
-// per axis), by a multiply and a shift: c * 86 / 256 lies within 0.07 below
-// c / 3 there, and c / 3 is never within 0.07 above an integer
-__device__ __forceinline__ int div_small(int c, int e) {
-  return (c * (e == 1 ? 256 : (e == 2 ? 128 : 86))) >> 8;
-}
-
 __device__ __forceinline__ void set_overflow(Counters* C) {
   C->overflow = 1u;
   C->n_items_eff = 0u;   // the deposit of this call then does nothing
@@ -116,39 +107,19 @@ __global__ void __launch_bounds__(256) count_to_capacity(unsigned* cnt, long lon
   }
 }
 
-// The position of one emission per lane that wants one (key = destination
-// tile key) in its key's range of the workgroup's round: the lane finds the
-// key's table slot and adds 1 to its count, whose old value is the position.
-// Lanes of a wave with the same key meet at one LDS address, which the LDS
-// serialises at less cost than grouping the lanes first (ballots and lane
-// reads per group, measured slower with 1 to 8 groups).  h = -1 when the
-// table is full (the emission is then not counted).
+// The position of an emission (key = destination tile key) in its key's range
+// of the workgroup's round: the lane finds the key's table slot h and adds 1
+// to its count, whose old value is the position.  Lanes of a wave with the
+// same key meet at one LDS address, which the LDS serialises at less cost
+// than grouping the lanes first (ballots and lane reads per group, measured
+// slower with 1 to 8 groups).  h = -1 when the table is full (the emission is
+// then not counted).
 template <int CAP>
-__device__ __forceinline__ void count_round(int* keys, unsigned* vals, bool want, int key, int& h, unsigned& at) {
-  h = -1;
-  at = 0;
-  if (want) {
-    h = slot_insert<CAP>(keys, key);
-    if (h >= 0) at = atomicAdd(&vals[h], 1u);
-  }
+__device__ __forceinline__ int count_key(int* keys, unsigned* vals, int key, unsigned& at) {
+  const int h = slot_insert<CAP>(keys, key);
+  at = h >= 0 ? atomicAdd(&vals[h], 1u) : 0u;
+  return h;
 }
-
-// exclusive prefix over the wave's lanes of v (0 <= v < 2^BITS) and the total
-template <int BITS>
-__device__ __forceinline__ int wave_prefix(int v, int& total) {
-  const unsigned long long below = (1ull << __lane_id()) - 1ull;
-  int off = 0, tot = 0;
-#pragma unroll
-  for (int b = 0; b < BITS; ++b) {
-    const unsigned long long m = __ballot((v >> b) & 1);
-    off += __popcll(m & below) << b;
-    tot += __popcll(m) << b;
-  }
-  total = tot;
-  return off;
-}
-__device__ __forceinline__ int wave_prefix4(int v, int& total) { return wave_prefix<4>(v, total); }
-__device__ __forceinline__ int wave_prefix5(int v, int& total) { return wave_prefix<5>(v, total); }
 
 // a reserved range in one word: its first slot (below 2^40; the host rejects
 // larger entry buffers) and, above it, how many of its slots lie within the
@@ -183,34 +154,31 @@ __device__ __forceinline__ long long reserved_slot(unsigned long long b, unsigne
 
 // Base-grid binning, persistent: each workgroup takes chunks of kHbChunk
 // particles (kHbPer per thread) in turn and loads its next chunk while it
-// bins this one.  Each valid particle
-// (finite, mass >= 0, within the TSC range of the base grid) emits one entry
-// per base tile its wrapped stencil touches.  Every wave lists its emissions
-// (tile key, particle) in its own LDS list, then counts the list 64 at a time
-// (a position in the key's range of the workgroup, written back over the
-// list word); one global add per key reserves the workgroup's ranges and
-// every wave writes its listed entries, taking each particle from the lane
-// that holds it.
+// bins this one.  Each valid particle (finite, mass >= 0, within the TSC
+// range of the base grid) has one entry, in the tile of its clamped cell.
+// Every lane counts its particles' keys in the workgroup's LDS table (a
+// position in the key's range of the workgroup), one global add per key
+// reserves the ranges, and every lane writes its particles from registers.
 // Per-chunk partials: base members and the largest mass.
+// Bound by latency (LDS counting, then one round of global reservations per
+// chunk).  One entry per particle instead of one per tile its stencil touches
+// needs no emission list, so twice the workgroups fit a CU and a third fewer
+// entries are written: 16.8M particles on 256^3 cells (16x8x8 tiles) 1,431 ->
+// 356 us, 134M particles 6.57 -> 2.11 ms.
 __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsigned long long* cursor,
                                                            const unsigned long long* start, int4* entries,
                                                            Counters* C, BlockTables BT) {
   __shared__ int keys[kHbCap];
   __shared__ unsigned vals[kHbCap];
   __shared__ unsigned long long base[kHbCap];
-  __shared__ unsigned long long wlist_all[(kHbThreads / 64) * kHbWList];
   __shared__ unsigned long long s_valid[kHbThreads / 64];
   __shared__ float s_mmax[kHbThreads / 64];
-  const int tid = threadIdx.x, lane = (int)__lane_id();
-  unsigned long long* wl = wlist_all + (tid >> 6) * kHbWList;
+  const int tid = threadIdx.x;
   const GridDesc& B = P.grids[0];
   const int bn[3] = {B.n[0], B.n[1], B.n[2]};
   const float bd[3] = {B.d[0], B.d[1], B.d[2]};
   const float bid[3] = {B.inv_d[0], B.inv_d[1], B.inv_d[2]};
   const int bnt0 = B.nt[0], bnt1 = B.nt[1];
-  auto particle = [&](long long i) {
-    return make_int4(__float_as_int(A.x[i]), __float_as_int(A.y[i]), __float_as_int(A.z[i]), __float_as_int(A.m[i]));
-  };
   const long long nchunks = (A.n + kHbChunk - 1) / kHbChunk;
   // the workgroup's next chunk of particles, loaded while this one is binned
   float fx[kHbPer], fy[kHbPer], fz[kHbPer], fm[kHbPer];
@@ -226,6 +194,8 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
   for (long long chunk = blockIdx.x; chunk < nchunks; chunk += gridDim.x) {
     const long long c0 = chunk * kHbChunk;
     float px[kHbPer], py[kHbPer], pz[kHbPer], pm[kHbPer];
+    int slot[kHbPer];       // the key's table slot, -1: no entry to write
+    unsigned at[kHbPer];    // the position in the key's range
 #pragma unroll
     for (int r = 0; r < kHbPer; ++r) { px[r] = fx[r]; py[r] = fy[r]; pz[r] = fz[r]; pm[r] = fm[r]; }
     fetch(chunk + gridDim.x);
@@ -234,7 +204,6 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
     unsigned err = 0;
     unsigned long long valid = 0;
     float mmax = 0.f;
-    int nw = 0;   // the wave's list length (uniform)
 #pragma unroll
     for (int r = 0; r < kHbPer; ++r) {
       const int k = r * kHbThreads + tid;
@@ -247,72 +216,31 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
         err |= kErrWrap;
         ok = false;
       }
-      int tx[3] = {0, 0, 0}, ty[3] = {0, 0, 0}, tz[3] = {0, 0, 0};
-      int nt = 0, nx_ = 1, ny_ = 1;
-      int hb[3] = {0, 0, 0};   // the home tile
+      slot[r] = -1;
+      at[r] = 0u;
       if (ok) {
         ++valid;
         mmax = fmaxf(mmax, m);
-        nx_ = base_axis_tiles(tsc_base_index(x, P.xl, bd[0], bid[0], bn[0]), bn[0], P.tshift[0], tx);
-        ny_ = base_axis_tiles(tsc_base_index(y, P.xl, bd[1], bid[1], bn[1]), bn[1], P.tshift[1], ty);
-        const int nz_ = base_axis_tiles(tsc_base_index(z, P.xl, bd[2], bid[2], bn[2]), bn[2], P.tshift[2], tz);
-        nt = nx_ * ny_ * nz_;
-        hb[0] = (home_cell(x, P.xl, bid[0], true, bn[0]) - 1) >> P.tshift[0];
-        hb[1] = (home_cell(y, P.xl, bid[1], true, bn[1]) - 1) >> P.tshift[1];
-        hb[2] = (home_cell(z, P.xl, bid[2], true, bn[2]) - 1) >> P.tshift[2];
-      }
-      int tot;
-      const int off = nw + wave_prefix5(nt, tot);
-      for (int c = 0; c < nt; ++c) {
-        const int q = div_small(c, nx_), qz = div_small(q, ny_);
-        const int a = c - q * nx_, b = q - qz * ny_;
-        const int ta = a == 0 ? tx[0] : (a == 1 ? tx[1] : tx[2]);
-        const int tb = b == 0 ? ty[0] : (b == 1 ? ty[1] : ty[2]);
-        const int tcz = qz == 0 ? tz[0] : (qz == 1 ? tz[1] : tz[2]);
-        const int key = 2 * ((tcz * bnt1 + tb) * bnt0 + ta) + ((ta == hb[0] && tb == hb[1] && tcz == hb[2]) ? 0 : 1);
-        if (off + c < kHbWList) wl[off + c] = (unsigned long long)(unsigned)key | ((unsigned long long)k << 32);
-        else emit_direct(cursor, start, entries, C, key, particle(c0 + k));
-      }
-      nw = min(nw + tot, kHbWList);
-    }
-    // count the list: a position in the key's range of the workgroup
-    for (int b0 = 0; b0 < nw; b0 += 64) {
-      const int idx = b0 + lane;
-      const bool want = idx < nw;
-      const unsigned long long w = want ? wl[idx] : 0ull;
-      int h;
-      unsigned at;
-      count_round<kHbCap>(keys, vals, want, (int)(unsigned)w, h, at);
-      if (want) {
-        if (h >= 0) {
-          wl[idx] = (w & 0xffffffff00000000ull) | ((unsigned long long)h << 16) | at;
-        } else {
-          wl[idx] = kEmSkip;
-          emit_direct(cursor, start, entries, C, (int)(unsigned)w, particle(c0 + (long long)(w >> 32)));
-        }
+        const int tx = (tsc_base_index(x, P.xl, bd[0], bid[0], bn[0]) - 1) >> P.tshift[0];
+        const int ty = (tsc_base_index(y, P.xl, bd[1], bid[1], bn[1]) - 1) >> P.tshift[1];
+        const int tz = (tsc_base_index(z, P.xl, bd[2], bid[2], bn[2]) - 1) >> P.tshift[2];
+        const int key = 2 * ((tz * bnt1 + ty) * bnt0 + tx);
+        slot[r] = count_key<kHbCap>(keys, vals, key, at[r]);
+        if (slot[r] < 0)
+          emit_direct(cursor, start, entries, C, key,
+                      make_int4(__float_as_int(x), __float_as_int(y), __float_as_int(z), __float_as_int(m)));
       }
     }
     __syncthreads();
     reserve_round<kHbCap, kHbThreads>(keys, vals, base, cursor, start, C);
     __syncthreads();
-    // the listed particle comes from the lane of this wave that loaded it
-    // (k = r * kHbThreads + tid: lane k % 64, register slot k / kHbThreads);
-    // every lane of the wave takes part in the shuffles
-    for (int b0 = 0; b0 < nw; b0 += 64) {
-      const int idx = b0 + lane;
-      const unsigned long long w = idx < nw ? wl[idx] : kEmSkip;
-      const int k = (int)(unsigned)(w >> 32);
-      const int src = k & 63, slot = (int)((unsigned)k / (unsigned)kHbThreads);
-      int4 e = make_int4(0, 0, 0, 0);
 #pragma unroll
-      for (int r = 0; r < kHbPer; ++r) {
-        const int4 u = make_int4(__shfl(__float_as_int(px[r]), src), __shfl(__float_as_int(py[r]), src),
-                                 __shfl(__float_as_int(pz[r]), src), __shfl(__float_as_int(pm[r]), src));
-        if (slot == r) e = u;
-      }
-      if (w == kEmSkip) continue;
-      const long long pos = reserved_slot(base[(w >> 16) & 0xffffu], (unsigned)(w & 0xffffu));
-      if (pos >= 0) entries[pos] = e;
+    for (int r = 0; r < kHbPer; ++r) {
+      if (slot[r] < 0) continue;
+      const long long pos = reserved_slot(base[slot[r]], at[r]);
+      if (pos >= 0)
+        entries[pos] = make_int4(__float_as_int(px[r]), __float_as_int(py[r]), __float_as_int(pz[r]),
+                                 __float_as_int(pm[r]));
     }
     // per-workgroup partials (members of the base grid, largest mass)
     valid = wave_sum(valid);
@@ -342,12 +270,14 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
 // 0).  Per item the target records are staged in LDS (kEmTargets at a time);
 // the item's entries are taken kEmPer per thread per round (one per round
 // where overlapping patches make the lists long).  In a
-// round every wave tests its entries against the targets and lists its
-// member emissions (destination tile key, entry) in its own LDS list, then
-// counts the list 64 emissions at a time (a position in the key's range of
-// the round for each, written back over the list word); one global add per
-// key reserves the round's ranges and every wave writes its listed entries,
-// reading each again from its source tile.
+// round every wave tests its entries against the targets and collects the
+// members; 64 of them at a time, one per lane, get their tile in the patch, a
+// position in the tile key's range of the round and a word in the wave's
+// list; one global add per key reserves the round's ranges and every wave
+// writes its listed entries, reading each again from its source tile.
+// Bound by VALU work and latency.  With one entry per member no lane loops
+// over the tiles of a stencil: 256^3 particles, 4 levels 1,111 -> 762 us;
+// 512^3, 6 levels 9.23 -> 6.06 ms.
 __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* items, long long item_lo,
                                                        long long item_hi, int level, int batch,
                                                        unsigned long long* cursor,
@@ -383,10 +313,9 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
       const int t = it.tile;
       const unsigned q0 = P.tgt_off[t], q1 = P.tgt_off[t + 1];
       if (q0 == q1) continue;
-      // the item's part of the tile's home entries: every member of this
-      // grid has exactly one, so each member is visited once
+      // the item's filled entries
       const long long e0 = it.begin;
-      const long long e1 = min(min(it.end, (long long)start[2 * t + 1]), (long long)cursor[2 * t]);
+      const long long e1 = min(it.end, (long long)cursor[2 * t]);
       if (e1 <= e0) continue;
       for (int k = tid; k < kEmCap; k += kEmThreads) { keys[k] = -1; vals[k] = 0u; }
       if (tid < 2) s_nwmax[tid] = 0;
@@ -408,7 +337,6 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
             const bool ok = r0 + k < e1;
             const int4 v = ok ? entries[r0 + k] : make_int4(0, 0, 0, 0);
             const float p[3] = {__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z)};
-            const bool home = ok;   // the range holds the tile's home entries only
             // the item's targets, one per pass: the box tests, with the
             // members listed (lane, target) in the wave's member list; every
             // 64 listed members, and at the end, the wave works through them
@@ -421,39 +349,33 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
               const float q[3] = {__int_as_float(u.x), __int_as_float(u.y), __int_as_float(u.z)};
               const BoxRec& R = recs[j];
               bool mem = lane < n;
-              int lo[3] = {0, 0, 0}, ext[3] = {1, 1, 1};
+              int tc[3] = {0, 0, 0};
               if (mem) {
                 ++pairs;
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
                   const int ci = (int)index_quotient(q[a] - R.org[a], R.d[a], R.inv_d[a]);
-                  const int c0 = max(ci - 1, 1), c1 = min(ci + 1, R.n[a]);
                   // a member whose quotient rounds onto the far face of the
                   // box (ci = N + 2) has no stencil cell in the patch
-                  mem = mem && c0 <= c1;
-                  lo[a] = (c0 - 1) >> P.tshift[a];
-                  ext[a] = ((c1 - 1) >> P.tshift[a]) - lo[a] + 1;
+                  mem = mem && ci <= R.n[a] + 1;
+                  tc[a] = (clampi(ci, 1, R.n[a]) - 1) >> P.tshift[a];
                 }
               }
-              const int nt = mem ? ext[0] * ext[1] * ext[2] : 0;
-              int hp[3] = {0, 0, 0};   // the member's home tile in the patch
-#pragma unroll
-              for (int a = 0; a < 3; ++a) hp[a] = (home_cell(q[a], R.org[a], R.inv_d[a], false, R.n[a]) - 1) >> P.tshift[a];
-              const int ks = i * kEmThreads + (tid & ~63) + src;
-              int tot;
-              const int off = nw + wave_prefix4(nt, tot);
-              for (int c = 0; c < nt; ++c) {
-                const int r = div_small(c, ext[0]), rz = div_small(r, ext[1]);
-                const int cx = lo[0] + c - r * ext[0], cy = lo[1] + r - rz * ext[1], cz = lo[2] + rz;
-                const int key = 2 * (R.tile0 + (cz * R.nt1 + cy) * R.nt0 + cx) +
-                                ((cx == hp[0] && cy == hp[1] && cz == hp[2]) ? 0 : 1);
-                if (off + c < kEmWList) wl[off + c] = (unsigned long long)(unsigned)key | ((unsigned long long)ks << 32);
-                else emit_direct(cursor, start, entries, C, key, u);
+              const unsigned long long mb = __ballot(mem);
+              const int off = nw + __popcll(mb & ((1ull << lane) - 1ull));
+              if (mem) {
+                const int ks = i * kEmThreads + (tid & ~63) + src;
+                const int key = 2 * (R.tile0 + (tc[2] * R.nt1 + tc[1]) * R.nt0 + tc[0]);
+                unsigned at = 0;
+                const int h = off < kEmWList ? count_key<kEmCap>(keys, vals, key, at) : -1;
+                if (h < 0) emit_direct(cursor, start, entries, C, key, u);
+                if (off < kEmWList)
+                  wl[off] = h < 0 ? kEmSkip : ((unsigned long long)ks << 32) | ((unsigned long long)h << 16) | at;
               }
-              nw = min(nw + tot, kEmWList);
+              nw = min(nw + __popcll(mb), kEmWList);
             };
             for (int j = 0; j < nq; ++j) {
-              const bool mem = home && in_box(recs[j], p[0], p[1], p[2]);
+              const bool mem = ok && in_box(recs[j], p[0], p[1], p[2]);
               const unsigned long long mb = __ballot(mem);
               if (mem) ml[nm + __popcll(mb & ((1ull << lane) - 1ull))] = (unsigned)lane | ((unsigned)j << 8);
               nm += __popcll(mb);
@@ -464,23 +386,6 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
               }
             }
             if (nm > 0) members(nm);
-          }
-          // ---- count the list: a position in the key's range of the round
-          for (int b0 = 0; b0 < nw; b0 += 64) {
-            const int idx = b0 + lane;
-            const bool want = idx < nw;
-            const unsigned long long w = want ? wl[idx] : 0ull;
-            int h;
-            unsigned at;
-            count_round<kEmCap>(keys, vals, want, (int)(unsigned)w, h, at);
-            if (want) {
-              if (h >= 0) {
-                wl[idx] = (w & 0xffffffff00000000ull) | ((unsigned long long)h << 16) | at;
-              } else {
-                wl[idx] = kEmSkip;
-                emit_direct(cursor, start, entries, C, (int)(unsigned)w, entries[r0 + (long long)(w >> 32)]);
-              }
-            }
           }
           if (lane == 0) atomicMax(&s_nwmax[par], nw);
           if (tid == 0) s_nwmax[par ^ 1] = 0;   // the next round's, before this barrier

@@ -98,8 +98,7 @@ struct Plan {
   int rad_malla;             // 1: RAD tables are exactly MALLA's recurrence (rad1 + (i-1)*radc)
   int merge_narrow;          // 1: narrow deposits may merge lanes (every non-centre weight product
                              // <= 0.45, so eight terms of a mass below 2^30 sum below 2^32)
-  int home_split;            // TSC count pass of the hierarchy binning: a member's entry in its
-                             // home tile t counts under key 2t, its other entries under 2t + 1
+  int pad;
   float rad1[3];
   float radc[3];
   // TSC binning along the hierarchy: the patches whose members are found
@@ -129,7 +128,7 @@ struct Counters {
   unsigned long long n_pairs;     // reduced from per-block partials
   unsigned long long n_entries;   // totals of the planning scans, copied by the gate kernel
   unsigned long long n_items;
-  unsigned long long n_split;
+  unsigned long long pad0;
   unsigned int err;               // bit 0: non-finite position/mass, bit 1: base index outside
                                   // the single-wrap range, bit 2: negative mass
   unsigned int mmax_bits;         // max particle mass, as FP32 bits (masses >= 0)
@@ -179,10 +178,8 @@ struct DepArgs {
   const int4* entries;       // binned entries, grouped by tile
   const Item* items;         // work queue
   const int* nitems_tile;    // items per tile
-  const int* split_slot;     // first scratch slot of a split tile, -1 otherwise
-  const int* split_tiles;    // the split tiles, in tile order
-  const unsigned long long* n_split_tiles;   // their count (device)
-  void* scratch;             // int64 (deterministic) or FP32 (atomic) tile accumulators
+  void* scratch;             // exchange cells: int64 (deterministic) or FP32 (atomic), a tile with its
+                             // one-cell halo per tile
   Counters* C;               // n_items_eff (the queue length) and mmax_bits (the fixed-point
                              // scale) are read here, so no host round trip precedes the deposit
   float* u1;
@@ -190,10 +187,9 @@ struct DepArgs {
   long long* tile_mass_i;    // deterministic: exact fixed-point mass per tile
   double* tile_mass_d;       // atomic: FP64 mass per tile
   int n_queues;              // queues in use (<= kQueues, <= grid)
-  // TSC binning along the hierarchy: tile t's range [start[2t], start[2t+2])
-  // holds its members' home entries from start[2t] to cursor[2t] and their
-  // other entries from start[2t+1] to cursor[2t+1]; items cover capacity
-  // ranges (both NULL otherwise: every item's range is filled)
+  // offsets of the tiles' entry ranges; with the hierarchy binning items cover
+  // capacity ranges, filled up to cursor[2t] (NULL otherwise: every item's
+  // range is filled)
   const unsigned long long* cursor;
   const unsigned long long* start;
   int hist_cells;            // table mode: int64 cells of the wide classes' histogram buffer

@@ -6,8 +6,10 @@
 //   scatter_kernel  particles -> 16-byte entries grouped by tile    [reads x,y,z,m]
 //   plan_items      tiles -> work items (chunks of <= chunk entries)
 //   deposit_kernel  ONE persistent launch over the item queue: LDS tile
-//                   accumulation, normalised coalesced stores, FP64-exact
-//                   tile mass partials
+//                   accumulation, the tile and its one-cell halo to the
+//                   exchange buffer
+//   combine_tiles   a tile's cells plus its neighbours' halo sums: normalised
+//                   coalesced stores, FP64-exact tile mass partials
 //   grid_sums       fixed-order per-grid mass sums
 // Plain form: one launch per grid with global FP32 atomics (plain_*).
 #include <hip/hip_runtime.h>
@@ -448,12 +450,11 @@ __global__ void __launch_bounds__(kScanThreads) scan_apply(const unsigned* in, l
 // ---------------------------------------------------------------------------
 // work items
 // ---------------------------------------------------------------------------
-// Work items.  plan_count: items per tile and the partial-tile slots a split
-// tile needs; after exclusive scans of both, plan_write places every tile's
-// items at its offset (no atomics: the item order is the tile order).
-// With chunk_wide = 0 the tile's whole range [start[2t], start[2t+2]) is
-// chunked as narrow entries (the TSC hierarchy binning, whose keys 2t and
-// 2t + 1 are a tile's home and other entries).
+// Work items.  plan_count: items per tile; after an exclusive scan,
+// plan_write places every tile's items at its offset (no atomics: the item
+// order is the tile order).  With chunk_wide = 0 the tile's whole range
+// [start[2t], start[2t+2]) is chunked as narrow entries (the TSC hierarchy
+// binning, which uses the keys 2t only).
 __device__ __forceinline__ void tile_chunks(const unsigned long long* start, int t, int chunk, int chunk_wide,
                                             long long& s0, long long& s1, long long& s2, int& cn, int& cw) {
   s0 = start[2 * t]; s1 = start[2 * t + 1]; s2 = start[2 * t + 2];
@@ -468,35 +469,23 @@ __device__ __forceinline__ void tile_chunks(const unsigned long long* start, int
 }
 
 __global__ void plan_count(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                           unsigned* nitems_tile, unsigned* nsplit_tile, unsigned* is_split) {
+                           unsigned* nitems_tile) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ntiles) return;
   long long s0, s1, s2;
   int cn, cw;
   tile_chunks(start, t, chunk, chunk_wide, s0, s1, s2, cn, cw);
-  const int tot = max(cn + cw, 1);   // an empty tile still writes its zeros
-  nitems_tile[t] = (unsigned)tot;
-  nsplit_tile[t] = tot > 1 ? 1u : 0u;   // one accumulator tile per split tile
-  is_split[t] = tot > 1 ? 1u : 0u;
+  nitems_tile[t] = (unsigned)(cn + cw);   // none for a tile without entries
 }
 
 __global__ void plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                           const unsigned long long* item_off, const unsigned long long* split_off,
-                           const unsigned long long* split_rank, Item* items, int* split_slot,
-                           int* split_tiles, long long* tile_mass, const Counters* C) {
+                           const unsigned long long* item_off, Item* items, const Counters* C) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ntiles || C->overflow) return;
   long long s0, s1, s2;
   int cn, cw;
   tile_chunks(start, t, chunk, chunk_wide, s0, s1, s2, cn, cw);
   const long long base = (long long)item_off[t];
-  const int tot = max(cn + cw, 1);
-  split_slot[t] = tot > 1 ? (int)split_off[t] : -1;
-  if (tot > 1) {
-    split_tiles[split_rank[t]] = t;
-    tile_mass[t] = 0;   // summed by split_reduce (zero bits: 0 as int64 and as FP64)
-  }
-  if (cn + cw == 0) { items[base] = Item{t, 0, s0, s0}; return; }
   int k = 0;
   for (int c = 0; c < cn; ++c, ++k) {
     const long long b = s0 + (long long)c * chunk;
@@ -516,14 +505,12 @@ __global__ void plan_write(const unsigned long long* start, int ntiles, int chun
 // device, whether they still suffice; if not, every later kernel of the call
 // does nothing and the host rebuilds with exact sizes.
 __global__ void gate_kernel(const unsigned long long* tot_entries, const unsigned long long* tot_items,
-                            const unsigned long long* tot_split, unsigned long long cap_entries,
-                            unsigned long long cap_items, unsigned long long cap_split, Counters* C) {
+                            unsigned long long cap_entries, unsigned long long cap_items, Counters* C) {
   if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  const unsigned long long ne = *tot_entries, ni = *tot_items, ns = *tot_split;
+  const unsigned long long ne = *tot_entries, ni = *tot_items;
   C->n_entries = ne;
   C->n_items = ni;
-  C->n_split = ns;
-  const bool over = ne > cap_entries || ni > cap_items || ns > cap_split || ni >= (1ull << 31);
+  const bool over = ne > cap_entries || ni > cap_items || ni >= (1ull << 31);
   C->overflow = over ? 1u : 0u;
   C->n_items_eff = over ? 0u : (unsigned)ni;
 }
@@ -769,14 +756,36 @@ __device__ __forceinline__ float base_centre(const Plan& P, int a, int i, int n)
   return r[i];
 }
 
-// tile-local coordinate of the stencil centre: on the periodic base grid the
-// image of the (wrapped) centre that lies next to the tile
-__device__ __forceinline__ int centre_local(int c, int org, int ext, int n, bool periodic) {
-  if (!periodic) return c - org;
-  int l = wrap1(c, n) - org;
-  if (l > ext) l -= n;
-  if (l < -1) l += n;
-  return l;
+// LDS layout of a deposit tile: cell (x, y, z), local coordinates from -1 (the
+// tile's halo) to T, at kTileFront + (x + 1) + HX * ((y + 1) + HY * (z + 2)).
+// Every entry's centre cell, clamped into its grid, lies in the tile, so a
+// stencil reaches at most one cell past the tile, or two where the centre
+// itself lies one cell outside a patch; that second cell is outside the patch
+// and never read.  It falls into the pad column, the pad row or the outer
+// planes (and, below row 0 of the first plane, into the front pad), so the
+// deposit needs no per-cell test.
+template <int TX, int TY, int TZ>
+struct TileLds {
+  static constexpr int HX = TX + 3, HY = TY + 3, HZ = TZ + 4;
+  static constexpr int kFront = HX + 1;
+  static constexpr int H = kFront + HX * HY * HZ;
+  // the tile with its one-cell halo, as written to the exchange buffer.  The
+  // odd row pitch spreads a stencil's adds over the LDS banks.
+  static constexpr int EX = TX + 2, EY = TY + 2, EZ = TZ + 2, E = EX * EY * EZ;
+  __device__ __forceinline__ static int at(int x, int y, int z) {
+    return kFront + (x + 1) + HX * ((y + 1) + HY * (z + 2));
+  }
+  // exchange cell c (x fastest) in the LDS tile
+  __device__ __forceinline__ static int of_exchange(int c) {
+    return kFront + c % EX + HX * ((c / EX) % EY + HY * (c / (EX * EY) + 1));
+  }
+};
+
+// Whether tile t received entries in this call (its exchange cells are then
+// written): the hierarchy binning fills [start[2t], cursor[2t]) of a
+// capacity range, the count pass fills [start[2t], start[2t+2]) exactly.
+__device__ __forceinline__ bool tile_filled(const DepArgs& D, int t) {
+  return D.cursor ? D.cursor[2 * t] > D.start[2 * t] : D.start[2 * t + 2] > D.start[2 * t];
 }
 
 // The wide entries of one class (kernel level irk, half-width N) of a work
@@ -787,7 +796,7 @@ __device__ __forceinline__ int centre_local(int c, int org, int ext, int n, bool
 // and z in FP64, each pass in place on the buffer; the result, rounded once
 // per cell, is added to the tile's accumulator.  Cells of the tile outside
 // the grid receive values that are never written out.
-template <int RED, int TX, int TY, int TZ, int HX, int HY>
+template <int RED, int TX, int TY, int TZ>
 __device__ void wide_histogram_form(const DepArgs& D, const Item& it, int irk, int i0, int j0, int k0c,
                                     const float* K, float scale, double dscale,
                                     typename AccT<RED>::T* acc, long long* hist) {
@@ -796,7 +805,7 @@ __device__ void wide_histogram_form(const DepArgs& D, const Item& it, int irk, i
   const int nk = 1 << irk;
   const int bx = TX + 2 * nk, by = TY + 2 * nk, bz = TZ + 2 * nk, nb = bx * by * bz;
   double* hd = reinterpret_cast<double*>(hist);
-  auto at = [](int a, int b, int c) { return (a + 2) + HX * ((b + 2) + HY * (c + 2)); };
+  auto at = [](int a, int b, int c) { return TileLds<TX, TY, TZ>::at(a, b, c); };
   for (int c = tid; c < nb; c += nthr) hist[c] = 0;
   __syncthreads();
   for (long long e = it.begin + tid; e < it.end; e += nthr) {
@@ -854,15 +863,10 @@ __device__ void wide_histogram_form(const DepArgs& D, const Item& it, int irk, i
 template <int MODE, int RED, int TX, int TY, int TZ>
 __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
   using Acc = typename AccT<RED>::T;
-  constexpr int T = TX * TY * TZ;
-  // the tile with a 2-cell halo; x and y rows padded by one cell (a row of
-  // 21 int64 cells instead of 20 spreads the stencil's adds over more LDS
-  // banks: 6% less deposit time on clustered particles)
-  constexpr int HX = TX + 5, HY = TY + 5, HZ = TZ + 4, H = HX * HY * HZ;
+  using L = TileLds<TX, TY, TZ>;
+  constexpr int HX = L::HX, HY = L::HY, H = L::H;
   __shared__ Acc acc[H];
   __shared__ unsigned s_item;
-  __shared__ long long s_redi[16];
-  __shared__ double s_redd[16];
   // table mode: the used part of the kernel table, row irk (2^(irk+1) + 1
   // values) at ktab_off(irk), centred at ktab_off(irk) + 2^irk
   __shared__ float s_ktab[MODE == 1 ? kKtabLds : 1];
@@ -883,8 +887,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     }
     // the first item's __syncthreads orders these writes before any read
   }
-  // interior cell (a, b, c) of the tile
-  auto at = [](int a, int b, int c) { return (a + 2) + HX * ((b + 2) + HY * (c + 2)); };
+  auto at = [](int a, int b, int c) { return L::at(a, b, c); };
 
   // workgroup w serves queue w mod n_queues, which hands out items
   // q, q + n_queues, ...; consecutive workgroups land on different XCDs, so
@@ -905,6 +908,15 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     const int ex = min(TX, G.n[0] - i0 + 1), ey = min(TY, G.n[1] - j0 + 1), ez = min(TZ, G.n[2] - k0c + 1);
     const bool periodic = g == 0;
 
+    // the item's filled entries: with the hierarchy binning the tile's
+    // entries end at cursor[2t]
+    long long len = it.end - it.begin;
+    if (D.cursor) len = min(it.end, (long long)D.cursor[2 * t]) - it.begin;
+    len = uniform64(len);   // wave-uniform: kept in scalar registers
+    if (len <= 0) {
+      __syncthreads();   // every wave has read s_item before thread 0 takes the next item
+      continue;
+    }
     for (int c = tid; c < H; c += nthr) acc[c] = 0;
     __syncthreads();
 
@@ -916,23 +928,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
       // would wait on the loads); the prefetch indices are clamped into the
       // item instead of tested, so every pass issues the same loads, and the
       // loop runs the same number of passes on every lane (ok = the lane holds
-      // an entry), which the lane merging of the TSC deposit needs.  An empty
-      // item reads nothing: no pass runs.
-      // the item's filled entries: [bA, bA + la) and [bB, bB + (len - la));
-      // with the hierarchy binning the tile's home entries end at cursor[2t]
-      // and its other entries run from start[2t+1] to cursor[2t+1]
-      long long la = it.end - it.begin, gap = 0, len = la;
-      if (D.cursor) {
-        const long long s1 = (long long)D.start[2 * t + 1];
-        la = max(min(min(it.end, s1), (long long)D.cursor[2 * t]) - it.begin, 0ll);
-        const long long bB = max(it.begin, s1);
-        gap = bB - (it.begin + la);
-        len = la + max(min(it.end, (long long)D.cursor[2 * t + 1]) - bB, 0ll);
-      }
-      // wave-uniform: kept in scalar registers
-      la = uniform64(la);
-      gap = uniform64(gap);
-      len = uniform64(len);
+      // an entry), which the lane merging of the TSC deposit needs.
       const int4* const eb = D.entries + uniform64(it.begin);
       auto narrow = [&](const int4 v, const bool ok) {
         int ci[3];
@@ -966,26 +962,18 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
         }
         // in [-1, ext] by construction of the binning; clamped so the array
         // bounds never depend on that
-        const int lx = clampi(centre_local(ci[0], i0, ex, G.n[0], periodic), -1, TX);
-        const int ly = clampi(centre_local(ci[1], j0, ey, G.n[1], periodic), -1, TY);
-        const int lz = clampi(centre_local(ci[2], k0c, ez, G.n[2], periodic), -1, TZ);
-        // corner (-1,-1,-1) of the stencil; halo coordinates are local + 2
-        const int corner = (lx + 1) + HX * ((ly + 1) + HY * (lz + 1));
+        const int lx = clampi((periodic ? wrap1(ci[0], G.n[0]) : ci[0]) - i0, -1, TX);
+        const int ly = clampi((periodic ? wrap1(ci[1], G.n[1]) : ci[1]) - j0, -1, TY);
+        const int lz = clampi((periodic ? wrap1(ci[2], G.n[2]) : ci[2]) - k0c, -1, TZ);
+        const int corner = at(lx - 1, ly - 1, lz - 1);
         if (MODE == 2 || P.merge_narrow)
           deposit27_merged<RED, HX, HY>(acc, corner, ok, m, wx, wy, wz, scale);
         else if (ok)
           deposit27<RED, HX, HY>(acc + corner, m, wx, wy, wz, scale);
       };
       // entry j of the item (j clamped to the last one)
-      auto at_j = [&](long long j) {
-        j = min(j, len - 1);
-        return eb[j + (j < la ? 0ll : gap)];
-      };
-      int4 va = make_int4(0, 0, 0, 0), vb = va;
-      if (len > 0) {
-        va = at_j(tid);
-        vb = at_j(tid + nthr);
-      }
+      auto at_j = [&](long long j) { return eb[min(j, len - 1)]; };
+      int4 va = at_j(tid), vb = at_j(tid + nthr);
       for (long long o = 0; o < len; o += 2 * nthr) {
         narrow(va, o + tid < len);
         va = at_j(o + 2 * nthr + tid);
@@ -1027,7 +1015,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
         const long long w = 2 * nk + 1;
         const long long passes = w * ((long long)bx * by * TX + (long long)TX * bz * TY + (long long)TX * TY * TZ);
         if ((it.flags & 2) && bx * by * bz <= D.hist_cells && 4ll * ncls * w * w * w > passes) {
-          wide_histogram_form<RED, TX, TY, TZ, HX, HY>(D, it, irk, i0, j0, k0c, K, scale, dscale, acc, s_hist);
+          wide_histogram_form<RED, TX, TY, TZ>(D, it, irk, i0, j0, k0c, K, scale, dscale, acc, s_hist);
           continue;
         }
         // direct: one wave per entry.  The entry's box clipped to the tile
@@ -1087,138 +1075,131 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     }
     __syncthreads();
 
-    // ---- a tile spanning a whole periodic axis: its halo cells are its own
-    // interior cells under the reference's wrap; fold them in ----
-    if (periodic && (G.nt[0] == 1 || G.nt[1] == 1 || G.nt[2] == 1)) {
-      for (int c = tid; c < H; c += nthr) {
-        const int a = c % HX - 2, b = (c / HX) % HY - 2, cz = c / (HX * HY) - 2;
-        if (a >= 0 && a < ex && b >= 0 && b < ey && cz >= 0 && cz < ez) continue;
-        const int ga = wrap1(i0 + a, G.n[0]) - i0, gb = wrap1(j0 + b, G.n[1]) - j0,
-                  gc = wrap1(k0c + cz, G.n[2]) - k0c;
-        if (ga < 0 || ga >= ex || gb < 0 || gb >= ey || gc < 0 || gc >= ez) continue;
-        const Acc v = acc[c];
-        if (v != 0) lds_add(acc + at(ga, gb, gc), v);
-      }
-      __syncthreads();
-    }
-
-    // ---- split tile: every item adds its interior into the tile's
-    // accumulator in global memory (int64 adds are exact, so the sum does not
-    // depend on the order of the items); split_reduce writes the cells ----
-    const int nit = D.nitems_tile[t];
-    const bool writer = nit == 1;
-    if (!writer) {
-      Acc* dst = reinterpret_cast<Acc*>(D.scratch) + (long long)D.split_slot[t] * T;
-      for (int c = tid; c < T; c += nthr) {
-        const Acc v = acc[at(c % TX, (c / TX) % TY, c / (TX * TY))];
+    // ---- the tile and its halo to the exchange buffer: stored when the tile
+    // has one item, added where several items share it (exact int64 adds, so
+    // the sum does not depend on their order; the cells were cleared) ----
+    Acc* dst = reinterpret_cast<Acc*>(D.scratch) + (long long)t * L::E;
+    if (D.nitems_tile[t] == 1) {
+      for (int c = tid; c < L::E; c += nthr) dst[c] = acc[L::of_exchange(c)];
+    } else {
+      for (int c = tid; c < L::E; c += nthr) {
+        const Acc v = acc[L::of_exchange(c)];
         if (v != 0) glb_add(dst + c, v);
-      }
-    }
-    if (writer) {
-      float* out = (g == 0 ? D.u1 : D.u11) + G.off;
-      long long msi = 0;
-      double msd = 0.0;
-      const double inv_scale = 1.0 / dscale;   // a power of two: exact
-      for (int c = tid; c < T; c += nthr) {
-        const int a = c % TX, b = (c / TX) % TY, cz = c / (TX * TY);
-        if (a >= ex || b >= ey || cz >= ez) continue;
-        const Acc v = acc[at(a, b, cz)];
-        if (RED == 0) msi += (long long)v;
-        else msd += (double)v;
-        float f = RED == 0 ? (float)((double)v * inv_scale) : (float)v;
-        f = f / G.den;
-        f = f / P.fdm;
-        out[(long long)(i0 - 1 + a) + (long long)G.ld1 * (j0 - 1 + b) + (long long)G.ld2 * (k0c - 1 + cz)] = f;
-      }
-      if (RED == 0) {
-        msi = block_sum(msi, s_redi);
-        if (tid == 0) D.tile_mass_i[t] = msi;
-      } else {
-        msd = block_sum(msd, s_redd);
-        if (tid == 0) D.tile_mass_d[t] = msd;
       }
     }
     __syncthreads();
   }
 }
 
-// Split tiles: the accumulated interiors normalised and written as the
-// deposit's writer does.  Work unit = (split tile, kPer * 256 consecutive
-// cells, kPer per thread with every load issued before the first store), so a
-// heavy tile is spread over many workgroups; the exact int64 (FP64 in atomic
-// mode) tile mass is accumulated per unit.
+// The output cells from the tiles' exchange cells.  A workgroup takes a tile
+// at a time: a cell is the tile's own sum plus what the stencils of the up to
+// 26 neighbouring tiles spilled over it (their halo cells; on the base grid
+// the neighbours wrap, and a tile spanning an axis is its own neighbour),
+// divided by DENBAS then FDM (FP32, the reference's two divisions) and stored
+// row by row.  The exact int64 (FP64 in atomic mode) tile mass is the sum of
+// the cells before the divisions.
+// Exchanging halo sums costs 14 B written and read per cell of a 16x8x8 tile
+// (179 us on 18.1M cells, 1.18 ms on 93.9M), less than the entries it saves:
+// a stencil crossing tile borders used to be binned, emitted and deposited
+// once per tile it touched, 1.5 to 1.8 entries per member (the whole build on
+// 256^3 particles and 4 levels 4.01 -> 2.22 ms, 512^3 and 6 levels 28.9 ->
+// 18.0 ms).
 template <int RED, int TX, int TY, int TZ>
-__global__ void __launch_bounds__(256) split_reduce(Plan P, DepArgs D) {
+__global__ void __launch_bounds__(256) combine_tiles(Plan P, DepArgs D) {
   using Acc = typename AccT<RED>::T;
+  using L = TileLds<TX, TY, TZ>;
   constexpr int T = TX * TY * TZ;
-  constexpr int kPer = 4;
-  constexpr int kCells = 256 * kPer;
-  constexpr int cpt = (T + kCells - 1) / kCells;
+  __shared__ long long s_nb[27];   // first exchange cell of each neighbour, -1: none or empty
   __shared__ long long s_redi[4];
   __shared__ double s_redd[4];
   if (D.C->overflow) return;
-  const double inv_scale = 1.0 / fixed_scale(D.C->mmax_bits);
-  const unsigned long long units = *D.n_split_tiles * cpt;
-  for (unsigned long long u = blockIdx.x; u < units; u += gridDim.x) {
-    const int t = D.split_tiles[u / cpt];
-    const int c0 = (int)(u % cpt) * kCells + threadIdx.x;
+  const double inv_scale = 1.0 / fixed_scale(D.C->mmax_bits);   // a power of two: exact
+  const int tid = threadIdx.x;
+  for (int t = blockIdx.x; t < P.ntiles; t += gridDim.x) {
     const int g = P.tile_grid[t];
     const GridDesc& G = P.grids[g];
+    const bool periodic = g == 0;
     const int local = t - G.tile0;
-    const int tx = local % G.nt[0], ty = (local / G.nt[0]) % G.nt[1], tz = local / (G.nt[0] * G.nt[1]);
-    const int i0 = tx * TX + 1, j0 = ty * TY + 1, k0c = tz * TZ + 1;
-    const int ex = min(TX, G.n[0] - i0 + 1), ey = min(TY, G.n[1] - j0 + 1), ez = min(TZ, G.n[2] - k0c + 1);
-    const Acc* part = reinterpret_cast<const Acc*>(D.scratch) + (long long)D.split_slot[t] * T;
-    float* out = (g == 0 ? D.u1 : D.u11) + G.off;
-    Acc v[kPer];
-    bool in[kPer];
+    const int tc[3] = {local % G.nt[0], (local / G.nt[0]) % G.nt[1], local / (G.nt[0] * G.nt[1])};
+    const int sh[3] = {TX, TY, TZ};
+    int o[3], ext[3], prev[3];   // first cell, cells, and the cell past the last one of the tile before
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int c = c0 + r * 256;
-      const int a = c % TX, b = (c / TX) % TY, cz = c / (TX * TY);
-      in[r] = c < T && a < ex && b < ey && cz < ez;
-      v[r] = in[r] ? part[c] : (Acc)0;
+    for (int a = 0; a < 3; ++a) {
+      o[a] = tc[a] * sh[a];
+      ext[a] = min(sh[a], G.n[a] - o[a]);
+      prev[a] = tc[a] > 0 ? sh[a] : G.n[a] - (G.nt[a] - 1) * sh[a];
     }
+    if (tid < 27) {
+      const int d[3] = {tid % 3 - 1, (tid / 3) % 3 - 1, tid / 9 - 1};
+      int c[3];
+      bool in = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        c[a] = tc[a] + d[a];
+        if (periodic) c[a] = c[a] < 0 ? G.nt[a] - 1 : (c[a] >= G.nt[a] ? 0 : c[a]);
+        else in = in && c[a] >= 0 && c[a] < G.nt[a];
+      }
+      const int tn = G.tile0 + (c[2] * G.nt[1] + c[1]) * G.nt[0] + c[0];
+      s_nb[tid] = in && tile_filled(D, tn) ? (long long)tn * L::E : -1ll;
+    }
+    __syncthreads();
+    const Acc* S = reinterpret_cast<const Acc*>(D.scratch);
+    float* out = (g == 0 ? D.u1 : D.u11) + G.off;
     long long msi = 0;
     double msd = 0.0;
+    for (int c = tid; c < T; c += 256) {
+      const int l[3] = {c % TX, (c / TX) % TY, c / (TX * TY)};
+      if (l[0] >= ext[0] || l[1] >= ext[1] || l[2] >= ext[2]) continue;
+      Acc v = 0;
+      if (s_nb[13] >= 0) v = S[s_nb[13] + (l[0] + 1) + L::EX * ((l[1] + 1) + L::EY * (l[2] + 1))];
+      int lo[3], hi[3];
+      bool edge = false;
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      if (!in[r]) continue;
-      const int c = c0 + r * 256;
-      const int a = c % TX, b = (c / TX) % TY, cz = c / (TX * TY);
-      if (RED == 0) msi += (long long)v[r];
-      else msd += (double)v[r];
-      float f = RED == 0 ? (float)((double)v[r] * inv_scale) : (float)v[r];
+      for (int a = 0; a < 3; ++a) {
+        lo[a] = l[a] == 0 ? -1 : 0;
+        hi[a] = l[a] == ext[a] - 1 ? 1 : 0;
+        edge = edge || lo[a] < 0 || hi[a] > 0;
+      }
+      if (edge) {
+        for (int dz = lo[2]; dz <= hi[2]; ++dz)
+          for (int dy = lo[1]; dy <= hi[1]; ++dy)
+            for (int dx = lo[0]; dx <= hi[0]; ++dx) {
+              const long long nb = s_nb[(dx + 1) + 3 * ((dy + 1) + 3 * (dz + 1))];
+              if ((dx | dy | dz) == 0 || nb < 0) continue;
+              // this cell in the neighbour's coordinates: past the last cell
+              // of the tile before, or the halo below the tile after
+              const int x = dx == 0 ? l[0] : (dx < 0 ? prev[0] : -1);
+              const int y = dy == 0 ? l[1] : (dy < 0 ? prev[1] : -1);
+              const int z = dz == 0 ? l[2] : (dz < 0 ? prev[2] : -1);
+              v += S[nb + (x + 1) + L::EX * ((y + 1) + L::EY * (z + 1))];
+            }
+      }
+      if (RED == 0) msi += (long long)v;
+      else msd += (double)v;
+      float f = RED == 0 ? (float)((double)v * inv_scale) : (float)v;
       f = f / G.den;
       f = f / P.fdm;
-      out[(long long)(i0 - 1 + a) + (long long)G.ld1 * (j0 - 1 + b) + (long long)G.ld2 * (k0c - 1 + cz)] = f;
+      out[(long long)(o[0] + l[0]) + (long long)G.ld1 * (o[1] + l[1]) + (long long)G.ld2 * (o[2] + l[2])] = f;
     }
     if (RED == 0) {
       msi = block_sum(msi, s_redi);
-      if (threadIdx.x == 0 && msi != 0)
-        atomicAdd(reinterpret_cast<unsigned long long*>(D.tile_mass_i + t), (unsigned long long)msi);
+      if (tid == 0) D.tile_mass_i[t] = msi;
     } else {
       msd = block_sum(msd, s_redd);
-      if (threadIdx.x == 0 && msd != 0.0) atomicAdd(D.tile_mass_d + t, msd);
+      if (tid == 0) D.tile_mass_d[t] = msd;
     }
   }
 }
 
-// clears the accumulator tiles of this call's split tiles (their count is on
-// the device); a kernel, not a memset, so the build can be captured
-__global__ void __launch_bounds__(256) zero_split(DepArgs D, int T, int elem_words) {
+// Clears the exchange cells of the tiles that several work items add to; a
+// kernel, not a memset, so the build can be captured.
+__global__ void __launch_bounds__(256) zero_split(DepArgs D, int ntiles, int words) {
   if (D.C->overflow) return;
-  const unsigned long long ns = *D.n_split_tiles;
-  const unsigned long long n = ns * (unsigned long long)T * (unsigned long long)elem_words;
-  unsigned* p = reinterpret_cast<unsigned*>(D.scratch);
-  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n;
-       i += (unsigned long long)gridDim.x * blockDim.x)
-    p[i] = 0u;
-  // the split tiles' masses, which split_reduce accumulates (zero bits are 0
-  // as int64 and as FP64)
-  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < ns;
-       i += (unsigned long long)gridDim.x * blockDim.x)
-    D.tile_mass_i[D.split_tiles[i]] = 0;
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    if (D.nitems_tile[t] <= 1) continue;
+    unsigned* p = reinterpret_cast<unsigned*>(D.scratch) + (long long)t * words;
+    for (int i = threadIdx.x; i < words; i += blockDim.x) p[i] = 0u;
+  }
 }
 
 // per-grid mass in a fixed order; FP64 (int64-exact in deterministic mode)
@@ -1666,26 +1647,20 @@ hipError_t launch_reduce_blocks(const BlockTables& BT, long long nblk, Counters*
 }
 
 hipError_t launch_plan_count(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                             unsigned* nitems_tile, unsigned* nsplit_tile, unsigned* is_split, hipStream_t s) {
-  plan_count<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, nitems_tile,
-                                                           nsplit_tile, is_split);
+                             unsigned* nitems_tile, hipStream_t s) {
+  plan_count<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, nitems_tile);
   return hipGetLastError();
 }
 
 hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                             const unsigned long long* item_off, const unsigned long long* split_off,
-                             const unsigned long long* split_rank, Item* items, int* split_slot,
-                             int* split_tiles, long long* tile_mass, const Counters* C, hipStream_t s) {
-  plan_write<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, item_off,
-                                                           split_off, split_rank, items, split_slot,
-                                                           split_tiles, tile_mass, C);
+                             const unsigned long long* item_off, Item* items, const Counters* C, hipStream_t s) {
+  plan_write<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, item_off, items, C);
   return hipGetLastError();
 }
 
 hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* tot_items,
-                       const unsigned long long* tot_split, unsigned long long cap_entries,
-                       unsigned long long cap_items, unsigned long long cap_split, Counters* C, hipStream_t s) {
-  gate_kernel<<<1, 64, 0, s>>>(tot_entries, tot_items, tot_split, cap_entries, cap_items, cap_split, C);
+                       unsigned long long cap_entries, unsigned long long cap_items, Counters* C, hipStream_t s) {
+  gate_kernel<<<1, 64, 0, s>>>(tot_entries, tot_items, cap_entries, cap_items, C);
   return hipGetLastError();
 }
 
@@ -1741,25 +1716,27 @@ bool tile_shape_supported(const int t[3]) {
 }
 
 template <int RED>
-static hipError_t split_shape(const Plan& P, const DepArgs& D, int grid, hipStream_t s) {
+static hipError_t combine_shape(const Plan& P, const DepArgs& D, int grid, hipStream_t s) {
   const int* t = P.tile;
-  if (t[0] == 8 && t[1] == 8 && t[2] == 8) split_reduce<RED, 8, 8, 8><<<grid, 256, 0, s>>>(P, D);
-  else if (t[0] == 16 && t[1] == 8 && t[2] == 8) split_reduce<RED, 16, 8, 8><<<grid, 256, 0, s>>>(P, D);
-  else if (t[0] == 16 && t[1] == 16 && t[2] == 8) split_reduce<RED, 16, 16, 8><<<grid, 256, 0, s>>>(P, D);
-  else if (t[0] == 16 && t[1] == 16 && t[2] == 16) split_reduce<RED, 16, 16, 16><<<grid, 256, 0, s>>>(P, D);
+  if (t[0] == 8 && t[1] == 8 && t[2] == 8) combine_tiles<RED, 8, 8, 8><<<grid, 256, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 8 && t[2] == 8) combine_tiles<RED, 16, 8, 8><<<grid, 256, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 8) combine_tiles<RED, 16, 16, 8><<<grid, 256, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 16) combine_tiles<RED, 16, 16, 16><<<grid, 256, 0, s>>>(P, D);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
+long long exchange_cells(const int t[3]) { return (long long)(t[0] + 2) * (t[1] + 2) * (t[2] + 2); }
+
 hipError_t launch_zero_split(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s) {
-  const int T = P.tile[0] * P.tile[1] * P.tile[2];
-  zero_split<<<(cus > 1 ? cus : 1) * 8, 256, 0, s>>>(D, T, reduction == 0 ? 2 : 1);
+  const int words = (int)exchange_cells(P.tile) * (reduction == 0 ? 2 : 1);
+  zero_split<<<std::max(1, std::min(P.ntiles, cus * 8)), 256, 0, s>>>(D, P.ntiles, words);
   return hipGetLastError();
 }
 
-hipError_t launch_split_reduce(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s) {
-  const int grid = (cus > 1 ? cus : 1) * 8;
-  return reduction == 0 ? split_shape<0>(P, D, grid, s) : split_shape<1>(P, D, grid, s);
+hipError_t launch_combine(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s) {
+  const int grid = std::max(1, std::min(P.ntiles, cus * 8));
+  return reduction == 0 ? combine_shape<0>(P, D, grid, s) : combine_shape<1>(P, D, grid, s);
 }
 
 hipError_t launch_deposit(const Plan& P, const DepArgs& D, int reduction, int grid, int block, hipStream_t s) {

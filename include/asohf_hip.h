@@ -96,7 +96,8 @@ typedef struct asohf_tune {
 typedef struct asohf_stats {
   int64_t n_particles;
   int64_t n_pairs;          /* (particle, grid) members under the mode's box rule */
-  int64_t n_entries;        /* binned (particle, tile) entries                     */
+  int64_t n_entries;        /* binned entries: one per 27-cell member, one per tile
+                               touched by a wider table-mode member                */
   int64_t n_tiles;
   int64_t n_items;          /* work items of the persistent deposit                */
   int64_t n_cells;          /* output cells written                                */
@@ -105,7 +106,7 @@ typedef struct asohf_stats {
   double ms_scatter;        /* scatter of the entries                              */
   double ms_deposit;        /* the persistent deposit kernel alone                 */
   double ms_sums;           /* item writing and grid sums                          */
-  double ms_split;          /* summation of split tiles' partials (split_reduce)   */
+  double ms_split;          /* output cells from the tiles' sums (combine_tiles)    */
 } asohf_stats;
 
 /* Context. device < 0 selects the current device. */
