@@ -151,8 +151,9 @@ struct PipeArgs {
   unsigned long long* start;
   unsigned long long* cursor;
   unsigned long long* bsum;
-  unsigned* nitems;
-  unsigned long long* item_off;
+  unsigned* nitems;                 // items per tile
+  unsigned* icnt;                   // narrow items per tile, then wide items per tile
+  unsigned long long* item_off;     // offsets of both
   double* grid_mass;
   long long nblk;
   long long nkeys;
@@ -175,7 +176,7 @@ struct asohf_ctx {
   asohf_tune tune{{16, 8, 8}, 256, 4096, 16};
   HostPlan plan;
   DBuf plan_blob;
-  DBuf cnt, start, cursor, bsum, counters, nitems, tmass, entries, items, scratch;
+  DBuf cnt, start, cursor, bsum, counters, nitems, icnt, tmass, entries, items, scratch;
   DBuf flags, idx, pool, pool_off, pool_nk, blk_pairs, blk_mmax, item_off;
   DBuf elist, eoff, ecount;
   DBuf ipairs;                             // members found per work item (TSC hierarchy binning)
@@ -795,7 +796,8 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   HIPCHK(ctx->bsum.ensure(sizeof(unsigned long long) * scan_scratch_elems(nkeys)), "allocating scan");
   HIPCHK(ctx->counters.ensure(sizeof(Counters)), "allocating counters");
   HIPCHK(ctx->nitems.ensure(sizeof(unsigned) * std::max(ntiles, 1)), "allocating tile state");
-  HIPCHK(ctx->item_off.ensure(sizeof(unsigned long long) * (ntiles + 1)), "allocating tile state");
+  HIPCHK(ctx->icnt.ensure(sizeof(unsigned) * 2 * std::max(ntiles, 1)), "allocating tile state");
+  HIPCHK(ctx->item_off.ensure(sizeof(unsigned long long) * (2ll * ntiles + 1)), "allocating tile state");
   HIPCHK(ctx->tmass.ensure(sizeof(double) * std::max(ntiles, 1)), "allocating tile sums");
   HIPCHK(ctx->scratch.ensure((size_t)std::max(ntiles, 1) * exchange_cells(a.P.tile) * a.elem),
          "allocating exchange cells");
@@ -831,14 +833,16 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   a.cursor = ctx->cursor.as<unsigned long long>();
   a.bsum = ctx->bsum.as<unsigned long long>();
   a.nitems = ctx->nitems.as<unsigned>();
+  a.icnt = ctx->icnt.as<unsigned>();
   a.item_off = ctx->item_off.as<unsigned long long>();
   a.grid_mass = grid_mass;
   a.chunk = std::max(ctx->tune.chunk, 64);
   // wide table-mode entries: a tile's classes are deposited in the
   // histogram form (a fixed cost per tile and class) when one work item
   // holds all of the tile's wide entries, otherwise (and for the widest
-  // classes) entry by entry; items of up to 8 chunks of entries
-  a.chunk_wide = a.chunk * 8;
+  // classes) entry by entry, which costs hundreds of adds each; so items are
+  // long (2^20 masses below 2^30 units sum below 2^53, exact in FP64)
+  a.chunk_wide = (int)std::min(std::max(a.chunk, 1 << 17) * 8ll, 1ll << 22);
   a.cus = ctx->cus;
   const int waves = std::max(ctx->tune.waves_per_cu, 1);
   a.block = ctx->tune.block;
@@ -870,16 +874,16 @@ static asohf_status enqueue_count(asohf_ctx* ctx, const PipeArgs& a, hipStream_t
   HIPCHK(launch_count(a.P, a.A, a.cnt, a.C, a.BT, a.cus, s), "count kernel");
   if (a.A.n > 0) HIPCHK(launch_reduce_blocks(a.BT, bin_blocks(a.A.n), a.C, a.cus, s), "block sums");
   HIPCHK(launch_scan(a.cnt, a.nkeys, a.bsum, a.start, a.cursor, s), "scan");
-  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, a.chunk_wide, a.nitems, s),
+  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, a.chunk_wide, a.icnt, a.nitems, s),
          "planning items");
-  HIPCHK(launch_scan(a.nitems, a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
+  HIPCHK(launch_scan(a.icnt, 2ll * a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
   return ASOHF_OK;
 }
 
 // gate, scatter, item plan, persistent deposit, grid sums; events between the
 // phases unless the sequence is being captured
 static asohf_status enqueue_deposit(asohf_ctx* ctx, const PipeArgs& a, hipStream_t s, bool events) {
-  HIPCHK(launch_gate(a.start + a.nkeys, a.item_off + a.ntiles, a.cap_entries, a.cap_items, a.C, s), "gate");
+  HIPCHK(launch_gate(a.start + a.nkeys, a.item_off, a.ntiles, a.cap_entries, a.cap_items, a.C, s), "gate");
   if (events) HIPCHK(hipEventRecord(ctx->ev[2], s), "event");
   HIPCHK(launch_scatter(a.P, a.A, a.cursor, const_cast<int4*>(a.D.entries), a.cap_entries, a.BT, a.C, a.cus, s), "scatter kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[3], s), "event");
@@ -888,6 +892,7 @@ static asohf_status enqueue_deposit(asohf_ctx* ctx, const PipeArgs& a, hipStream
   HIPCHK(launch_zero_split(a.P, a.D, a.red, a.cus, s), "clearing split tiles");
   if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
   HIPCHK(launch_deposit(a.P, a.D, a.red, a.grid, a.block, s), "deposit kernel");
+  if (a.P.nl > 0) HIPCHK(launch_deposit_wide(a.P, a.D, a.red, a.cus, s), "wide deposit kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[8], s), "event");
   HIPCHK(launch_combine(a.P, a.D, a.red, a.cus, s), "output cells");
   if (events) HIPCHK(hipEventRecord(ctx->ev[5], s), "event");
@@ -931,7 +936,7 @@ static asohf_status run_exact(asohf_ctx* ctx, const asohf_opts& o, const Parts& 
   HIPCHK(hipMemcpyAsync(ctx->hcount, a.C, sizeof(Counters), hipMemcpyDeviceToHost, s), "reading counters");
   HIPCHK(hipMemcpyAsync(ctx->hscalar, a.start + a.nkeys, sizeof(unsigned long long), hipMemcpyDeviceToHost, s),
          "reading totals");
-  HIPCHK(hipMemcpyAsync(ctx->hscalar + 1, a.item_off + a.ntiles, sizeof(unsigned long long),
+  HIPCHK(hipMemcpyAsync(ctx->hscalar + 1, a.item_off + 2ll * a.ntiles, sizeof(unsigned long long),
                         hipMemcpyDeviceToHost, s), "reading totals");
   HIPCHK(hipStreamSynchronize(s), "count pass");
   Counters hc = *ctx->hcount;
@@ -974,9 +979,9 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   HIPCHK(launch_count(a.P, a.A, a.cnt, a.C, a.BT, a.cus, s), "count kernel");
   HIPCHK(launch_count_to_capacity(a.cnt, a.nkeys, a.cus, s), "capacities");
   HIPCHK(launch_scan(a.cnt, a.nkeys, a.bsum, a.start, a.cursor, s), "scan");
-  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, 0, a.nitems, s),
+  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, 0, a.icnt, a.nitems, s),
          "planning items");
-  HIPCHK(launch_scan(a.nitems, a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
+  HIPCHK(launch_scan(a.icnt, 2ll * a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
   const int nl = a.P.nl;
   HIPCHK(hipMemcpyAsync(ctx->hcount, a.C, sizeof(Counters), hipMemcpyDeviceToHost, s), "reading counters");
   HIPCHK(hipMemcpyAsync(ctx->hscalar, a.start + a.nkeys, sizeof(unsigned long long), hipMemcpyDeviceToHost, s),
@@ -1301,7 +1306,7 @@ void asohf_hip_destroy(asohf_ctx* ctx) {
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
                   &ctx->item_off, &ctx->plan_blob, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum, &ctx->counters,
-                  &ctx->nitems, &ctx->tmass, &ctx->entries, &ctx->items,
+                  &ctx->nitems, &ctx->icnt, &ctx->tmass, &ctx->entries, &ctx->items,
                   &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1], &ctx->h_in[2],
                   &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0], &ctx->ord[1],
                   &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount, &ctx->sp_k[0],
@@ -2256,7 +2261,7 @@ asohf_status asohf_hip_release_workspaces(asohf_ctx* ctx) {
   ctx->gexec = nullptr;
   DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
                   &ctx->item_off, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum,
-                  &ctx->nitems, &ctx->tmass, &ctx->entries,
+                  &ctx->nitems, &ctx->icnt, &ctx->tmass, &ctx->entries,
                   &ctx->items, &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1],
                   &ctx->h_in[2], &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0],
                   &ctx->ord[1], &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount,

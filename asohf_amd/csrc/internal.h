@@ -134,11 +134,13 @@ struct Counters {
   unsigned int mmax_bits;         // max particle mass, as FP32 bits (masses >= 0)
   unsigned int overflow;          // 1: a workspace was smaller than this call needs; the
                                   // scatter, planning and deposit kernels then do nothing
-  unsigned int n_items_eff;       // items the deposit serves (0 after an overflow)
-  unsigned int pad[kLine - 12];
+  unsigned int n_items_eff;       // narrow items the deposit serves (0 after an overflow)
+  unsigned int n_wide_eff;        // wide items, which follow the narrow ones
+  unsigned int pad[kLine - 13];
   unsigned long long pool_fill[kPoolSubs * kLine / 2];   // sub-pool k at [k * kLine / 2]
   unsigned long long epool_fill[kPoolSubs * kLine / 2];  // emission lists, same layout
   unsigned int queue[kQueues * kLine];                   // queue q at [q * kLine]
+  unsigned int wqueue[kQueues * kLine];                  // the same for the wide items
   unsigned int equeue[kNLevels * kLine];                 // emission pass of level l at [l * kLine]
 };
 
@@ -149,7 +151,7 @@ static_assert(sizeof(unsigned long long) * 4 + sizeof(unsigned) * (kLine - 8) ==
 struct Item {
   int tile;
   int flags;                 // bit 0: wide (table-mode N >= 2) entries; bit 1: every wide entry
-                             // of the tile; bits 8+: the item's rank within its tile
+                             // of the tile
   long long begin;           // entry range [begin, end)
   long long end;
 };
@@ -192,9 +194,6 @@ struct DepArgs {
   // range is filled)
   const unsigned long long* cursor;
   const unsigned long long* start;
-  int hist_cells;            // table mode: int64 cells of the wide classes' histogram buffer
-                             // (dynamic LDS, set by the launcher; 0: every class walks directly)
-  int pad2;
 };
 
 enum : int { kErrNonFinite = 1, kErrWrap = 2, kErrNegMass = 4, kErrIndexRange = 8 };

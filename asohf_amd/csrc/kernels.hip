@@ -19,11 +19,6 @@
 
 namespace asohf {
 
-// LDS copy of the kernel table rows 0..kNLevels: row irk holds 2^(irk+1) + 1
-// values and starts after the rows below it
-__host__ __device__ constexpr int ktab_off(int irk) { return (2 << irk) - 2 + irk; }
-constexpr int kKtabLds = ktab_off(kNLevels + 1);
-
 // ---------------------------------------------------------------------------
 // fills (used instead of hipMemsetAsync so every step can live in a graph)
 // ---------------------------------------------------------------------------
@@ -450,9 +445,10 @@ __global__ void __launch_bounds__(kScanThreads) scan_apply(const unsigned* in, l
 // ---------------------------------------------------------------------------
 // work items
 // ---------------------------------------------------------------------------
-// Work items.  plan_count: items per tile; after an exclusive scan,
-// plan_write places every tile's items at its offset (no atomics: the item
-// order is the tile order).  With chunk_wide = 0 the tile's whole range
+// Work items.  plan_count: items per tile, narrow ones in cnt[t], wide ones in
+// cnt[ntiles + t]; after one exclusive scan over both halves, plan_write places
+// every tile's items (no atomics): all narrow items in tile order, then all
+// wide items.  With chunk_wide = 0 the tile's whole range
 // [start[2t], start[2t+2]) is chunked as narrow entries (the TSC hierarchy
 // binning, which uses the keys 2t only).
 __device__ __forceinline__ void tile_chunks(const unsigned long long* start, int t, int chunk, int chunk_wide,
@@ -469,12 +465,14 @@ __device__ __forceinline__ void tile_chunks(const unsigned long long* start, int
 }
 
 __global__ void plan_count(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                           unsigned* nitems_tile) {
+                           unsigned* cnt, unsigned* nitems_tile) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ntiles) return;
   long long s0, s1, s2;
   int cn, cw;
   tile_chunks(start, t, chunk, chunk_wide, s0, s1, s2, cn, cw);
+  cnt[t] = (unsigned)cn;
+  cnt[ntiles + t] = (unsigned)cw;
   nitems_tile[t] = (unsigned)(cn + cw);   // none for a tile without entries
 }
 
@@ -485,18 +483,18 @@ __global__ void plan_write(const unsigned long long* start, int ntiles, int chun
   long long s0, s1, s2;
   int cn, cw;
   tile_chunks(start, t, chunk, chunk_wide, s0, s1, s2, cn, cw);
-  const long long base = (long long)item_off[t];
-  int k = 0;
+  long long k = (long long)item_off[t];
   for (int c = 0; c < cn; ++c, ++k) {
     const long long b = s0 + (long long)c * chunk;
-    items[base + k] = Item{t, k << 8, b, min(b + (long long)chunk, s1)};
+    items[k] = Item{t, 0, b, min(b + (long long)chunk, s1)};
   }
   // bit 1: the item holds every wide entry of its tile (the histogram form
   // is used only then, so its one rounding per cell does not depend on how
   // the entries fall into items)
+  k = (long long)item_off[ntiles + t];
   for (int c = 0; c < cw; ++c, ++k) {
     const long long b = s1 + (long long)c * chunk_wide;
-    items[base + k] = Item{t, 1 | (cw == 1 ? 2 : 0) | (k << 8), b, min(b + (long long)chunk_wide, s2)};
+    items[k] = Item{t, 1 | (cw == 1 ? 2 : 0), b, min(b + (long long)chunk_wide, s2)};
   }
 }
 
@@ -504,15 +502,16 @@ __global__ void plan_write(const unsigned long long* start, int ntiles, int chun
 // call whose buffers were sized by an earlier call finds out here, on the
 // device, whether they still suffice; if not, every later kernel of the call
 // does nothing and the host rebuilds with exact sizes.
-__global__ void gate_kernel(const unsigned long long* tot_entries, const unsigned long long* tot_items,
+__global__ void gate_kernel(const unsigned long long* tot_entries, const unsigned long long* item_off, int ntiles,
                             unsigned long long cap_entries, unsigned long long cap_items, Counters* C) {
   if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  const unsigned long long ne = *tot_entries, ni = *tot_items;
+  const unsigned long long ne = *tot_entries, nn = item_off[ntiles], ni = item_off[2 * ntiles];
   C->n_entries = ne;
   C->n_items = ni;
   const bool over = ne > cap_entries || ni > cap_items || ni >= (1ull << 31);
   C->overflow = over ? 1u : 0u;
-  C->n_items_eff = over ? 0u : (unsigned)ni;
+  C->n_items_eff = over ? 0u : (unsigned)nn;
+  C->n_wide_eff = over ? 0u : (unsigned)(ni - nn);
 }
 
 // Fixed-point scale of the deterministic reduction: the power of two with
@@ -788,78 +787,6 @@ __device__ __forceinline__ bool tile_filled(const DepArgs& D, int t) {
   return D.cursor ? D.cursor[2 * t] > D.start[2 * t] : D.start[2 * t + 2] > D.start[2 * t];
 }
 
-// The wide entries of one class (kernel level irk, half-width N) of a work
-// item, in the histogram form: the fixed-point masses of the class's members
-// summed at their cells (the reference's IX, JY, KZ) on the tile's box
-// extended by N cells (every member of the item has its cell there: its box
-// meets the tile), exact int64 sums; then the kernel row applied along x, y
-// and z in FP64, each pass in place on the buffer; the result, rounded once
-// per cell, is added to the tile's accumulator.  Cells of the tile outside
-// the grid receive values that are never written out.
-template <int RED, int TX, int TY, int TZ>
-__device__ void wide_histogram_form(const DepArgs& D, const Item& it, int irk, int i0, int j0, int k0c,
-                                    const float* K, float scale, double dscale,
-                                    typename AccT<RED>::T* acc, long long* hist) {
-  using Acc = typename AccT<RED>::T;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int nk = 1 << irk;
-  const int bx = TX + 2 * nk, by = TY + 2 * nk, bz = TZ + 2 * nk, nb = bx * by * bz;
-  double* hd = reinterpret_cast<double*>(hist);
-  auto at = [](int a, int b, int c) { return TileLds<TX, TY, TZ>::at(a, b, c); };
-  for (int c = tid; c < nb; c += nthr) hist[c] = 0;
-  __syncthreads();
-  for (long long e = it.begin + tid; e < it.end; e += nthr) {
-    int ci[3], irk_e;
-    float m;
-    unpack_table(D.entries[e], ci[0], ci[1], ci[2], irk_e, m);
-    if (irk_e != irk) continue;
-    const int hx = ci[0] - i0 + nk, hy = ci[1] - j0 + nk, hz = ci[2] - k0c + nk;
-    if (hx < 0 || hx >= bx || hy < 0 || hy >= by || hz < 0 || hz >= bz) continue;
-    atomicAdd(reinterpret_cast<unsigned long long*>(hist + hx + bx * (hy + by * hz)),
-              (unsigned long long)__float2ll_rn(m * scale));
-  }
-  __syncthreads();
-  for (int c = tid; c < nb; c += nthr) hd[c] = (double)hist[c];
-  __syncthreads();
-  // x: every (y, z) row of the box; out(xo) = sum_d row(xo + N - d) K(d),
-  // written over row(xo), which no later output of the row reads
-  for (int r = tid; r < by * bz; r += nthr) {
-    double* row = hd + r * bx;
-    for (int xo = 0; xo < TX; ++xo) {
-      double s = 0.0;
-      for (int d = -nk; d <= nk; ++d) s += row[xo + nk - d] * (double)K[d];
-      row[xo] = s;
-    }
-  }
-  __syncthreads();
-  // y: every column (x of the tile, z of the box)
-  for (int r = tid; r < TX * bz; r += nthr) {
-    double* col = hd + (r % TX) + bx * by * (r / TX);
-    for (int yo = 0; yo < TY; ++yo) {
-      double s = 0.0;
-      for (int d = -nk; d <= nk; ++d) s += col[bx * (yo + nk - d)] * (double)K[d];
-      col[bx * yo] = s;
-    }
-  }
-  __syncthreads();
-  // z: every (x, y) of the tile, into the accumulator
-  const double inv_scale = 1.0 / dscale;   // a power of two: exact
-  for (int r = tid; r < TX * TY; r += nthr) {
-    const int xo = r % TX, yo = r / TX;
-    const double* col = hd + xo + bx * yo;
-    for (int zo = 0; zo < TZ; ++zo) {
-      double s = 0.0;
-      for (int d = -nk; d <= nk; ++d) s += col[bx * by * (zo + nk - d)] * (double)K[d];
-      if (s != 0.0) {
-        Acc* dst = acc + at(xo, yo, zo);
-        if (RED == 0) *reinterpret_cast<long long*>(dst) += __double2ll_rn(s);
-        else *reinterpret_cast<float*>(dst) += (float)(s * inv_scale);
-      }
-    }
-  }
-  __syncthreads();
-}
-
 template <int MODE, int RED, int TX, int TY, int TZ>
 __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
   using Acc = typename AccT<RED>::T;
@@ -867,26 +794,10 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
   constexpr int HX = L::HX, HY = L::HY, H = L::H;
   __shared__ Acc acc[H];
   __shared__ unsigned s_item;
-  // table mode: the used part of the kernel table, row irk (2^(irk+1) + 1
-  // values) at ktab_off(irk), centred at ktab_off(irk) + 2^irk
-  __shared__ float s_ktab[MODE == 1 ? kKtabLds : 1];
-  __shared__ unsigned s_ccnt[kNLevels + 1];
-  // table mode: the histogram buffer of the wide classes (dynamic LDS,
-  // D.hist_cells int64 cells)
-  extern __shared__ long long s_hist[];
   const int tid = threadIdx.x, nthr = blockDim.x;
-  const double dscale = fixed_scale(D.C->mmax_bits);
-  const float scale = (float)dscale;
+  const float scale = (float)fixed_scale(D.C->mmax_bits);
   const unsigned n_items = D.C->n_items_eff;
   const float k0[3] = {P.ktab[P.kmax - 1], P.ktab[P.kmax], P.ktab[P.kmax + 1]};
-  if (MODE == 1) {
-    for (int irk = 0; irk <= P.nl; ++irk) {
-      const int w = 2 * (1 << irk) + 1;
-      for (int j = tid; j < w; j += nthr)
-        s_ktab[ktab_off(irk) + j] = P.ktab[irk * P.kw + P.kmax - (1 << irk) + j];
-    }
-    // the first item's __syncthreads orders these writes before any read
-  }
   auto at = [](int a, int b, int c) { return L::at(a, b, c); };
 
   // workgroup w serves queue w mod n_queues, which hands out items
@@ -905,7 +816,6 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     const int local = t - G.tile0;
     const int tx = local % G.nt[0], ty = (local / G.nt[0]) % G.nt[1], tz = local / (G.nt[0] * G.nt[1]);
     const int i0 = tx * TX + 1, j0 = ty * TY + 1, k0c = tz * TZ + 1;
-    const int ex = min(TX, G.n[0] - i0 + 1), ey = min(TY, G.n[1] - j0 + 1), ez = min(TZ, G.n[2] - k0c + 1);
     const bool periodic = g == 0;
 
     // the item's filled entries: with the hierarchy binning the tile's
@@ -920,158 +830,64 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     for (int c = tid; c < H; c += nthr) acc[c] = 0;
     __syncthreads();
 
-    if (!(it.flags & 1)) {
-      // ---- narrow entries: one lane per entry, 27 cells.  Lane j of the
-      // workgroup takes entries j, j + nthr, ... of the item, so a wave reads
-      // 64 consecutive entries (1 KB, every entry fetched once).  Two entries
-      // per pass, in two registers refilled right after use (register copies
-      // would wait on the loads); the prefetch indices are clamped into the
-      // item instead of tested, so every pass issues the same loads, and the
-      // loop runs the same number of passes on every lane (ok = the lane holds
-      // an entry), which the lane merging of the TSC deposit needs.
-      const int4* const eb = D.entries + uniform64(it.begin);
-      auto narrow = [&](const int4 v, const bool ok) {
-        int ci[3];
-        float wx[3], wy[3], wz[3], m;
-        if (MODE == 2) {
-          const float p[3] = {__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z)};
-          m = __int_as_float(v.w);
-          float* w[3] = {wx, wy, wz};
-          // weights from the three centres RAD(I-1..I+1) on the base grid,
-          // MINIRADX(I-1..I+1) on a patch; the indices are the reference's
-          if (g == 0) {
+    // ---- narrow entries: one lane per entry, 27 cells.  Lane j of the
+    // workgroup takes entries j, j + nthr, ... of the item, so a wave reads
+    // 64 consecutive entries (1 KB, every entry fetched once).  Two entries
+    // per pass, in two registers refilled right after use (register copies
+    // would wait on the loads); the prefetch indices are clamped into the
+    // item instead of tested, so every pass issues the same loads, and the
+    // loop runs the same number of passes on every lane (ok = the lane holds
+    // an entry), which the lane merging of the TSC deposit needs.
+    const int4* const eb = D.entries + uniform64(it.begin);
+    auto narrow = [&](const int4 v, const bool ok) {
+      int ci[3];
+      float wx[3], wy[3], wz[3], m;
+      if (MODE == 2) {
+        const float p[3] = {__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z)};
+        m = __int_as_float(v.w);
+        float* w[3] = {wx, wy, wz};
+        // weights from the three centres RAD(I-1..I+1) on the base grid,
+        // MINIRADX(I-1..I+1) on a patch; the indices are the reference's
+        if (g == 0) {
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-              ci[a] = tsc_base_index(p[a], P.xl, G.d[a], G.inv_d[a], G.n[a]);
-              tsc_weights_f64(p[a], base_centre(P, a, ci[a] - 1, G.n[a]), base_centre(P, a, ci[a], G.n[a]),
-                              base_centre(P, a, ci[a] + 1, G.n[a]), G.inv_dd[a], w[a]);
-            }
-          } else {
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-              ci[a] = (int)index_quotient(p[a] - G.org[a], G.d[a], G.inv_d[a]);
-              tsc_weights_f64(p[a], minirad(G.pr[a], ci[a] - 1, G.d[a]), minirad(G.pr[a], ci[a], G.d[a]),
-                              minirad(G.pr[a], ci[a] + 1, G.d[a]), G.inv_dd[a], w[a]);
-            }
+          for (int a = 0; a < 3; ++a) {
+            ci[a] = tsc_base_index(p[a], P.xl, G.d[a], G.inv_d[a], G.n[a]);
+            tsc_weights_f64(p[a], base_centre(P, a, ci[a] - 1, G.n[a]), base_centre(P, a, ci[a], G.n[a]),
+                            base_centre(P, a, ci[a] + 1, G.n[a]), G.inv_dd[a], w[a]);
           }
         } else {
-          int irk;
-          unpack_table(v, ci[0], ci[1], ci[2], irk, m);
 #pragma unroll
-          for (int k = 0; k < 3; ++k) { wx[k] = k0[k]; wy[k] = k0[k]; wz[k] = k0[k]; }
-        }
-        // in [-1, ext] by construction of the binning; clamped so the array
-        // bounds never depend on that
-        const int lx = clampi((periodic ? wrap1(ci[0], G.n[0]) : ci[0]) - i0, -1, TX);
-        const int ly = clampi((periodic ? wrap1(ci[1], G.n[1]) : ci[1]) - j0, -1, TY);
-        const int lz = clampi((periodic ? wrap1(ci[2], G.n[2]) : ci[2]) - k0c, -1, TZ);
-        const int corner = at(lx - 1, ly - 1, lz - 1);
-        if (MODE == 2 || P.merge_narrow)
-          deposit27_merged<RED, HX, HY>(acc, corner, ok, m, wx, wy, wz, scale);
-        else if (ok)
-          deposit27<RED, HX, HY>(acc + corner, m, wx, wy, wz, scale);
-      };
-      // entry j of the item (j clamped to the last one)
-      auto at_j = [&](long long j) { return eb[min(j, len - 1)]; };
-      int4 va = at_j(tid), vb = at_j(tid + nthr);
-      for (long long o = 0; o < len; o += 2 * nthr) {
-        narrow(va, o + tid < len);
-        va = at_j(o + 2 * nthr + tid);
-        narrow(vb, o + nthr + tid < len);
-        vb = at_j(o + 3 * nthr + tid);
-      }
-    } else if (MODE == 1) {
-      // ---- wide table-mode entries (kernel level irk >= 1, half-width
-      // N = 2^irk), one class at a time.  Classes whose halo-extended box
-      // fits the histogram buffer: an NGP histogram of the members' masses
-      // at their cells, then the separable kernel, three 1-D passes (the
-      // histogram form of grids.f:888-951).  Larger classes: the direct walk
-      // of every entry's clipped box. ----
-      // entries per class (wave ballots, one LDS add per wave and class)
-      if (tid <= kNLevels) s_ccnt[tid] = 0u;
-      __syncthreads();
-      {
-        unsigned cnt[kNLevels + 1] = {};
-        for (long long b0 = it.begin; b0 < it.end; b0 += nthr) {
-          const long long e = b0 + tid;
-          const int irk_e = e < it.end ? (D.entries[e].y >> 16) : 0;
-#pragma unroll
-          for (int k = 1; k <= kNLevels; ++k) cnt[k] += (unsigned)__popcll(__ballot(irk_e == k));
-        }
-        if ((tid & 63) == 0)
-          for (int k = 1; k <= kNLevels; ++k)
-            if (cnt[k]) atomicAdd(&s_ccnt[k], cnt[k]);
-      }
-      __syncthreads();
-      for (int irk = 1; irk <= kNLevels; ++irk) {
-        const unsigned ncls = s_ccnt[irk];
-        if (ncls == 0u) continue;
-        const int nk = 1 << irk;
-        const float* K = s_ktab + ktab_off(irk) + nk;   // K[d], d in [-N, N]
-        const int bx = TX + 2 * nk, by = TY + 2 * nk, bz = TZ + 2 * nk;
-        // the histogram form when its buffer fits and its three passes cost
-        // less than the entries' direct adds (an LDS add counted as four
-        // FP64 multiply-adds)
-        const long long w = 2 * nk + 1;
-        const long long passes = w * ((long long)bx * by * TX + (long long)TX * bz * TY + (long long)TX * TY * TZ);
-        if ((it.flags & 2) && bx * by * bz <= D.hist_cells && 4ll * ncls * w * w * w > passes) {
-          wide_histogram_form<RED, TX, TY, TZ>(D, it, irk, i0, j0, k0c, K, scale, dscale, acc, s_hist);
-          continue;
-        }
-        // direct: one wave per entry.  The entry's box clipped to the tile
-        // (bx x by x bz cells) is walked as one flat range, lane l taking
-        // cells l, l + 64, ...; its (x, y, z) counters advance by constant
-        // steps, so the loop has no divisions.  Kernel values come from the
-        // LDS copy of the table; the next entry is loaded while this one
-        // deposits.  Terms are ((m*Kx)*Ky)*Kz as in the reference's loop.
-        const int wave = tid >> 6, lane = tid & 63, nwaves = nthr >> 6;
-        long long e = it.begin + wave;
-        int4 nxt = e < it.end ? D.entries[e] : make_int4(0, 0, 0, 0);
-        for (; e < it.end; e += nwaves) {
-          int ci[3], irk_e;
-          float m;
-          unpack_table(nxt, ci[0], ci[1], ci[2], irk_e, m);
-          if (e + nwaves < it.end) nxt = D.entries[e + nwaves];
-          if (irk_e != irk) continue;
-          const int xa = max(max(ci[0] - nk, 1), i0), xb = min(min(ci[0] + nk, G.n[0]), i0 + ex - 1);
-          const int ya = max(max(ci[1] - nk, 1), j0), yb = min(min(ci[1] + nk, G.n[1]), j0 + ey - 1);
-          const int za = max(max(ci[2] - nk, 1), k0c), zb = min(min(ci[2] + nk, G.n[2]), k0c + ez - 1);
-          if (xb < xa || yb < ya || zb < za) continue;
-          const int cx = xb - xa + 1, cy = yb - ya + 1, total = cx * cy * (zb - za + 1);
-          // q / n for q <= 64 * 16 and n <= 16: (q + 1/2) / n is at least 1/32
-          // away from an integer, far beyond the FP32 error of the product
-          const float rbx = 1.0f / (float)cx, rby = 1.0f / (float)cy;
-          auto divn = [](int q, float rn) { return (int)(((float)q + 0.5f) * rn); };
-          const int r0 = divn(lane, rbx);
-          int a = lane - r0 * cx;
-          int c = divn(r0, rby);
-          int b = r0 - c * cy;
-          const int dr = divn(64, rbx), da = 64 - dr * cx;
-          const int dc0 = divn(dr, rby), db0 = dr - dc0 * cy;
-          const int dc1 = divn(dr + 1, rby), db1 = dr + 1 - dc1 * cy;
-          const float ms = RED == 0 ? m * scale : m;
-          const float* Kx = K + (xa - ci[0]);
-          const float* Ky = K + (ya - ci[1]);
-          const float* Kz = K + (za - ci[2]);
-          Acc* base = acc + at(xa - i0, ya - j0, za - k0c);
-          for (int q2 = lane; q2 < total; q2 += 64) {
-            const float term = ((ms * Kx[a]) * Ky[b]) * Kz[c];
-            Acc* dst = base + (a + HX * (b + HY * c));
-            if (RED == 0) lds_add(reinterpret_cast<long long*>(dst), (long long)__float2int_rn(term));
-            else lds_add(reinterpret_cast<float*>(dst), term);
-            a += da;
-            const bool carry = a >= cx;
-            if (carry) a -= cx;
-            b += carry ? db1 : db0;
-            c += carry ? dc1 : dc0;
-            if (b >= cy) {
-              b -= cy;
-              ++c;
-            }
+          for (int a = 0; a < 3; ++a) {
+            ci[a] = (int)index_quotient(p[a] - G.org[a], G.d[a], G.inv_d[a]);
+            tsc_weights_f64(p[a], minirad(G.pr[a], ci[a] - 1, G.d[a]), minirad(G.pr[a], ci[a], G.d[a]),
+                            minirad(G.pr[a], ci[a] + 1, G.d[a]), G.inv_dd[a], w[a]);
           }
         }
-        __syncthreads();
+      } else {
+        int irk;
+        unpack_table(v, ci[0], ci[1], ci[2], irk, m);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { wx[k] = k0[k]; wy[k] = k0[k]; wz[k] = k0[k]; }
       }
+      // in [-1, ext] by construction of the binning; clamped so the array
+      // bounds never depend on that
+      const int lx = clampi((periodic ? wrap1(ci[0], G.n[0]) : ci[0]) - i0, -1, TX);
+      const int ly = clampi((periodic ? wrap1(ci[1], G.n[1]) : ci[1]) - j0, -1, TY);
+      const int lz = clampi((periodic ? wrap1(ci[2], G.n[2]) : ci[2]) - k0c, -1, TZ);
+      const int corner = at(lx - 1, ly - 1, lz - 1);
+      if (MODE == 2 || P.merge_narrow)
+        deposit27_merged<RED, HX, HY>(acc, corner, ok, m, wx, wy, wz, scale);
+      else if (ok)
+        deposit27<RED, HX, HY>(acc + corner, m, wx, wy, wz, scale);
+    };
+    // entry j of the item (j clamped to the last one)
+    auto at_j = [&](long long j) { return eb[min(j, len - 1)]; };
+    int4 va = at_j(tid), vb = at_j(tid + nthr);
+    for (long long o = 0; o < len; o += 2 * nthr) {
+      narrow(va, o + tid < len);
+      va = at_j(o + 2 * nthr + tid);
+      narrow(vb, o + nthr + tid < len);
+      vb = at_j(o + 3 * nthr + tid);
     }
     __syncthreads();
 
@@ -1088,6 +904,316 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
       }
     }
     __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// wide table-mode entries (kernel level irk >= 1, half-width N = 2^irk)
+// ---------------------------------------------------------------------------
+constexpr int kWideThreads = 512;
+constexpr int kWideCells = 8192;   // histogram cells (64 KB: two workgroups per CU)
+constexpr int kWideK = 2 * 64 + 1;  // longest kernel row of a histogram form (form 2 fits up to N = 32)
+
+// How a class's histogram is laid out for a block of BX x BY x BZ cells.  The
+// field of the class is the masses summed at their cells, convolved with the
+// kernel row along x, y and z (the histogram form of grids.f:888-951).  The
+// more of the convolution an entry does itself, the smaller the histogram:
+//   0  the mass at its cell: (BX+2N)(BY+2N)(BZ+2N) cells, one add per entry
+//   1  the mass times its kernel column: (BX+2N)(BY+2N) BZ cells, BZ adds
+//   2  the mass times its kernel plane: (BX+2N) BY BZ cells, BY BZ adds
+// 0 is taken while it fits, then 1, then 2; -1: none fits.  Row and plane
+// pitches keep the lanes of a pass on different LDS banks.
+struct WideShape {
+  int form, ny, nz, px, pz, cells;
+};
+template <int BX, int BY, int BZ>
+__host__ __device__ __forceinline__ WideShape wide_shape(int nk) {
+  WideShape w;
+  for (int f = 0; f < 3; ++f) {
+    w.form = f;
+    w.ny = f < 2 ? BY + 2 * nk : BY;
+    w.nz = f < 1 ? BZ + 2 * nk : BZ;
+    w.px = (BX + 2 * nk) | 1;
+    w.pz = w.px * w.ny;
+    w.cells = w.pz * w.nz;
+    // the x pass holds at most two groups of four outputs per thread
+    if (w.cells <= kWideCells && w.ny * w.nz * (BX / 4) <= 2 * kWideThreads) return w;
+  }
+  w.form = -1;
+  return w;
+}
+
+// Four outputs o..o+3 of a kernel row of half-width nk applied to a line of
+// stride st: s[i] = sum_j line[i + j] K[j - nk], j ascending.
+__device__ __forceinline__ void conv4(const double* line, int st, int nk, const double* K, double s[4]) {
+  double a = line[0], b = line[st], c = line[2 * st], d = line[3 * st];
+  const double* p = line + 4 * st;
+  s[0] = s[1] = s[2] = s[3] = 0.0;
+  auto tap = [&](double k, double w, double x, double y, double z) {
+    s[0] = __fma_rn(w, k, s[0]);
+    s[1] = __fma_rn(x, k, s[1]);
+    s[2] = __fma_rn(y, k, s[2]);
+    s[3] = __fma_rn(z, k, s[3]);
+  };
+  // 2 nk + 1 taps, nk even: four at a time, the window's registers in rotation
+#pragma unroll 1
+  for (int j = 0; j < 2 * nk; j += 4) {
+    tap(K[j], a, b, c, d);
+    a = p[0];
+    tap(K[j + 1], b, c, d, a);
+    b = p[st];
+    tap(K[j + 2], c, d, a, b);
+    c = p[2 * st];
+    tap(K[j + 3], d, a, b, c);
+    d = p[3 * st];
+    p += 4 * st;
+  }
+  tap(K[2 * nk], a, b, c, d);
+}
+
+// The wide items, persistent over 8 queues like the deposit.  A tile is taken
+// in blocks of at most 16 x 8 x 8 cells, a block class by class: the class's
+// masses (or masses times kernel values, see wide_shape) summed as exact
+// int64 fixed point on the histogram, then the remaining axes of the
+// convolution in FP64, each cell rounded once to the fixed-point unit.  The
+// histogram form is used when the item holds all of the tile's wide entries
+// (its rounding must not depend on how entries fall into items) and costs
+// fewer operations than adding every entry's clipped box cell by cell (an LDS
+// add counted as four FP64 multiply-adds).
+// Bound by reading the entries once per class and by the LDS reads of the
+// convolution.  As part of the narrow kernel the histogram had one layout, so
+// N = 8 and more walked every entry's box (29 G adds at 512^3, 6 levels), and
+// its LDS left one narrow workgroup per CU: 113 ms, now 14.4 here and 6.0 ms
+// in the narrow kernel; 256^3, 4 levels 1,094 -> 132 + 715 us.
+template <int RED, int TX, int TY, int TZ>
+__global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs D) {
+  using Acc = typename AccT<RED>::T;
+  using L = TileLds<TX, TY, TZ>;
+  constexpr int BX = TX, BY = TY < 8 ? TY : 8, BZ = TZ < 8 ? TZ : 8, B = BX * BY * BZ;
+  constexpr int nthr = kWideThreads;
+  static_assert(BX % 4 == 0 && BY % 4 == 0 && BZ % 4 == 0 && B / 4 <= nthr, "four outputs per thread and pass");
+  __shared__ long long hist[kWideCells];
+  __shared__ long long acc[B];   // int64 sums (deterministic) or FP64 bits (atomic)
+  __shared__ double s_k[kWideK];
+  __shared__ unsigned s_item;
+  __shared__ unsigned s_ccnt[kNLevels + 1];
+  double* hd = reinterpret_cast<double*>(hist);
+  const int tid = threadIdx.x;
+  const double dscale = fixed_scale(D.C->mmax_bits);
+  const float scale = (float)dscale;
+  const double inv_scale = 1.0 / dscale;   // a power of two: exact
+  const unsigned n_narrow = D.C->n_items_eff, n_wide = D.C->n_wide_eff;
+  // a cell's FP64 sum into the block's accumulator (one thread per cell)
+  auto put = [&](int c, double v) {
+    if (RED == 0) acc[c] += __double2ll_rn(v);
+    else reinterpret_cast<double*>(acc)[c] += v * inv_scale;
+  };
+  const int q = blockIdx.x % D.n_queues;
+  for (;;) {
+    if (tid == 0) s_item = atomicAdd(&D.C->wqueue[q * kLine], 1u) * D.n_queues + q;
+    if (tid <= kNLevels) s_ccnt[tid] = 0u;
+    __syncthreads();
+    const unsigned idx = __builtin_amdgcn_readfirstlane(s_item);
+    if (idx >= n_wide) break;
+    const Item it = D.items[n_narrow + idx];
+    const int t = __builtin_amdgcn_readfirstlane(it.tile);
+    const int g = __builtin_amdgcn_readfirstlane(P.tile_grid[t]);
+    const GridDesc& G = P.grids[g];
+    const int local = t - G.tile0;
+    const int i0 = (local % G.nt[0]) * TX + 1, j0t = ((local / G.nt[0]) % G.nt[1]) * TY + 1,
+              k0t = (local / (G.nt[0] * G.nt[1])) * TZ + 1;
+    // entries per class (wave ballots, one LDS add per wave and class)
+    {
+      unsigned cnt[kNLevels + 1] = {};
+      for (long long b0 = it.begin; b0 < it.end; b0 += nthr) {
+        const long long e = b0 + tid;
+        const int irk_e = e < it.end ? (D.entries[e].y >> 16) : 0;
+#pragma unroll
+        for (int k = 1; k <= kNLevels; ++k) cnt[k] += (unsigned)__popcll(__ballot(irk_e == k));
+      }
+      if ((tid & 63) == 0)
+        for (int k = 1; k <= kNLevels; ++k)
+          if (cnt[k]) atomicAdd(&s_ccnt[k], cnt[k]);
+    }
+    Acc* dst = reinterpret_cast<Acc*>(D.scratch) + (long long)t * L::E;
+    const bool alone = D.nitems_tile[t] == 1;
+    for (int sub = 0; sub < (TY / BY) * (TZ / BZ); ++sub) {
+      const int oy = (sub % (TY / BY)) * BY, oz = (sub / (TY / BY)) * BZ;
+      const int j0 = j0t + oy, k0 = k0t + oz;   // the block's first cell
+      if (j0 > G.n[1] || k0 > G.n[2]) continue;  // past the grid: never read
+      for (int c = tid; c < B; c += nthr) acc[c] = 0;   // zero bits: 0 as FP64 too
+      __syncthreads();
+      for (int irk = 1; irk <= kNLevels; ++irk) {
+        const unsigned ncls = s_ccnt[irk];
+        if (ncls == 0u) continue;
+        const int nk = 1 << irk;
+        const float* K = P.ktab + irk * P.kw + P.kmax;   // K[d], d in [-N, N]
+        const WideShape w = wide_shape<BX, BY, BZ>(nk);
+        const long long taps = 2 * nk + 1;
+        const long long box = (long long)min((int)taps, BX) * min((int)taps, BY) * min((int)taps, BZ);
+        const long long adds = w.form == 0 ? 1 : (w.form == 1 ? BZ : BY * BZ);
+        const long long passes = taps * ((long long)BX * w.ny * w.nz + (w.form < 2 ? (long long)BX * BY * w.nz : 0) +
+                                         (w.form < 1 ? B : 0));
+        if ((it.flags & 2) && w.form >= 0 && 4 * (long long)ncls * (box - adds) > passes) {
+          // ---- the histogram
+          if (tid < taps) s_k[tid] = (double)K[tid - nk];
+          for (int c = tid; c < w.cells; c += nthr) hist[c] = 0;
+          __syncthreads();
+          const double* Kd = s_k + nk;
+          int4 nxt = it.begin + tid < it.end ? D.entries[it.begin + tid] : make_int4(0, 0, 0, 0);
+          for (long long e = it.begin + tid; e < it.end; e += nthr) {
+            const int4 cur = nxt;
+            if (e + nthr < it.end) nxt = D.entries[e + nthr];
+            int ci[3], irk_e;
+            float m;
+            unpack_table(cur, ci[0], ci[1], ci[2], irk_e, m);
+            if (irk_e != irk) continue;
+            const int cx = ci[0] - i0, cy = ci[1] - j0, cz = ci[2] - k0;
+            if (cx < -nk || cx >= BX + nk || cy < -nk || cy >= BY + nk || cz < -nk || cz >= BZ + nk) continue;
+            const double ms = (double)(m * scale);
+            if (w.form == 0) {
+              lds_add(hist + (cx + nk) + w.px * (cy + nk) + w.pz * (cz + nk), __double2ll_rn(ms));
+              continue;
+            }
+            const int z0 = max(0, cz - nk), z1 = min(BZ - 1, cz + nk);
+            const int y0 = max(0, cy - nk), y1 = min(BY - 1, cy + nk);
+            for (int z = z0; z <= z1; ++z) {
+              const double mz = ms * Kd[z - cz];
+              if (w.form == 1) {
+                lds_add(hist + (cx + nk) + w.px * (cy + nk) + w.pz * z, __double2ll_rn(mz));
+                continue;
+              }
+              for (int y = y0; y <= y1; ++y)
+                lds_add(hist + (cx + nk) + w.px * y + w.pz * z, __double2ll_rn(mz * Kd[y - cy]));
+            }
+          }
+          __syncthreads();
+          for (int c = tid; c < w.cells; c += nthr) hd[c] = (double)hist[c];
+          __syncthreads();
+          // ---- x: lanes on consecutive rows (odd pitch), four outputs each
+          const int rows = w.ny * w.nz, ux = rows * (BX / 4);
+          double s[2][4];
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const int u = tid + r * nthr;
+            if (u < ux) conv4(hd + w.px * (u % rows) + 4 * (u / rows), 1, nk, s_k, s[r]);
+          }
+          if (w.form == 2) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+              const int u = tid + r * nthr;
+              if (u < ux)
+                for (int i = 0; i < 4; ++i) put(4 * (u / rows) + i + BX * (u % rows), s[r][i]);
+            }
+            __syncthreads();
+            continue;
+          }
+          const int pz = BX * w.ny + 16;   // plane pitch of the x pass's output
+          __syncthreads();
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const int u = tid + r * nthr;
+            if (u < ux) {
+              const int row = u % rows;
+              double* o = hd + 4 * (u / rows) + BX * (row % w.ny) + pz * (row / w.ny);
+              for (int i = 0; i < 4; ++i) o[i] = s[r][i];
+            }
+          }
+          __syncthreads();
+          // ---- y: lanes along x, then z
+          const int uy = BX * w.nz * (BY / 4);
+          const int ax = tid % BX, az = (tid / BX) % w.nz, ay = 4 * (tid / (BX * w.nz));
+          if (tid < uy) conv4(hd + ax + pz * az + BX * ay, BX, nk, s_k, s[0]);
+          if (w.form == 1) {
+            if (tid < uy)
+              for (int i = 0; i < 4; ++i) put(ax + BX * (ay + i + BY * az), s[0][i]);
+            __syncthreads();
+            continue;
+          }
+          __syncthreads();
+          if (tid < uy)
+            for (int i = 0; i < 4; ++i) hd[ax + BX * (ay + i + BY * az)] = s[0][i];
+          __syncthreads();
+          // ---- z: lanes along x and y
+          if (tid < B / 4) {
+            const int xy = tid % (BX * BY), zo = 4 * (tid / (BX * BY));
+            conv4(hd + xy + BX * BY * zo, BX * BY, nk, s_k, s[0]);
+            for (int i = 0; i < 4; ++i) put(xy + BX * BY * (zo + i), s[0][i]);
+          }
+          __syncthreads();
+          continue;
+        }
+        // ---- direct: one wave per entry.  The entry's box clipped to the
+        // block (bx x by x bz cells) is walked as one flat range, lane l taking
+        // cells l, l + 64, ...; its (x, y, z) counters advance by constant
+        // steps, so the loop has no divisions.  The next entry is loaded while
+        // this one deposits.  Terms are ((m*Kx)*Ky)*Kz as in the reference's
+        // loop.
+        const int ex = min(BX, G.n[0] - i0 + 1), ey = min(BY, G.n[1] - j0 + 1), ez = min(BZ, G.n[2] - k0 + 1);
+        const int wave = tid >> 6, lane = tid & 63, nwaves = nthr >> 6;
+        long long e = it.begin + wave;
+        int4 nxt = e < it.end ? D.entries[e] : make_int4(0, 0, 0, 0);
+        for (; e < it.end; e += nwaves) {
+          int ci[3], irk_e;
+          float m;
+          unpack_table(nxt, ci[0], ci[1], ci[2], irk_e, m);
+          if (e + nwaves < it.end) nxt = D.entries[e + nwaves];
+          if (irk_e != irk) continue;
+          const int xa = max(ci[0] - nk, i0), xb = min(ci[0] + nk, i0 + ex - 1);
+          const int ya = max(ci[1] - nk, j0), yb = min(ci[1] + nk, j0 + ey - 1);
+          const int za = max(ci[2] - nk, k0), zb = min(ci[2] + nk, k0 + ez - 1);
+          if (xb < xa || yb < ya || zb < za) continue;
+          const int cx = xb - xa + 1, cy = yb - ya + 1, total = cx * cy * (zb - za + 1);
+          // q / n for q <= 64 * 16 and n <= 16: (q + 1/2) / n is at least 1/32
+          // away from an integer, far beyond the FP32 error of the product
+          const float rbx = 1.0f / (float)cx, rby = 1.0f / (float)cy;
+          auto divn = [](int v, float rn) { return (int)(((float)v + 0.5f) * rn); };
+          const int r0 = divn(lane, rbx);
+          int a = lane - r0 * cx;
+          int c = divn(r0, rby);
+          int b = r0 - c * cy;
+          const int dr = divn(64, rbx), da = 64 - dr * cx;
+          const int dc0 = divn(dr, rby), db0 = dr - dc0 * cy;
+          const int dc1 = divn(dr + 1, rby), db1 = dr + 1 - dc1 * cy;
+          const float ms = RED == 0 ? m * scale : m;
+          const float* Kx = K + (xa - ci[0]);
+          const float* Ky = K + (ya - ci[1]);
+          const float* Kz = K + (za - ci[2]);
+          long long* base = acc + (xa - i0) + BX * ((ya - j0) + BY * (za - k0));
+          for (int q2 = lane; q2 < total; q2 += 64) {
+            const float term = ((ms * Kx[a]) * Ky[b]) * Kz[c];
+            long long* cell = base + (a + BX * (b + BY * c));
+            if (RED == 0) lds_add(cell, (long long)__float2int_rn(term));
+            else atomicAdd(reinterpret_cast<double*>(cell), (double)term);
+            a += da;
+            const bool carry = a >= cx;
+            if (carry) a -= cx;
+            b += carry ? db1 : db0;
+            c += carry ? dc1 : dc0;
+            if (b >= cy) {
+              b -= cy;
+              ++c;
+            }
+          }
+        }
+        __syncthreads();
+      }
+      // the block's cells to the tile's exchange cells, as the deposit's
+      for (int c = tid; c < B; c += nthr) {
+        Acc* cell = dst + (c % BX + 1) + L::EX * (((c / BX) % BY + oy + 1) + L::EY * (c / (BX * BY) + oz + 1));
+        const Acc v = RED == 0 ? (Acc)acc[c] : (Acc)reinterpret_cast<double*>(acc)[c];
+        if (alone) *cell = v;
+        else if (v != 0) glb_add(cell, v);
+      }
+      __syncthreads();
+    }
+    // wide boxes are clipped to their tile: nothing in the halo
+    if (alone)
+      for (int c = tid; c < L::E; c += nthr) {
+        const int x = c % L::EX, y = (c / L::EX) % L::EY, z = c / (L::EX * L::EY);
+        if (x == 0 || x == L::EX - 1 || y == 0 || y == L::EY - 1 || z == 0 || z == L::EZ - 1) dst[c] = 0;
+      }
+    __syncthreads();   // the item's class counts are read above
   }
 }
 
@@ -1647,8 +1773,8 @@ hipError_t launch_reduce_blocks(const BlockTables& BT, long long nblk, Counters*
 }
 
 hipError_t launch_plan_count(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                             unsigned* nitems_tile, hipStream_t s) {
-  plan_count<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, nitems_tile);
+                             unsigned* cnt, unsigned* nitems_tile, hipStream_t s) {
+  plan_count<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, cnt, nitems_tile);
   return hipGetLastError();
 }
 
@@ -1658,56 +1784,40 @@ hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int ch
   return hipGetLastError();
 }
 
-hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* tot_items,
+hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* item_off, int ntiles,
                        unsigned long long cap_entries, unsigned long long cap_items, Counters* C, hipStream_t s) {
-  gate_kernel<<<1, 64, 0, s>>>(tot_entries, tot_items, cap_entries, cap_items, C);
-  return hipGetLastError();
-}
-
-// Table mode: the histogram buffer of the wide classes takes the LDS left
-// beside the kernel's static arrays, sized for the largest class of the
-// geometry whose extended box fits there (smaller classes use a part of it).
-template <int MODE, int RED, int TX, int TY, int TZ>
-static hipError_t dep(const Plan& P, const DepArgs& D, int grid, int block, hipStream_t s) {
-  DepArgs d2 = D;
-  d2.hist_cells = 0;
-  size_t dyn = 0;
-  if (MODE == 1) {
-    static long long avail = -1;   // int64 cells of LDS beside the static arrays (per instantiation)
-    if (avail < 0) {
-      int dev = 0, maxl = 0;
-      hipFuncAttributes fa;
-      hipError_t e = hipGetDevice(&dev);
-      if (e == hipSuccess) e = hipDeviceGetAttribute(&maxl, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-      if (e == hipSuccess)
-        e = hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&deposit_kernel<MODE, RED, TX, TY, TZ>));
-      if (e != hipSuccess) return e;
-      avail = std::max<long long>(((long long)maxl - (long long)fa.sharedSizeBytes - 256) / 8, 0);
-      if (avail > 0) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&deposit_kernel<MODE, RED, TX, TY, TZ>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)(avail * 8));
-        if (e != hipSuccess) return e;
-      }
-    }
-    for (int irk = 1; irk <= P.nl; ++irk) {
-      const long long nk = 1ll << irk;
-      const long long nb = (TX + 2 * nk) * (TY + 2 * nk) * (TZ + 2 * nk);
-      if (nb <= avail) d2.hist_cells = (int)nb;
-    }
-    dyn = sizeof(long long) * (size_t)d2.hist_cells;
-  }
-  deposit_kernel<MODE, RED, TX, TY, TZ><<<grid, block, dyn, s>>>(P, d2);
+  gate_kernel<<<1, 64, 0, s>>>(tot_entries, item_off, ntiles, cap_entries, cap_items, C);
   return hipGetLastError();
 }
 
 template <int MODE, int RED>
 static hipError_t dep_shape(const Plan& P, const DepArgs& D, int grid, int block, hipStream_t s) {
   const int* t = P.tile;
-  if (t[0] == 8 && t[1] == 8 && t[2] == 8) return dep<MODE, RED, 8, 8, 8>(P, D, grid, block, s);
-  if (t[0] == 16 && t[1] == 8 && t[2] == 8) return dep<MODE, RED, 16, 8, 8>(P, D, grid, block, s);
-  if (t[0] == 16 && t[1] == 16 && t[2] == 8) return dep<MODE, RED, 16, 16, 8>(P, D, grid, block, s);
-  if (t[0] == 16 && t[1] == 16 && t[2] == 16) return dep<MODE, RED, 16, 16, 16>(P, D, grid, block, s);
-  return hipErrorInvalidValue;
+  if (t[0] == 8 && t[1] == 8 && t[2] == 8) deposit_kernel<MODE, RED, 8, 8, 8><<<grid, block, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 8 && t[2] == 8) deposit_kernel<MODE, RED, 16, 8, 8><<<grid, block, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 8) deposit_kernel<MODE, RED, 16, 16, 8><<<grid, block, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 16) deposit_kernel<MODE, RED, 16, 16, 16><<<grid, block, 0, s>>>(P, D);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+template <int RED>
+static hipError_t wide_shape_launch(const Plan& P, const DepArgs& D, int grid, hipStream_t s) {
+  const int* t = P.tile;
+  if (t[0] == 8 && t[1] == 8 && t[2] == 8) deposit_wide<RED, 8, 8, 8><<<grid, kWideThreads, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 8 && t[2] == 8) deposit_wide<RED, 16, 8, 8><<<grid, kWideThreads, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 8) deposit_wide<RED, 16, 16, 8><<<grid, kWideThreads, 0, s>>>(P, D);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 16) deposit_wide<RED, 16, 16, 16><<<grid, kWideThreads, 0, s>>>(P, D);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+// the wide table-mode items: two workgroups per CU fit (LDS)
+hipError_t launch_deposit_wide(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s) {
+  DepArgs d2 = D;
+  const int grid = std::max(cus, 1) * 2;
+  d2.n_queues = std::min(kQueues, grid);
+  return reduction == 0 ? wide_shape_launch<0>(P, d2, grid, s) : wide_shape_launch<1>(P, d2, grid, s);
 }
 
 bool tile_shape_supported(const int t[3]) {

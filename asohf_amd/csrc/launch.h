@@ -25,13 +25,14 @@ hipError_t launch_scan(const unsigned* in, long long n, unsigned long long* bsum
                        unsigned long long* cursor, hipStream_t s);
 hipError_t launch_reduce_blocks(const BlockTables& BT, long long nblk, Counters* C, int cus, hipStream_t s);
 hipError_t launch_plan_count(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                             unsigned* nitems_tile, hipStream_t s);
+                             unsigned* cnt, unsigned* nitems_tile, hipStream_t s);
 hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
                              const unsigned long long* item_off, Item* items, const Counters* C, hipStream_t s);
-hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* tot_items,
+hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* item_off, int ntiles,
                        unsigned long long cap_entries, unsigned long long cap_items, Counters* C, hipStream_t s);
 bool tile_shape_supported(const int t[3]);
 hipError_t launch_deposit(const Plan& P, const DepArgs& D, int reduction, int grid, int block, hipStream_t s);
+hipError_t launch_deposit_wide(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s);
 hipError_t launch_zero_split(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s);
 // the output cells and tile masses from the tiles' exchange cells (exchange_cells
 // accumulators per tile)
