@@ -132,6 +132,7 @@ struct HostPlan {
   std::vector<BoxRec> grec;
   std::vector<int> level_tile0;   // first tile of every level, [nl + 2]
   unsigned emit_levels = 0;       // bit l: some tile of level l has targets
+  bool table_base = false;        // table mode: no base tile has more than kTableTargets targets
   Plan dev{};
   long long ncells = 0;
   long long u11_cells = 0;   // cells of the patch output array
@@ -160,10 +161,11 @@ struct PipeArgs {
   unsigned long long cap_entries;   // entries and items the buffers hold
   unsigned long long cap_items;
   int ntiles, chunk, chunk_wide, red, grid, block, cus, elem;
-  // TSC binning along the hierarchy
+  // binning through the base grid
   unsigned* item_pairs;
+  TableBin TB;
   long long lvl_items[kNLevels + 2];   // items of level l: [lvl_items[l], lvl_items[l + 1])
-  long long n_items;
+  long long n_items, n_narrow;
   unsigned emit_levels;
   int nl;
 };
@@ -179,6 +181,7 @@ struct asohf_ctx {
   DBuf cnt, start, cursor, bsum, counters, nitems, icnt, tmass, entries, items, scratch;
   DBuf flags, idx, pool, pool_off, pool_nk, blk_pairs, blk_mmax, item_off;
   DBuf elist, eoff, ecount;
+  DBuf spc, outside, units;                // table mode: species of the base entries, particles outside the box, work units
   DBuf ipairs;                             // members found per work item (TSC hierarchy binning)
   void* noalloc = nullptr;                 // this device's scratch array of order.hip (device address)
   DBuf sp_k[4], sp_dens, sp_cnt, sp_tmp;   // species partition
@@ -195,6 +198,7 @@ struct asohf_ctx {
   uint64_t hier_key = 0;
   long long hier_items[kNLevels + 2] = {};
   long long hier_nitems = 0;
+  long long hier_nnarrow = 0;
   hipGraphExec_t gexec = nullptr;   // the captured batched build and the arguments it holds
   PipeArgs gkey;
   DBuf h_in[4], h_out[2], h_mass;    // device copies for the host entry point
@@ -209,6 +213,12 @@ struct asohf_ctx {
   bool stats_phases = false;
   std::map<std::pair<int, int>, std::vector<float>> ktab_cache;
 };
+
+// base-tile targets up to which table mode bins through the base grid
+constexpr unsigned kTableTargets = 1024;
+// particles outside the box that table mode's binning lists; a call with more
+// takes the count and scatter passes
+constexpr long long kOutsideMax = 1ll << 20;
 
 // particles from which the adjoint gathers in base-cell order
 constexpr long long kAdjointSortMin = 1ll << 20;
@@ -557,14 +567,15 @@ static asohf_status build_plan(asohf_ctx* ctx, const asohf_geom* g, int mode, co
   for (int l = nl; l >= 1; --l)
     H.level_tile0[l] = g->npatch[l] > 0 ? H.grids[1 + level_start[l]].tile0 : H.level_tile0[l + 1];
   H.level_tile0[0] = 0;
-  // ---- TSC binning along the hierarchy: every level-l patch (l >= 1) gets an
-  // emitter, the deepest grid found whose membership box holds the patch's box
-  // in FP32 (so every member of the patch is a member of the emitter): a
-  // patch of the level above whose box holds it, else one two levels up, ...,
-  // else the base grid, which holds every particle.  The patch is then a
-  // target of every emitter tile whose home region (the positions whose
-  // clamped cell lies in the tile) can meet its box. ----
-  if (mode == ASOHF_MODE_TSC) {
+  // ---- binning through the base grid.  TSC: every level-l patch (l >= 1)
+  // gets an emitter, the deepest grid found whose membership box holds the
+  // patch's box in FP32 (so every member of the patch is a member of the
+  // emitter): a patch of the level above whose box holds it, else one two
+  // levels up, ..., else the base grid, which holds every particle.  Table
+  // mode: the base grid is every patch's emitter.  The patch is then a target
+  // of every emitter tile whose home region (the positions whose clamped cell
+  // lies in the tile) can meet its box. ----
+  {
     H.grec.resize(H.grids.size());
     for (size_t gi = 0; gi < H.grids.size(); ++gi) H.grec[gi] = make_rec((int)gi);
     auto contains = [&](const GridDesc& Q, const GridDesc& Cg) {
@@ -596,7 +607,7 @@ static asohf_status build_plan(asohf_ctx* ctx, const asohf_geom* g, int mode, co
         const int gc = 1 + p;
         const GridDesc& Cg = H.grids[gc];
         int ge = 0;
-        for (int lq = l - 1; lq >= 1 && ge == 0; --lq) {
+        for (int lq = l - 1; mode == ASOHF_MODE_TSC && lq >= 1 && ge == 0; --lq) {
           const int f = find_container(lq, Cg);
           if (f > 0) ge = f;
         }
@@ -628,10 +639,12 @@ static asohf_status build_plan(asohf_ctx* ctx, const asohf_geom* g, int mode, co
       std::vector<unsigned> fill(H.tgt_off.begin(), H.tgt_off.end() - 1);
       for (const auto& e : tp) H.tgt[fill[e.first]++] = e.second;
     }
-  } else {
-    H.tgt_off.assign(ntiles + 1, 0u);
-    H.tgt.assign(1, 0);
-    H.grec.assign(1, BoxRec{});
+    // Table mode tests every base entry against its tile's whole list, about
+    // a dozen instructions per 64 entries and target: at 54 targets (512^3, 6
+    // levels, mean over the particles) a tenth of what the count and scatter
+    // passes took; past a thousand it would cost more than they do.
+    H.table_base = mode == ASOHF_MODE_TABLE;
+    for (int t = 0; t < ntiles && H.table_base; ++t) H.table_base = H.tgt_off[t + 1] - H.tgt_off[t] <= kTableTargets;
   }
   // ---- upload ----
   size_t off = 0;
@@ -960,7 +973,7 @@ static asohf_status run_exact(asohf_ctx* ctx, const asohf_opts& o, const Parts& 
 }
 
 // ---------------------------------------------------------------------------
-// TSC: binning along the hierarchy (hier.hip)
+// binning through the base grid (hier.hip)
 // ---------------------------------------------------------------------------
 static uint64_t hier_key(const asohf_ctx* ctx, const Parts& A, int red) {
   uint64_t h = ctx->plan.key;
@@ -979,13 +992,18 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   HIPCHK(launch_count(a.P, a.A, a.cnt, a.C, a.BT, a.cus, s), "count kernel");
   HIPCHK(launch_count_to_capacity(a.cnt, a.nkeys, a.cus, s), "capacities");
   HIPCHK(launch_scan(a.cnt, a.nkeys, a.bsum, a.start, a.cursor, s), "scan");
-  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, 0, a.icnt, a.nitems, s),
+  HIPCHK(launch_plan_count(a.start, a.ntiles, a.chunk, a.P.mode == 2 ? 0 : a.chunk_wide, a.icnt, a.nitems, s),
          "planning items");
   HIPCHK(launch_scan(a.icnt, 2ll * a.ntiles, a.bsum, a.item_off, nullptr, s), "item offsets");
   const int nl = a.P.nl;
   HIPCHK(hipMemcpyAsync(ctx->hcount, a.C, sizeof(Counters), hipMemcpyDeviceToHost, s), "reading counters");
   HIPCHK(hipMemcpyAsync(ctx->hscalar, a.start + a.nkeys, sizeof(unsigned long long), hipMemcpyDeviceToHost, s),
          "reading totals");
+  // entries of the base grid, whose species table mode keeps
+  HIPCHK(hipMemcpyAsync(ctx->hscalar + nl + 3, a.start + 2ll * H.level_tile0[1 <= nl ? 1 : nl + 1], sizeof(unsigned long long),
+                        hipMemcpyDeviceToHost, s), "reading totals");
+  HIPCHK(hipMemcpyAsync(ctx->hscalar + nl + 4, a.item_off + 2ll * a.ntiles, sizeof(unsigned long long),
+                        hipMemcpyDeviceToHost, s), "reading totals");
   for (int l = 0; l <= nl + 1; ++l)
     HIPCHK(hipMemcpyAsync(ctx->hscalar + 1 + l, a.item_off + H.level_tile0[l], sizeof(unsigned long long),
                           hipMemcpyDeviceToHost, s), "reading item offsets");
@@ -993,18 +1011,27 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   asohf_status st = decode_err(ctx, ctx->hcount->err);
   if (st != ASOHF_OK) return st;
   const unsigned long long cap_entries = ctx->hscalar[0];
-  const long long n_items = (long long)ctx->hscalar[1 + nl + 1];
+  const long long n_items = (long long)ctx->hscalar[nl + 4];
   if (n_items >= (1ll << 31)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^31 work items");
   if (cap_entries >= (1ull << 40)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^40 tile entries");
   for (int l = 0; l <= nl + 1; ++l) ctx->hier_items[l] = (long long)ctx->hscalar[1 + l];
   HIPCHK(ctx->entries.ensure(sizeof(int4) * std::max<unsigned long long>(cap_entries, 1)), "allocating entries");
   HIPCHK(ctx->items.ensure(sizeof(Item) * std::max<long long>(n_items, 1)), "allocating work items");
   HIPCHK(ctx->ipairs.ensure(sizeof(unsigned) * std::max<long long>(n_items, 1)), "allocating item sums");
+  if (a.P.mode == 1) {
+    HIPCHK(ctx->spc.ensure(std::max<unsigned long long>(ctx->hscalar[nl + 3], 1)), "allocating species");
+    HIPCHK(ctx->outside.ensure(sizeof(unsigned) * std::max<long long>(std::min(a.A.n, kOutsideMax), 1)),
+           "allocating the outside list");
+    const long long units = ctx->hier_items[1] * emit_pieces(a.chunk);
+    if (units >= (1ll << 32)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^32 emission work units");
+    HIPCHK(ctx->units.ensure(sizeof(unsigned long long) * std::max<long long>(units, 1)), "allocating work units");
+  }
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
-  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, 0, a.item_off, const_cast<Item*>(a.D.items), a.C, s),
+  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.P.mode == 2 ? 0 : a.chunk_wide, a.item_off, const_cast<Item*>(a.D.items), a.C, s),
          "writing items");
   ctx->hier_nitems = n_items;
+  ctx->hier_nnarrow = ctx->hier_items[nl + 1];
   return ASOHF_OK;
 }
 
@@ -1015,6 +1042,13 @@ static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
   a.D.cursor = a.cursor;
   a.item_pairs = ctx->ipairs.as<unsigned>();
   a.n_items = ctx->hier_nitems;
+  a.n_narrow = ctx->hier_nnarrow;
+  if (a.P.mode == 1) {
+    a.TB.species = ctx->spc.as<unsigned char>();
+    a.TB.outside = ctx->outside.as<unsigned>();
+    a.TB.units = ctx->units.as<unsigned long long>();
+    a.TB.outside_cap = (unsigned)std::min(a.A.n, kOutsideMax);
+  }
   for (int l = 0; l <= kNLevels + 1; ++l) a.lvl_items[l] = ctx->hier_items[std::min(l, a.P.nl + 1)];
   a.emit_levels = ctx->plan.emit_levels;
   a.nl = a.P.nl;
@@ -1027,17 +1061,23 @@ static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
 // grid sums and the call's statistics; no host round trip (graph-capturable).
 static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t s, bool events) {
   HIPCHK(launch_fill_u32((unsigned*)a.C, 0u, sizeof(Counters) / 4, s), "clearing counters");
-  HIPCHK(launch_fill_u32(&a.C->n_items_eff, (unsigned)a.n_items, 1, s), "queue length");
+  HIPCHK(launch_fill_u32(&a.C->n_items_eff, (unsigned)a.n_narrow, 1, s), "queue length");
+  if (a.n_items > a.n_narrow)
+    HIPCHK(launch_fill_u32(&a.C->n_wide_eff, (unsigned)(a.n_items - a.n_narrow), 1, s), "queue length");
   HIPCHK(launch_fill_u32(a.item_pairs, 0u, a.n_items, s), "clearing item sums");
   HIPCHK(launch_cursor_reset(a.start, a.cursor, a.nkeys, a.cus, s), "cursors");
-  HIPCHK(launch_bin_base_tsc(a.P, a.A, a.cursor, a.start, const_cast<int4*>(a.D.entries), a.C, a.BT, a.cus, s),
+  HIPCHK(launch_bin_base(a.P, a.A, a.cursor, a.start, const_cast<int4*>(a.D.entries), a.C, a.BT, a.TB, a.cus, s),
          "base-grid binning");
   if (a.A.n > 0) HIPCHK(launch_reduce_blocks(a.BT, hier_bin_blocks(a.A.n), a.C, a.cus, s), "block sums");
   if (events) {
     HIPCHK(hipEventRecord(ctx->ev[1], s), "event");
     HIPCHK(hipEventRecord(ctx->ev[2], s), "event");
   }
-  for (int l = 0; l < a.nl; ++l) {
+  if (a.P.mode == 1 && a.nl > 0)
+    HIPCHK(launch_emit_table(a.P, a.A, a.D.items, a.lvl_items[1], a.chunk, a.cursor, a.start, const_cast<int4*>(a.D.entries),
+                             a.item_pairs, a.C, a.TB, a.cus, s),
+           "emission pass");
+  for (int l = 0; a.P.mode == 2 && l < a.nl; ++l) {
     if (!(a.emit_levels & (1u << l))) continue;
     HIPCHK(launch_emit_tsc(a.P, a.D.items, a.lvl_items[l], a.lvl_items[l + 1], l, a.cursor, a.start,
                            const_cast<int4*>(a.D.entries), a.item_pairs, a.C, a.cus, s),
@@ -1047,6 +1087,7 @@ static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t 
   HIPCHK(launch_zero_split(a.P, a.D, a.red, a.cus, s), "clearing split tiles");
   if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
   HIPCHK(launch_deposit(a.P, a.D, a.red, a.grid, a.block, s), "deposit kernel");
+  if (a.n_items > a.n_narrow) HIPCHK(launch_deposit_wide(a.P, a.D, a.red, a.cus, s), "wide deposit kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[8], s), "event");
   HIPCHK(launch_combine(a.P, a.D, a.red, a.cus, s), "output cells");
   if (events) HIPCHK(hipEventRecord(ctx->ev[5], s), "event");
@@ -1055,8 +1096,10 @@ static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t 
   return ASOHF_OK;
 }
 
+// *many_outside: table mode met more particles outside the box than its list
+// holds and wrote nothing
 static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A, float* u1, float* u11,
-                             double* grid_mass, hipStream_t s) {
+                             double* grid_mass, hipStream_t s, bool* many_outside) {
   for (int attempt = 0; attempt < 2; ++attempt) {
     PipeArgs a;
     // the count pass keeps no emission lists here
@@ -1119,6 +1162,10 @@ static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A
     if (hc.overflow) {
       // a tile received more entries than its capacity: plan them again
       ctx->hier_sized = false;
+      if (a.P.mode == 1 && hc.n_outside > a.TB.outside_cap) {
+        *many_outside = true;
+        return ASOHF_OK;
+      }
       continue;
     }
     hc.n_items = (unsigned long long)a.n_items;
@@ -1136,7 +1183,11 @@ static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A
 static asohf_status run_batched(asohf_ctx* ctx, const asohf_opts& o, const Parts& A, float* u1, float* u11,
                                 double* grid_mass, hipStream_t s) {
   if (A.n > (1ll << 32)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^32 particles");
-  if (o.mode == ASOHF_MODE_TSC && !ctx->hier_off) return run_hier(ctx, o, A, u1, u11, grid_mass, s);
+  if (!ctx->hier_off && (o.mode == ASOHF_MODE_TSC || ctx->plan.table_base)) {
+    bool many_outside = false;
+    const asohf_status st = run_hier(ctx, o, A, u1, u11, grid_mass, s, &many_outside);
+    if (st != ASOHF_OK || !many_outside) return st;
+  }
   ctx->hier_sized = false;   // this path re-plans the offsets and items the hierarchy binning keeps
   if (!ctx->sized) return run_exact(ctx, o, A, u1, u11, grid_mass, s);
   PipeArgs a;
@@ -1276,8 +1327,8 @@ asohf_status asohf_hip_create(asohf_ctx** out, int32_t device) {
   if (hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) { delete ctx; return ASOHF_ERR_HIP; }
   ctx->cus = prop.multiProcessorCount;
   {
-    // ASOHF_TSC_BINNING=hash: the TSC build bins with the patch-hash count
-    // and scatter passes (the kernel-table mode always does)
+    // ASOHF_TSC_BINNING=hash: the build bins with the patch-hash count and
+    // scatter passes
     const char* b = getenv("ASOHF_TSC_BINNING");
     ctx->hier_off = b && strcmp(b, "hash") == 0;
   }
@@ -1285,7 +1336,7 @@ asohf_status asohf_hip_create(asohf_ctx** out, int32_t device) {
   for (auto& e : ctx->ev)
     if (hipEventCreate(&e) != hipSuccess) { asohf_hip_destroy(ctx); return ASOHF_ERR_HIP; }
   if (hipHostMalloc((void**)&ctx->hcount, sizeof(Counters)) != hipSuccess ||
-      hipHostMalloc((void**)&ctx->hscalar, sizeof(unsigned long long) * 16) != hipSuccess) {
+      hipHostMalloc((void**)&ctx->hscalar, sizeof(unsigned long long) * 24) != hipSuccess) {
     asohf_hip_destroy(ctx);
     return ASOHF_ERR_OOM;
   }
@@ -1306,7 +1357,7 @@ void asohf_hip_destroy(asohf_ctx* ctx) {
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
                   &ctx->item_off, &ctx->plan_blob, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum, &ctx->counters,
-                  &ctx->nitems, &ctx->icnt, &ctx->tmass, &ctx->entries, &ctx->items,
+                  &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries, &ctx->items,
                   &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1], &ctx->h_in[2],
                   &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0], &ctx->ord[1],
                   &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount, &ctx->sp_k[0],
@@ -2261,7 +2312,7 @@ asohf_status asohf_hip_release_workspaces(asohf_ctx* ctx) {
   ctx->gexec = nullptr;
   DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
                   &ctx->item_off, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum,
-                  &ctx->nitems, &ctx->icnt, &ctx->tmass, &ctx->entries,
+                  &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries,
                   &ctx->items, &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1],
                   &ctx->h_in[2], &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0],
                   &ctx->ord[1], &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount,
@@ -2270,7 +2321,6 @@ asohf_status asohf_hip_release_workspaces(asohf_ctx* ctx) {
                   &ctx->pk_cnt, &ctx->pk_geo, &ctx->mk_geo, &ctx->mk_err, &ctx->vg_cnt, &ctx->vg_start,
                   &ctx->vg_pairs};
   for (DBuf* b : bufs) b->release();
-  ctx->ipairs.release();
   ctx->sized = false;   // the next batched call sizes its buffers again
   ctx->hier_sized = false;
   return ASOHF_OK;

@@ -1,15 +1,16 @@
-// hier.hip -- TSC binning along the patch hierarchy (gfx950).
+// hier.hip -- binning through the base grid and along the patch hierarchy
+// (gfx950).
 //
-// The batched TSC build bins each (particle, grid) member into the tile that
-// holds its centre cell (clamped into the grid); what its 27-cell stencil
-// spills over the tile's border is exchanged between tiles after the deposit.
+// The batched build bins each 27-cell (particle, grid) member into the tile
+// that holds its centre cell (clamped into the grid); what its stencil spills
+// over the tile's border is exchanged between tiles after the deposit.
 // Instead of testing every particle against a hash of every level's patch
-// boxes, the binning follows the hierarchy:
+// boxes, the binning starts from the base-grid tiles:
 //
-//   bin_base_tsc  particles -> base-grid tile entries (16 B: x, y, z, m);
+//   bin_base      particles -> base-grid tile entries (16 B: x, y, z, m);
 //                 every particle is a member of the base grid
-//                 (grids.f:1159-1246)
-//   emit_tsc      for one level at a time: the entries of a level-l tile are
+//                 (grids.f:761-835, 1159-1246)
+//   emit_tsc      TSC, one level at a time: the entries of a level-l tile are
 //                 tested against the patch boxes of the tile's target
 //                 list: the patches whose membership box lies inside this
 //                 grid's box (found on the host in FP32, the values the
@@ -18,6 +19,12 @@
 //                 A member gets its entry in that patch, exactly as the
 //                 reference's strict box test and index expressions give it
 //                 (grids.f:1294-1323).
+//   emit_table    kernel table: the base entries are tested against every
+//                 patch whose membership box can hold a particle of the tile
+//                 (grids.f:871-909); members whose box of 2N+1 cells meets the
+//                 patch get their entries there.  (The boxes reach a base cell
+//                 past the patch, so following the hierarchy would need
+//                 entries for five times as many members as deposit.)
 //
 // Entries go to per-tile ranges whose capacities come from an exact count
 // pass (the first call on a geometry, or after an overflow): every workgroup
@@ -26,6 +33,8 @@
 // reserves its own slot directly.  A reservation past a tile's capacity sets
 // the overflow flag (nothing is written past it) and the host rebuilds the
 // capacities exactly.
+#include <type_traits>
+
 #include "dev.h"
 #include "launch.h"
 
@@ -75,7 +84,8 @@ __device__ __forceinline__ int slot_insert(int* keys, int k) {
 
 __device__ __forceinline__ void set_overflow(Counters* C) {
   C->overflow = 1u;
-  C->n_items_eff = 0u;   // the deposit of this call then does nothing
+  C->n_items_eff = 0u;   // the deposits of this call then do nothing
+  C->n_wide_eff = 0u;
 }
 
 // one entry written at its own reserved slot (the path of an emission that
@@ -154,20 +164,23 @@ __device__ __forceinline__ long long reserved_slot(unsigned long long b, unsigne
 
 // Base-grid binning, persistent: each workgroup takes chunks of kHbChunk
 // particles (kHbPer per thread) in turn and loads its next chunk while it
-// bins this one.  Each valid particle (finite, mass >= 0, within the TSC
-// range of the base grid) has one entry, in the tile of its clamped cell.
-// Every lane counts its particles' keys in the workgroup's LDS table (a
-// position in the key's range of the workgroup), one global add per key
-// reserves the ranges, and every lane writes its particles from registers.
-// Per-chunk partials: base members and the largest mass.
+// bins this one.  Each valid particle (finite, mass >= 0, within the range the
+// mode accepts) has one entry, in the tile of its clamped (TSC) or wrapped
+// (table) cell.  Every lane counts its particles' keys in the workgroup's LDS
+// table (a position in the key's range of the workgroup), one global add per
+// key reserves the ranges, and every lane writes its particles from registers.
+// Table mode also writes each entry's species; a particle outside the box,
+// whose tile is a periodic image, gets kSpOutside and goes to the outside
+// list.  Per-chunk partials: base members and the largest mass.
 // Bound by latency (LDS counting, then one round of global reservations per
 // chunk).  One entry per particle instead of one per tile its stencil touches
 // needs no emission list, so twice the workgroups fit a CU and a third fewer
 // entries are written: 16.8M particles on 256^3 cells (16x8x8 tiles) 1,431 ->
 // 356 us, 134M particles 6.57 -> 2.11 ms.
-__global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsigned long long* cursor,
-                                                           const unsigned long long* start, int4* entries,
-                                                           Counters* C, BlockTables BT) {
+template <int MODE>
+__global__ void __launch_bounds__(kHbThreads) bin_base(Plan P, Parts A, unsigned long long* cursor,
+                                                       const unsigned long long* start, int4* entries,
+                                                       Counters* C, BlockTables BT, TableBin TB) {
   __shared__ int keys[kHbCap];
   __shared__ unsigned vals[kHbCap];
   __shared__ unsigned long long base[kHbCap];
@@ -196,6 +209,7 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
     float px[kHbPer], py[kHbPer], pz[kHbPer], pm[kHbPer];
     int slot[kHbPer];       // the key's table slot, -1: no entry to write
     unsigned at[kHbPer];    // the position in the key's range
+    int sp[kHbPer];         // table mode: the particle's species
 #pragma unroll
     for (int r = 0; r < kHbPer; ++r) { px[r] = fx[r]; py[r] = fy[r]; pz[r] = fz[r]; pm[r] = fm[r]; }
     fetch(chunk + gridDim.x);
@@ -204,6 +218,9 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
     unsigned err = 0;
     unsigned long long valid = 0;
     float mmax = 0.f;
+    // the particles are ordered by species: most chunks hold one
+    const int sp_lo = MODE == 1 ? species_of(A, c0) : 0;
+    const int sp_hi = MODE == 1 ? species_of(A, min(c0 + kHbChunk, A.n) - 1) : 0;
 #pragma unroll
     for (int r = 0; r < kHbPer; ++r) {
       const int k = r * kHbThreads + tid;
@@ -211,24 +228,55 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
       const float x = px[r], y = py[r], z = pz[r], m = pm[r];
       if (ok && !(isfinite(x) && isfinite(y) && isfinite(z) && isfinite(m))) { err |= kErrNonFinite; ok = false; }
       if (ok && m < 0.f) { err |= kErrNegMass; ok = false; }
-      if (ok && !(tsc_base_in_range(x, P.xl, bid[0], bn[0]) && tsc_base_in_range(y, P.xl, bid[1], bn[1]) &&
-                  tsc_base_in_range(z, P.xl, bid[2], bn[2]))) {
-        err |= kErrWrap;
-        ok = false;
-      }
       slot[r] = -1;
       at[r] = 0u;
+      sp[r] = 0;
+      int c[3];   // the cell whose tile takes the entry
+      if (MODE == 2) {
+        if (ok && !(tsc_base_in_range(x, P.xl, bid[0], bn[0]) && tsc_base_in_range(y, P.xl, bid[1], bn[1]) &&
+                    tsc_base_in_range(z, P.xl, bid[2], bn[2]))) {
+          err |= kErrWrap;
+          ok = false;
+        }
+        if (ok) {
+          c[0] = tsc_base_index(x, P.xl, bd[0], bid[0], bn[0]);
+          c[1] = tsc_base_index(y, P.xl, bd[1], bid[1], bn[1]);
+          c[2] = tsc_base_index(z, P.xl, bd[2], bid[2], bn[2]);
+        }
+      } else if (ok) {
+        const float t[3] = {index_quotient(x - P.xl, bd[0], bid[0]), index_quotient(y - P.xl, bd[1], bid[1]),
+                            index_quotient(z - P.xl, bd[2], bid[2])};
+        sp[r] = sp_lo == sp_hi ? sp_lo : species_of(A, c0 + k);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          ok = ok && t[a] > -1.0e9f && t[a] < 1.0e9f;
+          const int i = ok ? (int)t[a] + 1 : 1;
+          ok = ok && i >= 2 - bn[a] && i <= 2 * bn[a] - 1;   // the single wrap must land in 1..N
+          if (t[a] < 0.f || i > bn[a]) sp[r] = kSpOutside;
+          c[a] = wrap1(i, bn[a]);
+        }
+        if (!ok) err |= kErrWrap;
+        else if (sp[r] == kSpOutside) {
+          const unsigned o = atomicAdd(&C->n_outside, 1u);
+          if (o < TB.outside_cap) TB.outside[o] = (unsigned)(c0 + k);
+          else set_overflow(C);
+        }
+      }
       if (ok) {
         ++valid;
         mmax = fmaxf(mmax, m);
-        const int tx = (tsc_base_index(x, P.xl, bd[0], bid[0], bn[0]) - 1) >> P.tshift[0];
-        const int ty = (tsc_base_index(y, P.xl, bd[1], bid[1], bn[1]) - 1) >> P.tshift[1];
-        const int tz = (tsc_base_index(z, P.xl, bd[2], bid[2], bn[2]) - 1) >> P.tshift[2];
+        const int tx = (c[0] - 1) >> P.tshift[0], ty = (c[1] - 1) >> P.tshift[1], tz = (c[2] - 1) >> P.tshift[2];
         const int key = 2 * ((tz * bnt1 + ty) * bnt0 + tx);
         slot[r] = count_key<kHbCap>(keys, vals, key, at[r]);
-        if (slot[r] < 0)
-          emit_direct(cursor, start, entries, C, key,
-                      make_int4(__float_as_int(x), __float_as_int(y), __float_as_int(z), __float_as_int(m)));
+        if (slot[r] < 0) {
+          const unsigned long long p = atomicAdd(&cursor[key], 1ull);
+          if (p < start[key + 1]) {
+            entries[p] = make_int4(__float_as_int(x), __float_as_int(y), __float_as_int(z), __float_as_int(m));
+            if (MODE == 1) TB.species[p] = (unsigned char)sp[r];
+          } else {
+            set_overflow(C);
+          }
+        }
       }
     }
     __syncthreads();
@@ -238,9 +286,11 @@ __global__ void __launch_bounds__(kHbThreads) bin_base_tsc(Plan P, Parts A, unsi
     for (int r = 0; r < kHbPer; ++r) {
       if (slot[r] < 0) continue;
       const long long pos = reserved_slot(base[slot[r]], at[r]);
-      if (pos >= 0)
+      if (pos >= 0) {
         entries[pos] = make_int4(__float_as_int(px[r]), __float_as_int(py[r]), __float_as_int(pz[r]),
                                  __float_as_int(pm[r]));
+        if (MODE == 1) TB.species[pos] = (unsigned char)sp[r];
+      }
     }
     // per-workgroup partials (members of the base grid, largest mass)
     valid = wave_sum(valid);
@@ -420,6 +470,335 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
   }
 }
 
+// ---------------------------------------------------------------------------
+// kernel-table emission
+// ---------------------------------------------------------------------------
+constexpr int kEtThreads = 256;
+constexpr int kEtPiece = 1024;     // entries of a work unit (a collected member keeps 10 bits of it)
+constexpr int kEtTargets = 32;     // target records staged in LDS at once
+constexpr int kEtCap = 1024;       // LDS key slots
+constexpr int kEtWList = 128;      // emissions a wave lists before it works through them
+constexpr int kEtPend = 128;       // members a wave collects before it works through them
+constexpr unsigned long long kEtFull = ~0ull;   // a key's reservation past its capacity
+
+// A target patch in LDS: its strict membership box, its first cell's corner,
+// its sides, the largest cell side (with 1/64 of slack) and its ratio to the x
+// side for the tests; the cell and tile fields for the members.
+struct EtTarget {
+  float lo[3], hi[3], org[3], nd[3];
+  float dl, ratio;
+  int level, tile0;
+  float d[3], inv_d[3];
+  int n[3], nt0, nt1, pad[5];
+};
+static_assert(sizeof(EtTarget) == 128, "four 16-byte LDS reads for the tests");
+
+// slot of key k in the table, -1 when it is not there (slot_insert found its
+// probe path full)
+template <int CAP>
+__device__ __forceinline__ int slot_find(const int* keys, int k) {
+  unsigned h = slot_hash((unsigned)k, CAP - 1);
+#pragma unroll 1
+  for (int p = 0; p < kHbProbe; ++p) {
+    const int cur = keys[h];
+    if (cur == k) return (int)h;
+    if (cur == -1) return -1;
+    h = (h + 1) & (CAP - 1);
+  }
+  return -1;
+}
+
+// exclusive prefix over the wave's lanes of v >= 0, and the total
+__device__ __forceinline__ int wave_exclusive(int v, int& total) {
+  int s = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(s, o, 64);
+    if ((int)__lane_id() >= o) s += t;
+  }
+  total = __shfl(s, 63, 64);
+  return s - v;
+}
+
+// The call's emission work units: (item << 32 | piece) for every piece of
+// kEtPiece filled entries of the items of tiles with targets.
+__global__ void __launch_bounds__(256) list_units(Plan P, const Item* items, long long n_items,
+                                                  const unsigned long long* cursor, unsigned long long* units,
+                                                  Counters* C) {
+  const long long ii = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  int n = 0;
+  if (ii < n_items) {
+    const Item it = items[ii];
+    if (P.tgt_off[it.tile] < P.tgt_off[it.tile + 1]) {
+      const long long len = min(it.end, (long long)cursor[2 * it.tile]) - it.begin;
+      n = len > 0 ? (int)((len + kEtPiece - 1) / kEtPiece) : 0;
+    }
+  }
+  int tot;
+  const int off = wave_exclusive(n, tot);
+  unsigned b0 = 0;
+  if (__lane_id() == 0 && tot) b0 = atomicAdd(&C->n_units, (unsigned)tot);
+  b0 = __builtin_amdgcn_readfirstlane(b0);
+  for (int k = 0; k < n; ++k) units[b0 + off + k] = ((unsigned long long)ii << 32) | (unsigned)k;
+}
+
+// The kernel-table members of every patch from the base-grid entries.  A work
+// unit is kEtPiece entries of a base tile's work item; workgroups take units
+// from the list in turn, the next one's number on its way while this one is
+// worked through; up to kEtTargets target patches at a time are staged
+// in LDS and worked through in two passes over the unit's entries:
+//   count  every wave tests its 64 entries against each target (the
+//          reference's strict box, counted as members), keeps as a bit mask
+//          those whose 2N+1 cells can meet the patch (the distance to the patch
+//          against N cells) and adds up their emissions per tile key in the
+//          LDS table: one for the tile of the centre cell where N = 1, one per
+//          tile the clipped box touches otherwise
+//   write  after one global add per key reserved the unit's ranges, the same
+//          members again from the masks, every emission written at the next
+//          slot of its key's range
+// Both passes collect members over the wave's entries and work through 64 at a
+// time, one per lane (their entries read again), and spread the emissions of
+// wide members densely over the lanes.
+// Bound by VALU work (9.4 G instructions at 512^3: 54 targets per entry on
+// average, 4.1 members, 1.8 tiles each).  The count and scatter passes over
+// the patch hash this replaces, and what it takes with bin_base<1>: 512^3, 6
+// levels 70.1 -> 23.3 ms; 256^3, 4 levels 2,235 -> 1,206 us; 128^3, 3 levels
+// 175 -> 127 us.  One pass that listed the emissions for a reservation per
+// round of 256 entries took 35.6 ms, and 97 ms with lists short enough for six
+// workgroups per CU: what overflowed them reserved one by one.
+__global__ void __launch_bounds__(kEtThreads) emit_table(Plan P, const Item* items, const unsigned long long* units,
+                                                         unsigned long long* cursor, const unsigned long long* start,
+                                                         int4* entries, unsigned* item_pairs, Counters* C,
+                                                         TableBin TB) {
+  __shared__ int keys[kEtCap];
+  __shared__ unsigned long long slots[kEtCap];   // emissions of a key, then its next slot
+  __shared__ unsigned long long mask[kEtPiece / 64][kEtTargets];
+  __shared__ unsigned long long wlist_all[(kEtThreads / 64) * kEtWList];   // key | member's lane << 32
+  __shared__ unsigned pend_all[(kEtThreads / 64) * kEtPend];               // entry of the unit | target << 10
+  __shared__ EtTarget targets[kEtTargets];
+  __shared__ unsigned s_next;
+  const int tid = threadIdx.x, lane = (int)__lane_id();
+  unsigned long long* wl = wlist_all + (tid >> 6) * kEtWList;
+  unsigned* pd = pend_all + (tid >> 6) * kEtPend;
+  const float dx = P.grids[0].d[0];
+  const unsigned n_units = C->n_units;
+  unsigned unit = blockIdx.x;
+  while (unit < n_units) {
+    // the next unit's number, read at the end of this one
+    unsigned next = 0;
+    if (tid == 0) next = gridDim.x + atomicAdd(&C->equeue[0], 1u);
+    const unsigned long long u = units[unit];
+    const long long ii = (long long)(u >> 32);
+    const Item it = items[ii];
+    const int t = it.tile;
+    const unsigned q0 = P.tgt_off[t], q1 = P.tgt_off[t + 1];
+    const long long e0 = it.begin + (long long)(unsigned)u * kEtPiece;
+    const int ne = (int)(min(min(it.end, e0 + kEtPiece), (long long)cursor[2 * t]) - e0);
+    const int4* const ent = entries + e0;
+    const unsigned char* const spc = TB.species + e0;
+    unsigned pairs = 0;   // the wave's members (uniform)
+    for (unsigned q = q0; q < q1; q += kEtTargets) {
+      const int nq = (int)min((unsigned)kEtTargets, q1 - q);
+      for (int k = tid; k < kEtCap; k += kEtThreads) { keys[k] = -1; slots[k] = 0ull; }
+      if (tid < nq) {
+        const BoxRec& R = P.grec[P.tgt[q + tid]];
+        EtTarget& T = targets[tid];
+        const float dm = fmaxf(R.d[0], fmaxf(R.d[1], R.d[2]));
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          T.lo[a] = R.lo[a];
+          T.hi[a] = R.hi[a];
+          T.org[a] = R.org[a];
+          T.nd[a] = (float)R.n[a] * R.d[a];
+          T.d[a] = R.d[a];
+          T.inv_d[a] = R.inv_d[a];
+          T.n[a] = R.n[a];
+        }
+        T.dl = 1.015625f * dm;
+        T.ratio = dm / R.d[0];
+        T.level = R.level;
+        T.tile0 = R.tile0;
+        T.nt0 = R.nt0;
+        T.nt1 = R.nt1;
+      }
+      __syncthreads();
+      auto work = [&](auto pass_c) {
+        constexpr int pass = decltype(pass_c)::value;
+        int np = 0;
+        // the first n collected members, one per lane
+        auto members = [&](int n) {
+          const unsigned w = pd[lane < n ? lane : 0];
+          const int src = (int)(w & (kEtPiece - 1));
+          const EtTarget& R = targets[w >> 10];
+          const int4 u = ent[src];
+          const int su = (int)spc[src];
+          const float x[3] = {__int_as_float(u.x), __int_as_float(u.y), __int_as_float(u.z)};
+          bool mem = lane < n;
+          const int irk = max(R.level - su, 0), nk = 1 << irk;
+          int ci[3], lo[3], ext[3] = {1, 1, 1};
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            ci[a] = (int)floorf(index_quotient(x[a] - R.org[a], R.d[a], R.inv_d[a])) + 1;
+            const int c0 = max(ci[a] - nk, 1), c1 = min(ci[a] + nk, R.n[a]);
+            mem = mem && c0 <= c1;
+            if (irk == 0) {
+              lo[a] = (clampi(ci[a], 1, R.n[a]) - 1) >> P.tshift[a];
+            } else {
+              lo[a] = (c0 - 1) >> P.tshift[a];
+              ext[a] = ((c1 - 1) >> P.tshift[a]) - lo[a] + 1;
+            }
+          }
+          const int4 pe = pack_table(ci[0], ci[1], ci[2], irk, __int_as_float(u.w));
+          auto emit = [&](bool want, int key, const int4& q4) {
+            if (!want) return;
+            if (pass == 0) {
+              const int h = slot_insert<kEtCap>(keys, key);
+              if (h >= 0) atomicAdd(&slots[h], 1ull);
+            } else {
+              const int h = slot_find<kEtCap>(keys, key);
+              if (h < 0) {
+                emit_direct(cursor, start, entries, C, key, q4);
+              } else if (slots[h] != kEtFull) {   // (a full key's slots never change in this pass)
+                entries[atomicAdd(&slots[h], 1ull)] = q4;
+              }
+            }
+          };
+          const int nt = mem ? ext[0] * ext[1] * ext[2] : 0;
+          int key = 2 * (R.tile0 + (lo[2] * R.nt1 + lo[1]) * R.nt0 + lo[0]) + (irk > 0 ? 1 : 0);
+          if (!__ballot(nt > 1)) {
+            emit(nt > 0, key, pe);
+            return;
+          }
+          int tot;
+          const int off = wave_exclusive(nt, tot);
+          int c = 0, cx = 0, cy = 0, row = key, plane = key;
+          for (int w0 = 0; w0 < tot; w0 += kEtWList) {
+            for (; c < nt && off + c < w0 + kEtWList; ++c) {
+              wl[off + c - w0] = (unsigned long long)(unsigned)key | ((unsigned long long)lane << 32);
+              key += 2;
+              if (++cx == ext[0]) {
+                cx = 0;
+                row += 2 * R.nt0;
+                if (++cy == ext[1]) {
+                  cy = 0;
+                  plane += 2 * R.nt0 * R.nt1;
+                  row = plane;
+                }
+                key = row;
+              }
+            }
+            const int len = min(tot - w0, kEtWList);
+            for (int b0 = 0; b0 < len; b0 += 64) {
+              const bool want = b0 + lane < len;
+              const unsigned long long word = wl[want ? b0 + lane : 0];
+              const int from = (int)(word >> 32);
+              int4 q4 = make_int4(0, 0, 0, 0);
+              if (pass == 1) q4 = make_int4(__shfl(pe.x, from), __shfl(pe.y, from), __shfl(pe.z, from), 0);
+              emit(want, (int)(unsigned)word, q4);
+            }
+          }
+        };
+#pragma unroll 1
+        for (int r = tid >> 6; 64 * r < ne; r += kEtThreads / 64) {
+          const bool in = 64 * r + lane < ne;
+          float p[3] = {0.f, 0.f, 0.f}, reach = 0.f;
+          bool ok = false;
+          if (pass == 0) {
+            const int4 v = in ? ent[64 * r + lane] : make_int4(0, 0, 0, 0);
+            const int sp = in ? (int)spc[64 * r + lane] : kSpOutside;
+            ok = sp != kSpOutside;   // a particle outside the box is enumerated by itself
+            p[0] = __int_as_float(v.x);
+            p[1] = __int_as_float(v.y);
+            p[2] = __int_as_float(v.z);
+            reach = ldexpf(dx, -sp);   // N cells of any level >= the species
+          }
+#pragma unroll 1
+          for (int j = 0; j < nq; ++j) {
+            unsigned long long tb = 0;
+            if (pass == 0) {
+              const EtTarget& T = targets[j];
+              const unsigned long long mb =
+                  __ballot(ok && T.lo[0] < p[0] && p[0] < T.hi[0] && T.lo[1] < p[1] && p[1] < T.hi[1] &&
+                           T.lo[2] < p[2] && p[2] < T.hi[2]);
+              if (mb) {
+                pairs += (unsigned)__popcll(mb);
+                // distance past the patch's cells [org, org + n d] against
+                // N cells (at least one); 1/64 of a cell of slack covers the
+                // rounding of the cell index (16,512 cells of 2^-22) and of
+                // this test
+                const float lim = fmaxf(reach * T.ratio + T.dl * 0.015625f, T.dl);
+                float far = 0.f;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                  const float f = p[a] - T.org[a];
+                  far = fmaxf(far, fmaxf(-f, f - T.nd[a]));
+                }
+                tb = mb & __ballot(far <= lim);
+              }
+              if (lane == 0) mask[r][j] = tb;
+            } else {
+              tb = mask[r][j];
+            }
+            if (!tb) continue;
+            if ((tb >> lane) & 1ull)
+              pd[np + __popcll(tb & ((1ull << lane) - 1ull))] = (unsigned)(64 * r + lane) | ((unsigned)j << 10);
+            np += __popcll(tb);
+            if (np >= 64) {
+              members(64);
+              np -= 64;
+              if (lane < np) pd[lane] = pd[64 + lane];
+            }
+          }
+        }
+        if (np > 0) members(np);
+      };
+      work(std::integral_constant<int, 0>());
+      __syncthreads();
+      for (int k = tid; k < kEtCap; k += kEtThreads) {
+        const int key = keys[k];
+        const unsigned long long v = slots[k];
+        if (key >= 0 && v) {
+          const unsigned long long b0 = atomicAdd(&cursor[key], v);
+          slots[k] = b0;
+          if (b0 + v > start[key + 1]) {   // past the capacity: nothing is written, the call is redone
+            slots[k] = kEtFull;
+            set_overflow(C);
+          }
+        }
+      }
+      __syncthreads();
+      work(std::integral_constant<int, 1>());
+      __syncthreads();   // the next batch stages its targets and clears the table
+    }
+    if (lane == 0 && pairs) atomicAdd(&item_pairs[ii], pairs);
+    if (tid == 0) s_next = next;
+    __syncthreads();
+    unit = s_next;
+    __syncthreads();   // every wave has read s_next
+  }
+}
+
+// Table-mode particles outside the box [-L/2, L/2): their base tile is a
+// periodic image, so its target list says nothing about them.  One thread per
+// listed particle walks the patch hash and reserves its entries one by one.
+__global__ void __launch_bounds__(256) emit_outside(Plan P, Parts A, unsigned long long* cursor,
+                                                    const unsigned long long* start, int4* entries, Counters* C,
+                                                    TableBin TB) {
+  const unsigned n = min(C->n_outside, TB.outside_cap);
+  unsigned err = 0;
+  unsigned long long pairs = 0;
+  for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const long long i = (long long)TB.outside[k];
+    enumerate_particle<1>(
+        P, i, A.x[i], A.y[i], A.z[i], A.m[i], species_of(A, i),
+        [&](int g, int t, int wide, int4 e) {
+          if (g > 0) emit_direct(cursor, start, entries, C, 2 * t + wide, e);   // the base entry is binned
+        },
+        [&](int g, int, int, int) { pairs += g > 0 ? 1 : 0; }, err);
+  }
+  if (pairs) atomicAdd(&C->n_pairs, pairs);
+}
+
 // statistics of the call: members = base members + the members every emission
 // item found; entries = the filled part of every tile's range.  Every
 // workgroup adds its grid-stride slice to the counters (cleared at the start
@@ -461,20 +840,49 @@ hipError_t launch_count_to_capacity(unsigned* cnt, long long nkeys, int cus, hip
   return hipGetLastError();
 }
 
-hipError_t launch_bin_base_tsc(const Plan& P, const Parts& A, unsigned long long* cursor,
-                               const unsigned long long* start, int4* entries, Counters* C,
-                               const BlockTables& BT, int cus, hipStream_t s) {
+template <int MODE>
+static hipError_t bin_base_mode(const Plan& P, const Parts& A, unsigned long long* cursor,
+                                const unsigned long long* start, int4* entries, Counters* C, const BlockTables& BT,
+                                const TableBin& TB, int cus, hipStream_t s) {
   const long long nb = hier_bin_blocks(A.n);
   if (nb == 0) return hipSuccess;
   static int per_cu = 0;
   if (per_cu <= 0) {
     int k = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, bin_base_tsc, kHbThreads, 0) != hipSuccess || k <= 0) k = 4;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, bin_base<MODE>, kHbThreads, 0) != hipSuccess || k <= 0) k = 4;
     per_cu = k;
   }
   // the workgroups that fit the chip at once, each taking chunks in turn
   const long long grid = std::min<long long>(nb, (long long)cus * per_cu);
-  bin_base_tsc<<<(unsigned)grid, kHbThreads, 0, s>>>(P, A, cursor, start, entries, C, BT);
+  bin_base<MODE><<<(unsigned)grid, kHbThreads, 0, s>>>(P, A, cursor, start, entries, C, BT, TB);
+  return hipGetLastError();
+}
+
+hipError_t launch_bin_base(const Plan& P, const Parts& A, unsigned long long* cursor,
+                           const unsigned long long* start, int4* entries, Counters* C, const BlockTables& BT,
+                           const TableBin& TB, int cus, hipStream_t s) {
+  return P.mode == 2 ? bin_base_mode<2>(P, A, cursor, start, entries, C, BT, TB, cus, s)
+                     : bin_base_mode<1>(P, A, cursor, start, entries, C, BT, TB, cus, s);
+}
+
+long long emit_pieces(int chunk) { return (chunk + kEtPiece - 1) / kEtPiece; }
+
+hipError_t launch_emit_table(const Plan& P, const Parts& A, const Item* items, long long n_items, int chunk,
+                             unsigned long long* cursor, const unsigned long long* start, int4* entries,
+                             unsigned* item_pairs, Counters* C, const TableBin& TB, int cus, hipStream_t s) {
+  if (n_items > 0) {
+    static int per_cu = 0;
+    if (per_cu <= 0) {
+      int nb = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, emit_table, kEtThreads, 0) != hipSuccess || nb <= 0) nb = 4;
+      per_cu = nb;
+    }
+    list_units<<<(unsigned)((n_items + 255) / 256), 256, 0, s>>>(P, items, n_items, cursor, TB.units, C);
+    const long long most = n_items * emit_pieces(chunk);
+    const int grid = (int)std::min<long long>(most, (long long)cus * per_cu);
+    emit_table<<<grid, kEtThreads, 0, s>>>(P, items, TB.units, cursor, start, entries, item_pairs, C, TB);
+  }
+  emit_outside<<<std::max(cus, 1), 256, 0, s>>>(P, A, cursor, start, entries, C, TB);
   return hipGetLastError();
 }
 

@@ -101,9 +101,9 @@ struct Plan {
   int pad;
   float rad1[3];
   float radc[3];
-  // TSC binning along the hierarchy: the patches whose members are found
-  // from tile t's home entries are tgt[tgt_off[t] .. tgt_off[t+1]) (grid
-  // ids); grec[g] is grid g's box and fields in candidate-record form
+  // binning through the base grid: the patches whose members are found from
+  // tile t's entries are tgt[tgt_off[t] .. tgt_off[t+1]) (grid ids); grec[g]
+  // is grid g's box and fields in candidate-record form
   const unsigned* tgt_off;   // [ntiles + 1]
   const int* tgt;
   const BoxRec* grec;        // [1 + P]
@@ -136,7 +136,9 @@ struct Counters {
                                   // scatter, planning and deposit kernels then do nothing
   unsigned int n_items_eff;       // narrow items the deposit serves (0 after an overflow)
   unsigned int n_wide_eff;        // wide items, which follow the narrow ones
-  unsigned int pad[kLine - 13];
+  unsigned int n_outside;         // table mode: particles outside the box
+  unsigned int n_units;           // table mode: the emission's work units
+  unsigned int pad[kLine - 15];
   unsigned long long pool_fill[kPoolSubs * kLine / 2];   // sub-pool k at [k * kLine / 2]
   unsigned long long epool_fill[kPoolSubs * kLine / 2];  // emission lists, same layout
   unsigned int queue[kQueues * kLine];                   // queue q at [q * kLine]
@@ -175,6 +177,16 @@ struct BlockTables {
   int pad;
 };
 
+// Table mode's binning through the base grid.
+constexpr int kSpOutside = 255;
+struct TableBin {
+  unsigned char* species;    // species of every base-grid entry, kSpOutside: particle outside the box
+  unsigned* outside;         // particles outside the box
+  unsigned long long* units; // the emission's work units
+  unsigned outside_cap;
+  unsigned pad;
+};
+
 // Arguments of the persistent deposit.
 struct DepArgs {
   const int4* entries;       // binned entries, grouped by tile
@@ -189,9 +201,10 @@ struct DepArgs {
   long long* tile_mass_i;    // deterministic: exact fixed-point mass per tile
   double* tile_mass_d;       // atomic: FP64 mass per tile
   int n_queues;              // queues in use (<= kQueues, <= grid)
-  // offsets of the tiles' entry ranges; with the hierarchy binning items cover
-  // capacity ranges, filled up to cursor[2t] (NULL otherwise: every item's
-  // range is filled)
+  // offsets of the tiles' entry ranges; with the binning through the base grid
+  // items cover capacity ranges, filled up to cursor[2t] (narrow) and
+  // cursor[2t+1] (wide), and the base grid's entries are positions in both
+  // modes (NULL otherwise: every item's range is filled)
   const unsigned long long* cursor;
   const unsigned long long* start;
 };

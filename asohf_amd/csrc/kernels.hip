@@ -781,10 +781,11 @@ struct TileLds {
 };
 
 // Whether tile t received entries in this call (its exchange cells are then
-// written): the hierarchy binning fills [start[2t], cursor[2t]) of a
-// capacity range, the count pass fills [start[2t], start[2t+2]) exactly.
+// written): the binning through the base grid fills capacity ranges up to the
+// cursors, the count pass fills [start[2t], start[2t+2]) exactly.
 __device__ __forceinline__ bool tile_filled(const DepArgs& D, int t) {
-  return D.cursor ? D.cursor[2 * t] > D.start[2 * t] : D.start[2 * t + 2] > D.start[2 * t];
+  if (!D.cursor) return D.start[2 * t + 2] > D.start[2 * t];
+  return D.cursor[2 * t] > D.start[2 * t] || D.cursor[2 * t + 1] > D.start[2 * t + 1];
 }
 
 template <int MODE, int RED, int TX, int TY, int TZ>
@@ -818,8 +819,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     const int i0 = tx * TX + 1, j0 = ty * TY + 1, k0c = tz * TZ + 1;
     const bool periodic = g == 0;
 
-    // the item's filled entries: with the hierarchy binning the tile's
-    // entries end at cursor[2t]
+    // the item's filled entries
     long long len = it.end - it.begin;
     if (D.cursor) len = min(it.end, (long long)D.cursor[2 * t]) - it.begin;
     len = uniform64(len);   // wave-uniform: kept in scalar registers
@@ -865,7 +865,11 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
         }
       } else {
         int irk;
-        unpack_table(v, ci[0], ci[1], ci[2], irk, m);
+        if (D.cursor && g == 0)
+          unpack_table(table_base_entry(P, __int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z),
+                                        __int_as_float(v.w)), ci[0], ci[1], ci[2], irk, m);
+        else
+          unpack_table(v, ci[0], ci[1], ci[2], irk, m);
 #pragma unroll
         for (int k = 0; k < 3; ++k) { wx[k] = k0[k]; wy[k] = k0[k]; wz[k] = k0[k]; }
       }
@@ -983,8 +987,10 @@ __device__ __forceinline__ void conv4(const double* line, int st, int nk, const 
 // Bound by reading the entries once per class and by the LDS reads of the
 // convolution.  As part of the narrow kernel the histogram had one layout, so
 // N = 8 and more walked every entry's box (29 G adds at 512^3, 6 levels), and
-// its LDS left one narrow workgroup per CU: 113 ms, now 14.4 here and 6.0 ms
-// in the narrow kernel; 256^3, 4 levels 1,094 -> 132 + 715 us.
+// its LDS left one narrow workgroup per CU: 113 ms, now 10.8 here and 6.2 ms
+// in the narrow kernel; 256^3, 4 levels 1,094 -> 68 + 762 us.  256 threads or
+// a 41 KB histogram (three workgroups per CU) were slower: 19.2 and 17.5 ms
+// when this took 14.7.
 template <int RED, int TX, int TY, int TZ>
 __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs D) {
   using Acc = typename AccT<RED>::T;
@@ -1015,8 +1021,13 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
     __syncthreads();
     const unsigned idx = __builtin_amdgcn_readfirstlane(s_item);
     if (idx >= n_wide) break;
-    const Item it = D.items[n_narrow + idx];
+    Item it = D.items[n_narrow + idx];
     const int t = __builtin_amdgcn_readfirstlane(it.tile);
+    if (D.cursor) it.end = min(it.end, (long long)D.cursor[2 * t + 1]);
+    if (it.end <= it.begin) {
+      __syncthreads();   // every wave has read s_item before thread 0 takes the next item
+      continue;
+    }
     const int g = __builtin_amdgcn_readfirstlane(P.tile_grid[t]);
     const GridDesc& G = P.grids[g];
     const int local = t - G.tile0;
@@ -1025,11 +1036,18 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
     // entries per class (wave ballots, one LDS add per wave and class)
     {
       unsigned cnt[kNLevels + 1] = {};
-      for (long long b0 = it.begin; b0 < it.end; b0 += nthr) {
-        const long long e = b0 + tid;
-        const int irk_e = e < it.end ? (D.entries[e].y >> 16) : 0;
+      for (long long b0 = it.begin; b0 < it.end; b0 += 4 * nthr) {   // four loads in flight
+        int irk_e[4];
 #pragma unroll
-        for (int k = 1; k <= kNLevels; ++k) cnt[k] += (unsigned)__popcll(__ballot(irk_e == k));
+        for (int r = 0; r < 4; ++r) {
+          const long long e = b0 + r * nthr + tid;
+          irk_e[r] = e < it.end ? (D.entries[e].y >> 16) : 0;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+          for (int k = 1; k <= kNLevels; ++k) cnt[k] += (unsigned)__popcll(__ballot(irk_e[r] == k));
+        }
       }
       if ((tid & 63) == 0)
         for (int k = 1; k <= kNLevels; ++k)
@@ -1043,7 +1061,7 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
       if (j0 > G.n[1] || k0 > G.n[2]) continue;  // past the grid: never read
       for (int c = tid; c < B; c += nthr) acc[c] = 0;   // zero bits: 0 as FP64 too
       __syncthreads();
-      for (int irk = 1; irk <= kNLevels; ++irk) {
+      for (int irk = 1; irk <= P.nl; ++irk) {
         const unsigned ncls = s_ccnt[irk];
         if (ncls == 0u) continue;
         const int nk = 1 << irk;
@@ -1070,9 +1088,9 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
             if (irk_e != irk) continue;
             const int cx = ci[0] - i0, cy = ci[1] - j0, cz = ci[2] - k0;
             if (cx < -nk || cx >= BX + nk || cy < -nk || cy >= BY + nk || cz < -nk || cz >= BZ + nk) continue;
-            const double ms = (double)(m * scale);
+            const double ms = (double)(m * scale);   // below 2^30 units
             if (w.form == 0) {
-              lds_add(hist + (cx + nk) + w.px * (cy + nk) + w.pz * (cz + nk), __double2ll_rn(ms));
+              lds_add(hist + (cx + nk) + w.px * (cy + nk) + w.pz * (cz + nk), (long long)__double2int_rn(ms));
               continue;
             }
             const int z0 = max(0, cz - nk), z1 = min(BZ - 1, cz + nk);
@@ -1080,11 +1098,11 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
             for (int z = z0; z <= z1; ++z) {
               const double mz = ms * Kd[z - cz];
               if (w.form == 1) {
-                lds_add(hist + (cx + nk) + w.px * (cy + nk) + w.pz * z, __double2ll_rn(mz));
+                lds_add(hist + (cx + nk) + w.px * (cy + nk) + w.pz * z, (long long)__double2int_rn(mz));
                 continue;
               }
               for (int y = y0; y <= y1; ++y)
-                lds_add(hist + (cx + nk) + w.px * y + w.pz * z, __double2ll_rn(mz * Kd[y - cy]));
+                lds_add(hist + (cx + nk) + w.px * y + w.pz * z, (long long)__double2int_rn(mz * Kd[y - cy]));
             }
           }
           __syncthreads();
@@ -1143,22 +1161,39 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
           __syncthreads();
           continue;
         }
-        // ---- direct: one wave per entry.  The entry's box clipped to the
-        // block (bx x by x bz cells) is walked as one flat range, lane l taking
-        // cells l, l + 64, ...; its (x, y, z) counters advance by constant
-        // steps, so the loop has no divisions.  The next entry is loaded while
-        // this one deposits.  Terms are ((m*Kx)*Ky)*Kz as in the reference's
-        // loop.
+        // ---- direct: a wave reads 64 entries and takes those of the class one
+        // by one (short lists: every wave reads them all and takes every
+        // eighth, so no wave is left without work).  The entry's box clipped to the block (bx x by x bz cells) is
+        // walked as one flat range, lane l taking cells l, l + 64, ...; its
+        // (x, y, z) counters advance by constant steps, so the loop has no
+        // divisions.  Terms are ((m*Kx)*Ky)*Kz as in the reference's loop.
         const int ex = min(BX, G.n[0] - i0 + 1), ey = min(BY, G.n[1] - j0 + 1), ez = min(BZ, G.n[2] - k0 + 1);
         const int wave = tid >> 6, lane = tid & 63, nwaves = nthr >> 6;
-        long long e = it.begin + wave;
-        int4 nxt = e < it.end ? D.entries[e] : make_int4(0, 0, 0, 0);
-        for (; e < it.end; e += nwaves) {
+        const int4 none = make_int4(0, 0, 0, 0);   // class 0
+        static_assert(nthr / 64 == 8, "every eighth lane");
+        const bool shared = it.end - it.begin <= 4 * nthr;
+        const unsigned long long share = shared ? 0x0101010101010101ull << wave : ~0ull;
+        const int step = shared ? 64 : 64 * nwaves;
+        long long e = it.begin + (shared ? 0 : 64 * wave);
+        int4 nxt = e + lane < it.end ? D.entries[e + lane] : none;
+        unsigned long long todo = 0;
+        int4 mine = none;
+        for (;;) {
+          if (!todo) {
+            if (e >= it.end) break;
+            mine = nxt;
+            e += step;
+            nxt = e + lane < it.end ? D.entries[e + lane] : none;
+            todo = __ballot((mine.y >> 16) == irk) & share;
+            continue;
+          }
+          const int src = __ffsll((long long)todo) - 1;
+          todo &= todo - 1;
           int ci[3], irk_e;
           float m;
-          unpack_table(nxt, ci[0], ci[1], ci[2], irk_e, m);
-          if (e + nwaves < it.end) nxt = D.entries[e + nwaves];
-          if (irk_e != irk) continue;
+          unpack_table(make_int4(__builtin_amdgcn_readlane(mine.x, src), __builtin_amdgcn_readlane(mine.y, src),
+                                 __builtin_amdgcn_readlane(mine.z, src), 0),
+                       ci[0], ci[1], ci[2], irk_e, m);
           const int xa = max(ci[0] - nk, i0), xb = min(ci[0] + nk, i0 + ex - 1);
           const int ya = max(ci[1] - nk, j0), yb = min(ci[1] + nk, j0 + ey - 1);
           const int za = max(ci[2] - nk, k0), zb = min(ci[2] + nk, k0 + ez - 1);

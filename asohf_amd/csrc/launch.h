@@ -39,13 +39,17 @@ hipError_t launch_zero_split(const Plan& P, const DepArgs& D, int reduction, int
 long long exchange_cells(const int tile[3]);
 hipError_t launch_combine(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s);
 hipError_t launch_grid_sums(const Plan& P, const DepArgs& D, int reduction, double* grid_mass, hipStream_t s);
-// TSC binning along the hierarchy (hier.hip)
+// binning through the base grid (hier.hip)
 hipError_t launch_cursor_reset(const unsigned long long* start, unsigned long long* cursor, long long nkeys,
                                int cus, hipStream_t s);
 hipError_t launch_count_to_capacity(unsigned* cnt, long long nkeys, int cus, hipStream_t s);
-hipError_t launch_bin_base_tsc(const Plan& P, const Parts& A, unsigned long long* cursor,
-                               const unsigned long long* start, int4* entries, Counters* C,
-                               const BlockTables& BT, int cus, hipStream_t s);
+hipError_t launch_bin_base(const Plan& P, const Parts& A, unsigned long long* cursor,
+                           const unsigned long long* start, int4* entries, Counters* C, const BlockTables& BT,
+                           const TableBin& TB, int cus, hipStream_t s);
+long long emit_pieces(int chunk);   // emission work units of an item of `chunk` entries
+hipError_t launch_emit_table(const Plan& P, const Parts& A, const Item* items, long long n_items, int chunk,
+                             unsigned long long* cursor, const unsigned long long* start, int4* entries,
+                             unsigned* item_pairs, Counters* C, const TableBin& TB, int cus, hipStream_t s);
 hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, long long item_hi, int level,
                            unsigned long long* cursor, const unsigned long long* start, int4* entries,
                            unsigned* item_pairs, Counters* C, int cus, hipStream_t s);
