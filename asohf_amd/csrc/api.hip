@@ -163,6 +163,9 @@ struct PipeArgs {
   int ntiles, chunk, chunk_wide, red, grid, block, cus, elem;
   // binning through the base grid
   unsigned* item_pairs;
+  unsigned* split_n;                   // tiles with several work items, and their list
+  int* split_tiles;
+  unsigned* host;                      // pinned counters the last kernel writes
   TableBin TB;
   long long lvl_items[kNLevels + 2];   // items of level l: [lvl_items[l], lvl_items[l + 1])
   long long n_items, n_narrow;
@@ -173,6 +176,7 @@ struct PipeArgs {
 struct asohf_ctx {
   int device = 0;
   int cus = 0;
+  double clock_khz = 0;   // rate of the device clock
   hipStream_t stream = nullptr;
   std::string err;
   asohf_tune tune{{16, 8, 8}, 256, 4096, 16};
@@ -182,6 +186,7 @@ struct asohf_ctx {
   DBuf flags, idx, pool, pool_off, pool_nk, blk_pairs, blk_mmax, item_off;
   DBuf elist, eoff, ecount;
   DBuf spc, outside, units;                // table mode: species of the base entries, particles outside the box, work units
+  DBuf split;                              // tiles with several work items: their number, then the list
   DBuf ipairs;                             // members found per work item (TSC hierarchy binning)
   void* noalloc = nullptr;                 // this device's scratch array of order.hip (device address)
   DBuf sp_k[4], sp_dens, sp_cnt, sp_tmp;   // species partition
@@ -855,7 +860,8 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   // holds all of the tile's wide entries, otherwise (and for the widest
   // classes) entry by entry, which costs hundreds of adds each; so items are
   // long (2^20 masses below 2^30 units sum below 2^53, exact in FP64)
-  a.chunk_wide = (int)std::min(std::max(a.chunk, 1 << 17) * 8ll, 1ll << 22);
+  a.P.per_tile = a.P.mode == 1 && a.red == 1 ? 1 : 0;
+  a.chunk_wide = a.P.per_tile ? a.chunk * 8 : (int)std::min(std::max(a.chunk, 1 << 17) * 8ll, 1ll << 22);
   a.cus = ctx->cus;
   const int waves = std::max(ctx->tune.waves_per_cu, 1);
   a.block = ctx->tune.block;
@@ -900,7 +906,8 @@ static asohf_status enqueue_deposit(asohf_ctx* ctx, const PipeArgs& a, hipStream
   if (events) HIPCHK(hipEventRecord(ctx->ev[2], s), "event");
   HIPCHK(launch_scatter(a.P, a.A, a.cursor, const_cast<int4*>(a.D.entries), a.cap_entries, a.BT, a.C, a.cus, s), "scatter kernel");
   if (events) HIPCHK(hipEventRecord(ctx->ev[3], s), "event");
-  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.chunk_wide, a.item_off, const_cast<Item*>(a.D.items), a.C, s),
+  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.chunk_wide, a.item_off, const_cast<Item*>(a.D.items), nullptr,
+                           nullptr, a.C, s),
          "writing items");
   HIPCHK(launch_zero_split(a.P, a.D, a.red, a.cus, s), "clearing split tiles");
   if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
@@ -1028,7 +1035,12 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   }
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
-  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.P.mode == 2 ? 0 : a.chunk_wide, a.item_off, const_cast<Item*>(a.D.items), a.C, s),
+  HIPCHK(ctx->split.ensure(sizeof(int) * (a.ntiles + 1ll)), "allocating the split tiles");
+  a.split_n = ctx->split.as<unsigned>();
+  a.split_tiles = ctx->split.as<int>() + 1;
+  HIPCHK(launch_fill_u32(a.split_n, 0u, 1, s), "clearing the split tiles");
+  HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.P.mode == 2 ? 0 : a.chunk_wide, a.item_off,
+                           const_cast<Item*>(a.D.items), a.split_tiles, a.split_n, a.C, s),
          "writing items");
   ctx->hier_nitems = n_items;
   ctx->hier_nnarrow = ctx->hier_items[nl + 1];
@@ -1041,6 +1053,9 @@ static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
   a.D.items = ctx->items.as<Item>();
   a.D.cursor = a.cursor;
   a.item_pairs = ctx->ipairs.as<unsigned>();
+  a.split_n = ctx->split.as<unsigned>();
+  a.split_tiles = ctx->split.as<int>() + 1;
+  a.host = (unsigned*)ctx->hcount;
   a.n_items = ctx->hier_nitems;
   a.n_narrow = ctx->hier_nnarrow;
   if (a.P.mode == 1) {
@@ -1059,40 +1074,29 @@ static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
 // One call on the planned capacities: base-grid binning, one emission pass
 // per level, the persistent deposit over every item, the output cells, the
 // grid sums and the call's statistics; no host round trip (graph-capturable).
-static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t s, bool events) {
-  HIPCHK(launch_fill_u32((unsigned*)a.C, 0u, sizeof(Counters) / 4, s), "clearing counters");
-  HIPCHK(launch_fill_u32(&a.C->n_items_eff, (unsigned)a.n_narrow, 1, s), "queue length");
-  if (a.n_items > a.n_narrow)
-    HIPCHK(launch_fill_u32(&a.C->n_wide_eff, (unsigned)(a.n_items - a.n_narrow), 1, s), "queue length");
-  HIPCHK(launch_fill_u32(a.item_pairs, 0u, a.n_items, s), "clearing item sums");
-  HIPCHK(launch_cursor_reset(a.start, a.cursor, a.nkeys, a.cus, s), "cursors");
-  HIPCHK(launch_bin_base(a.P, a.A, a.cursor, a.start, const_cast<int4*>(a.D.entries), a.C, a.BT, a.TB, a.cus, s),
-         "base-grid binning");
-  if (a.A.n > 0) HIPCHK(launch_reduce_blocks(a.BT, hier_bin_blocks(a.A.n), a.C, a.cus, s), "block sums");
-  if (events) {
-    HIPCHK(hipEventRecord(ctx->ev[1], s), "event");
-    HIPCHK(hipEventRecord(ctx->ev[2], s), "event");
-  }
+static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t s) {
+  int4* const entries = const_cast<int4*>(a.D.entries);
+  HIPCHK(launch_begin_call(a.D, a.P.tile, a.red, a.n_narrow, a.n_items - a.n_narrow, a.item_pairs, a.n_items, a.cursor,
+                           a.nkeys, a.split_tiles, a.split_n, a.cus, s),
+         "starting the call");
+  HIPCHK(launch_bin_base(a.P, a.A, a.cursor, a.start, entries, a.C, a.BT, a.TB, a.cus, s), "base-grid binning");
+  HIPCHK(launch_after_bin(a.P, a.A, a.BT, a.D.items, a.lvl_items[1], a.cursor, a.start, entries, a.C, a.TB, a.cus, s),
+         "block sums");
   if (a.P.mode == 1 && a.nl > 0)
-    HIPCHK(launch_emit_table(a.P, a.A, a.D.items, a.lvl_items[1], a.chunk, a.cursor, a.start, const_cast<int4*>(a.D.entries),
-                             a.item_pairs, a.C, a.TB, a.cus, s),
+    HIPCHK(launch_emit_table(a.P, a.D.items, a.lvl_items[1], a.chunk, a.cursor, a.start, entries, a.item_pairs, a.C,
+                             a.TB, a.cus, s),
            "emission pass");
   for (int l = 0; a.P.mode == 2 && l < a.nl; ++l) {
     if (!(a.emit_levels & (1u << l))) continue;
-    HIPCHK(launch_emit_tsc(a.P, a.D.items, a.lvl_items[l], a.lvl_items[l + 1], l, a.cursor, a.start,
-                           const_cast<int4*>(a.D.entries), a.item_pairs, a.C, a.cus, s),
+    HIPCHK(launch_emit_tsc(a.P, a.D.items, a.lvl_items[l], a.lvl_items[l + 1], l, a.cursor, a.start, entries,
+                           a.item_pairs, a.C, a.cus, s),
            "emission pass");
   }
-  if (events) HIPCHK(hipEventRecord(ctx->ev[3], s), "event");
-  HIPCHK(launch_zero_split(a.P, a.D, a.red, a.cus, s), "clearing split tiles");
-  if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
   HIPCHK(launch_deposit(a.P, a.D, a.red, a.grid, a.block, s), "deposit kernel");
   if (a.n_items > a.n_narrow) HIPCHK(launch_deposit_wide(a.P, a.D, a.red, a.cus, s), "wide deposit kernel");
-  if (events) HIPCHK(hipEventRecord(ctx->ev[8], s), "event");
   HIPCHK(launch_combine(a.P, a.D, a.red, a.cus, s), "output cells");
-  if (events) HIPCHK(hipEventRecord(ctx->ev[5], s), "event");
-  if (a.grid_mass) HIPCHK(launch_grid_sums(a.P, a.D, a.red, a.grid_mass, s), "grid sums");
-  HIPCHK(launch_hier_stats(a.item_pairs, a.n_items, a.start, a.cursor, a.nkeys, a.C, a.cus, s), "statistics");
+  HIPCHK(launch_finish_call(a.P, a.D, a.red, a.grid_mass, a.item_pairs, a.n_items, a.nkeys, a.host, a.cus, s),
+         "sums");
   return ASOHF_OK;
 }
 
@@ -1120,16 +1124,15 @@ static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A
     }
     hier_bind(ctx, a);
     hipStream_t rs = s;
-    bool phases = true;
-    if (o.use_graph && !planned) {
-      phases = false;
+    const bool graph_form = o.use_graph && !planned;
+    if (graph_form) {
       rs = ctx->stream;
       if (!ctx->gexec || memcmp(&ctx->gkey, &a, sizeof(a)) != 0) {
         if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
         ctx->gexec = nullptr;
         hipGraph_t graph = nullptr;
         HIPCHK(hipStreamBeginCapture(rs, hipStreamCaptureModeThreadLocal), "graph capture");
-        st = enqueue_hier(ctx, a, rs, false);
+        st = enqueue_hier(ctx, a, rs);
         const hipError_t e = hipStreamEndCapture(rs, &graph);
         if (st != ASOHF_OK) {
           if (e == hipSuccess && graph) (void)hipGraphDestroy(graph);
@@ -1146,17 +1149,15 @@ static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A
         HIPCHK(hipEventRecord(ctx->ev[7], s), "event");
         HIPCHK(hipStreamWaitEvent(rs, ctx->ev[7], 0), "stream wait");
       }
-      HIPCHK(hipEventRecord(ctx->ev[0], rs), "event");
       HIPCHK(hipGraphLaunch(ctx->gexec, rs), "graph launch");
     } else {
-      if (!planned) HIPCHK(hipEventRecord(ctx->ev[0], rs), "event");
-      st = enqueue_hier(ctx, a, rs, true);
+      st = enqueue_hier(ctx, a, rs);
       if (st != ASOHF_OK) return st;
     }
-    HIPCHK(hipEventRecord(ctx->ev[6], rs), "event");
-    HIPCHK(hipMemcpyAsync(ctx->hcount, a.C, sizeof(Counters), hipMemcpyDeviceToHost, rs), "reading counters");
+    if (planned) HIPCHK(hipEventRecord(ctx->ev[6], rs), "event");
     HIPCHK(hipStreamSynchronize(rs), "batched build");
-    Counters hc = *ctx->hcount;
+    // the last kernel wrote the scalar counters and the clock to the host
+    Counters& hc = *ctx->hcount;
     st = decode_err(ctx, hc.err);
     if (st != ASOHF_OK) return st;
     if (hc.overflow) {
@@ -1169,7 +1170,17 @@ static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A
       continue;
     }
     hc.n_items = (unsigned long long)a.n_items;
-    set_stats(ctx, A, hc, phases);
+    set_stats(ctx, A, hc, false);
+    ctx->stats_pending = planned;   // a planned call's total includes its planning: from the events
+    auto ms = [&](int k0, int k1) { return (double)(hc.clk[k1] - hc.clk[k0]) / ctx->clock_khz; };
+    ctx->stats.ms_total = ms(kClkBegin, kClkEnd);
+    if (!graph_form) {   // the graph form reports the total only
+      ctx->stats.ms_bin = ms(kClkBegin, kClkBinned);
+      ctx->stats.ms_scatter = ms(kClkBinned, kClkDeposit);
+      ctx->stats.ms_deposit = ms(kClkDeposit, kClkCombine);
+      ctx->stats.ms_split = ms(kClkCombine, kClkSums);
+      ctx->stats.ms_sums = ms(kClkSums, kClkEnd);
+    }
     return ASOHF_OK;
   }
   return fail(ctx, ASOHF_ERR_CAPACITY, "tile capacities overflowed right after an exact count");
@@ -1183,7 +1194,12 @@ static asohf_status run_hier(asohf_ctx* ctx, const asohf_opts& o, const Parts& A
 static asohf_status run_batched(asohf_ctx* ctx, const asohf_opts& o, const Parts& A, float* u1, float* u11,
                                 double* grid_mass, hipStream_t s) {
   if (A.n > (1ll << 32)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^32 particles");
-  if (!ctx->hier_off && (o.mode == ASOHF_MODE_TSC || ctx->plan.table_base)) {
+  // Kernel table with atomic sums: an FP32 sum of equal terms drifts by an
+  // amount that depends on how many of them each partial sum holds, and the
+  // grid masses report that drift.  This form keeps the partial sums it always
+  // had: count and scatter passes, an entry in every tile a stencil touches.
+  const bool per_tile = o.mode == ASOHF_MODE_TABLE && o.reduction == ASOHF_REDUCE_ATOMIC;
+  if (!ctx->hier_off && !per_tile && (o.mode == ASOHF_MODE_TSC || ctx->plan.table_base)) {
     bool many_outside = false;
     const asohf_status st = run_hier(ctx, o, A, u1, u11, grid_mass, s, &many_outside);
     if (st != ASOHF_OK || !many_outside) return st;
@@ -1326,6 +1342,12 @@ asohf_status asohf_hip_create(asohf_ctx** out, int32_t device) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, ctx->device) != hipSuccess) { delete ctx; return ASOHF_ERR_HIP; }
   ctx->cus = prop.multiProcessorCount;
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device) != hipSuccess || khz <= 0) {
+    delete ctx;
+    return ASOHF_ERR_HIP;
+  }
+  ctx->clock_khz = khz;
   {
     // ASOHF_TSC_BINNING=hash: the build bins with the patch-hash count and
     // scatter passes
@@ -1357,7 +1379,7 @@ void asohf_hip_destroy(asohf_ctx* ctx) {
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
                   &ctx->item_off, &ctx->plan_blob, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum, &ctx->counters,
-                  &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries, &ctx->items,
+                  &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->split, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries, &ctx->items,
                   &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1], &ctx->h_in[2],
                   &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0], &ctx->ord[1],
                   &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount, &ctx->sp_k[0],
@@ -2312,7 +2334,7 @@ asohf_status asohf_hip_release_workspaces(asohf_ctx* ctx) {
   ctx->gexec = nullptr;
   DBuf* bufs[] = {&ctx->pool, &ctx->pool_off, &ctx->pool_nk, &ctx->blk_pairs, &ctx->blk_mmax,
                   &ctx->item_off, &ctx->cnt, &ctx->start, &ctx->cursor, &ctx->bsum,
-                  &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries,
+                  &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->split, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries,
                   &ctx->items, &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1],
                   &ctx->h_in[2], &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0],
                   &ctx->ord[1], &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount,

@@ -36,6 +36,11 @@ __device__ __forceinline__ unsigned wave_or(unsigned v) {
   return v;
 }
 
+// the device clock at the start of a kernel that opens a phase of the call
+__device__ __forceinline__ void stamp(Counters* C, int k) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) C->clk[k] = wall_clock64();
+}
+
 // fixed-shape block sum (deterministic for a given blockDim)
 template <class T>
 __device__ T block_sum(T v, T* sh) {
@@ -254,10 +259,22 @@ __device__ __forceinline__ void unpack_table(int4 e, int& ix, int& jy, int& kz, 
   m = __int_as_float(e.z);
 }
 
+// Tiles touched by the wrapped cells {c-1, c, c+1} along one base axis.
+// Returns the number of distinct tile indices (1..3) in t[].
+__device__ __forceinline__ int base_axis_tiles(int c, int n, int sh, int t[3]) {
+  int a = (wrap1(c - 1, n) - 1) >> sh, b = (wrap1(c, n) - 1) >> sh, d = (wrap1(c + 1, n) - 1) >> sh;
+  int k = 0;
+  t[k++] = a;
+  if (b != a) t[k++] = b;
+  if (d != a && d != b) t[k++] = d;
+  return k;
+}
+
 // Enumerates the entries of a particle, calling emit(g, tile, wide, entry):
 // a 27-cell member (TSC, or a table-mode member with N = 1) once, for the tile
 // that holds its centre cell (clamped into a patch, wrapped on the base grid);
-// a wide member (N >= 2) once per tile its clipped box touches.  member(g, ix,
+// a wide member (N >= 2), and with P.per_tile any table-mode member, once per
+// tile its (clipped or wrapped) box touches.  member(g, ix,
 // jy, kz) is called once per (particle, grid) member of the mode's box rule
 // with the reference's cell index of that grid (before any wrap or
 // clipping).  err receives validation flags.
@@ -307,9 +324,19 @@ __device__ __forceinline__ void enumerate_particle(const Plan& P, long long i, f
     int4 e;
     if (MODE == 2) e = make_int4(__float_as_int(x), __float_as_int(y), __float_as_int(z), __float_as_int(m));
     else e = pack_table(ix, jy, kz, 0, m);
-    const int tx = (wrap1(ix, bn[0]) - 1) >> P.tshift[0], ty = (wrap1(jy, bn[1]) - 1) >> P.tshift[1],
-              tz = (wrap1(kz, bn[2]) - 1) >> P.tshift[2];
-    emit(0, btile0 + (tz * bnt1 + ty) * bnt0 + tx, 0, e);
+    if (MODE == 1 && P.per_tile) {
+      int tx[3], ty[3], tz[3];
+      const int nx_ = base_axis_tiles(ix, bn[0], P.tshift[0], tx);
+      const int ny_ = base_axis_tiles(jy, bn[1], P.tshift[1], ty);
+      const int nz_ = base_axis_tiles(kz, bn[2], P.tshift[2], tz);
+      for (int c = 0; c < nz_; ++c)
+        for (int b = 0; b < ny_; ++b)
+          for (int a = 0; a < nx_; ++a) emit(0, btile0 + (tz[c] * bnt1 + ty[b]) * bnt0 + tx[a], 0, e);
+    } else {
+      const int tx = (wrap1(ix, bn[0]) - 1) >> P.tshift[0], ty = (wrap1(jy, bn[1]) - 1) >> P.tshift[1],
+                tz = (wrap1(kz, bn[2]) - 1) >> P.tshift[2];
+      emit(0, btile0 + (tz * bnt1 + ty) * bnt0 + tx, 0, e);
+    }
   }
   // ---------------- patches, level by level ----------------
   // When every patch's membership box lies inside a box of the level above
@@ -354,7 +381,7 @@ __device__ __forceinline__ void enumerate_particle(const Plan& P, long long i, f
       if (MODE == 2) e = make_int4(__float_as_int(x), __float_as_int(y), __float_as_int(z), __float_as_int(m));
       else e = pack_table(ci[0], ci[1], ci[2], irk, m);
       const int wide = (MODE == 1 && irk > 0) ? 1 : 0;
-      if (!wide) {
+      if (!wide && !(MODE == 1 && P.per_tile)) {
         const int tx = (clampi(ci[0], 1, gn[0]) - 1) >> P.tshift[0], ty = (clampi(ci[1], 1, gn[1]) - 1) >> P.tshift[1],
                   tz = (clampi(ci[2], 1, gn[2]) - 1) >> P.tshift[2];
         emit(g, gtile0 + (tz * gnt1 + ty) * gnt0 + tx, 0, e);

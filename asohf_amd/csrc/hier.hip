@@ -99,14 +99,6 @@ __device__ __forceinline__ void emit_direct(unsigned long long* cursor, const un
 
 }  // namespace
 
-// cursor[k] = start[k]: every tile's range starts empty
-__global__ void __launch_bounds__(256) cursor_reset(const unsigned long long* start, unsigned long long* cursor,
-                                                    long long nkeys) {
-  for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < nkeys;
-       k += (long long)gridDim.x * blockDim.x)
-    cursor[k] = start[k];
-}
-
 // per-key capacity from an exact count: the count plus an eighth plus 32
 // entries, so a later snapshot with a similar distribution fits
 __global__ void __launch_bounds__(256) count_to_capacity(unsigned* cnt, long long nkeys) {
@@ -520,28 +512,6 @@ __device__ __forceinline__ int wave_exclusive(int v, int& total) {
   return s - v;
 }
 
-// The call's emission work units: (item << 32 | piece) for every piece of
-// kEtPiece filled entries of the items of tiles with targets.
-__global__ void __launch_bounds__(256) list_units(Plan P, const Item* items, long long n_items,
-                                                  const unsigned long long* cursor, unsigned long long* units,
-                                                  Counters* C) {
-  const long long ii = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  int n = 0;
-  if (ii < n_items) {
-    const Item it = items[ii];
-    if (P.tgt_off[it.tile] < P.tgt_off[it.tile + 1]) {
-      const long long len = min(it.end, (long long)cursor[2 * it.tile]) - it.begin;
-      n = len > 0 ? (int)((len + kEtPiece - 1) / kEtPiece) : 0;
-    }
-  }
-  int tot;
-  const int off = wave_exclusive(n, tot);
-  unsigned b0 = 0;
-  if (__lane_id() == 0 && tot) b0 = atomicAdd(&C->n_units, (unsigned)tot);
-  b0 = __builtin_amdgcn_readfirstlane(b0);
-  for (int k = 0; k < n; ++k) units[b0 + off + k] = ((unsigned long long)ii << 32) | (unsigned)k;
-}
-
 // The kernel-table members of every patch from the base-grid entries.  A work
 // unit is kEtPiece entries of a base tile's work item; workgroups take units
 // from the list in turn, the next one's number on its way while this one is
@@ -778,60 +748,71 @@ __global__ void __launch_bounds__(kEtThreads) emit_table(Plan P, const Item* ite
   }
 }
 
-// Table-mode particles outside the box [-L/2, L/2): their base tile is a
-// periodic image, so its target list says nothing about them.  One thread per
-// listed particle walks the patch hash and reserves its entries one by one.
-__global__ void __launch_bounds__(256) emit_outside(Plan P, Parts A, unsigned long long* cursor,
-                                                    const unsigned long long* start, int4* entries, Counters* C,
-                                                    TableBin TB) {
-  const unsigned n = min(C->n_outside, TB.outside_cap);
-  unsigned err = 0;
-  unsigned long long pairs = 0;
-  for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-    const long long i = (long long)TB.outside[k];
-    enumerate_particle<1>(
-        P, i, A.x[i], A.y[i], A.z[i], A.m[i], species_of(A, i),
-        [&](int g, int t, int wide, int4 e) {
-          if (g > 0) emit_direct(cursor, start, entries, C, 2 * t + wide, e);   // the base entry is binned
-        },
-        [&](int g, int, int, int) { pairs += g > 0 ? 1 : 0; }, err);
-  }
-  if (pairs) atomicAdd(&C->n_pairs, pairs);
-}
-
-// statistics of the call: members = base members + the members every emission
-// item found; entries = the filled part of every tile's range.  Every
-// workgroup adds its grid-stride slice to the counters (cleared at the start
-// of the call; integer sums, so the order does not matter).
-__global__ void __launch_bounds__(256) hier_stats(const unsigned* item_pairs, long long n_items,
-                                                 const unsigned long long* start,
-                                                 const unsigned long long* cursor, long long nkeys, Counters* C) {
-  __shared__ unsigned long long sp[4], se[4];
-  unsigned long long p = 0, e = 0;
+// Between the base binning and the emission: the call's base members and
+// largest mass from the per-chunk partials (as reduce_blocks folds them), and
+// in table mode the emission's work units, (item << 32 | piece) for every piece
+// of kEtPiece filled entries of the items of tiles with targets, and the
+// particles outside the box [-L/2, L/2), whose base tile is a periodic image, so
+// that its target list says nothing about them: one thread each walks the patch
+// hash and reserves its entries one by one.
+template <int MODE>
+__global__ void __launch_bounds__(256) after_bin(Plan P, Parts A, BlockTables BT, long long nblk, const Item* items,
+                                                 long long n_items, unsigned long long* cursor,
+                                                 const unsigned long long* start, int4* entries, Counters* C,
+                                                 TableBin TB) {
+  __shared__ unsigned long long sp[4];
+  __shared__ float sm[4];
+  stamp(C, kClkBinned);
   const long long i0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, di = (long long)gridDim.x * blockDim.x;
-  for (long long i = i0; i < n_items; i += di) p += item_pairs[i];
-  for (long long k = i0; k < nkeys; k += di) e += cursor[k] - start[k];
+  unsigned long long p = 0;
+  float mm = 0.f;
+  for (long long b = i0; b < nblk; b += di) {
+    p += BT.pairs[b];
+    mm = fmaxf(mm, __uint_as_float(BT.mmax[b]));
+  }
+  if (MODE == 1 && P.nl > 0) {
+    for (long long k0 = i0 - __lane_id(); k0 < n_items; k0 += di) {
+      const long long ii = k0 + __lane_id();
+      int n = 0;
+      if (ii < n_items) {
+        const Item it = items[ii];
+        if (P.tgt_off[it.tile] < P.tgt_off[it.tile + 1]) {
+          const long long len = min(it.end, (long long)cursor[2 * it.tile]) - it.begin;
+          n = len > 0 ? (int)((len + kEtPiece - 1) / kEtPiece) : 0;
+        }
+      }
+      int tot;
+      const int off = wave_exclusive(n, tot);
+      unsigned b0 = 0;
+      if (__lane_id() == 0 && tot) b0 = atomicAdd(&C->n_units, (unsigned)tot);
+      b0 = __builtin_amdgcn_readfirstlane(b0);
+      for (int k = 0; k < n; ++k) TB.units[b0 + off + k] = ((unsigned long long)ii << 32) | (unsigned)k;
+    }
+    const unsigned n = min(C->n_outside, TB.outside_cap);
+    unsigned err = 0;
+    for (long long k = i0; k < n; k += di) {
+      const long long i = (long long)TB.outside[k];
+      enumerate_particle<1>(
+          P, i, A.x[i], A.y[i], A.z[i], A.m[i], species_of(A, i),
+          [&](int g, int t, int wide, int4 e) {
+            if (g > 0) emit_direct(cursor, start, entries, C, 2 * t + wide, e);   // the base entry is binned
+          },
+          [&](int g, int, int, int) { p += g > 0 ? 1 : 0; }, err);
+    }
+  }
   p = wave_sum(p);
-  e = wave_sum(e);
-  if ((threadIdx.x & 63) == 0) { sp[threadIdx.x >> 6] = p; se[threadIdx.x >> 6] = e; }
+  mm = wave_max(mm);
+  if ((threadIdx.x & 63) == 0) { sp[threadIdx.x >> 6] = p; sm[threadIdx.x >> 6] = mm; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long tp = 0, te = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) { tp += sp[w]; te += se[w]; }
-    if (tp) atomicAdd(&C->n_pairs, tp);
-    if (te) atomicAdd(&C->n_entries, te);
+    p = sp[0] + sp[1] + sp[2] + sp[3];
+    mm = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
+    if (p) atomicAdd(&C->n_pairs, p);
+    atomicMax(&C->mmax_bits, __float_as_uint(mm) & 0x7fffffffu);   // the sign bit cleared: a -0 mass counts as 0
   }
 }
 
 long long hier_bin_blocks(long long n) { return (n + kHbChunk - 1) / kHbChunk; }
-
-hipError_t launch_cursor_reset(const unsigned long long* start, unsigned long long* cursor, long long nkeys,
-                               int cus, hipStream_t s) {
-  if (nkeys <= 0) return hipSuccess;
-  const long long want = (nkeys + 255) / 256;
-  cursor_reset<<<(int)std::min<long long>(want, (long long)cus * 16), 256, 0, s>>>(start, cursor, nkeys);
-  return hipGetLastError();
-}
 
 hipError_t launch_count_to_capacity(unsigned* cnt, long long nkeys, int cus, hipStream_t s) {
   if (nkeys <= 0) return hipSuccess;
@@ -867,22 +848,30 @@ hipError_t launch_bin_base(const Plan& P, const Parts& A, unsigned long long* cu
 
 long long emit_pieces(int chunk) { return (chunk + kEtPiece - 1) / kEtPiece; }
 
-hipError_t launch_emit_table(const Plan& P, const Parts& A, const Item* items, long long n_items, int chunk,
+hipError_t launch_after_bin(const Plan& P, const Parts& A, const BlockTables& BT, const Item* items,
+                            long long n_items, unsigned long long* cursor, const unsigned long long* start,
+                            int4* entries, Counters* C, const TableBin& TB, int cus, hipStream_t s) {
+  const long long nblk = hier_bin_blocks(A.n);
+  const long long want = (std::max(nblk, P.mode == 1 && P.nl > 0 ? n_items : 0ll) + 255) / 256;
+  const int grid = (int)std::min<long long>(std::max<long long>(want, 1), (long long)std::max(cus, 1) * 4);
+  if (P.mode == 2) after_bin<2><<<grid, 256, 0, s>>>(P, A, BT, nblk, items, n_items, cursor, start, entries, C, TB);
+  else after_bin<1><<<grid, 256, 0, s>>>(P, A, BT, nblk, items, n_items, cursor, start, entries, C, TB);
+  return hipGetLastError();
+}
+
+hipError_t launch_emit_table(const Plan& P, const Item* items, long long n_items, int chunk,
                              unsigned long long* cursor, const unsigned long long* start, int4* entries,
                              unsigned* item_pairs, Counters* C, const TableBin& TB, int cus, hipStream_t s) {
-  if (n_items > 0) {
-    static int per_cu = 0;
-    if (per_cu <= 0) {
-      int nb = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, emit_table, kEtThreads, 0) != hipSuccess || nb <= 0) nb = 4;
-      per_cu = nb;
-    }
-    list_units<<<(unsigned)((n_items + 255) / 256), 256, 0, s>>>(P, items, n_items, cursor, TB.units, C);
-    const long long most = n_items * emit_pieces(chunk);
-    const int grid = (int)std::min<long long>(most, (long long)cus * per_cu);
-    emit_table<<<grid, kEtThreads, 0, s>>>(P, items, TB.units, cursor, start, entries, item_pairs, C, TB);
+  if (n_items <= 0) return hipSuccess;
+  static int per_cu = 0;
+  if (per_cu <= 0) {
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, emit_table, kEtThreads, 0) != hipSuccess || nb <= 0) nb = 4;
+    per_cu = nb;
   }
-  emit_outside<<<std::max(cus, 1), 256, 0, s>>>(P, A, cursor, start, entries, C, TB);
+  const long long most = n_items * emit_pieces(chunk);
+  emit_table<<<(int)std::min<long long>(most, (long long)cus * per_cu), kEtThreads, 0, s>>>(
+      P, items, TB.units, cursor, start, entries, item_pairs, C, TB);
   return hipGetLastError();
 }
 
@@ -904,16 +893,6 @@ hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, 
   const int batch = (int)std::max<long long>(1, std::min<long long>(8, n / ((long long)grid * 16)));
   emit_tsc<<<grid, kEmThreads, 0, s>>>(P, items, item_lo, item_hi, level, batch, cursor, start, entries, item_pairs,
                                        C);
-  return hipGetLastError();
-}
-
-hipError_t launch_hier_stats(const unsigned* item_pairs, long long n_items, const unsigned long long* start,
-                             const unsigned long long* cursor, long long nkeys, Counters* C, int cus,
-                             hipStream_t s) {
-  const long long want = (std::max(n_items, nkeys) + 255) / 256;
-  if (want <= 0) return hipSuccess;
-  hier_stats<<<(int)std::min<long long>(want, (long long)std::max(cus, 1) * 4), 256, 0, s>>>(item_pairs, n_items, start,
-                                                                                          cursor, nkeys, C);
   return hipGetLastError();
 }
 

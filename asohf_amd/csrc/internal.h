@@ -98,7 +98,8 @@ struct Plan {
   int rad_malla;             // 1: RAD tables are exactly MALLA's recurrence (rad1 + (i-1)*radc)
   int merge_narrow;          // 1: narrow deposits may merge lanes (every non-centre weight product
                              // <= 0.45, so eight terms of a mass below 2^30 sum below 2^32)
-  int pad;
+  int per_tile;              // 1: a 27-cell member has an entry in every tile its stencil touches
+                             // (table mode, atomic: see run_batched); no exchange between tiles
   float rad1[3];
   float radc[3];
   // binning through the base grid: the patches whose members are found from
@@ -138,7 +139,9 @@ struct Counters {
   unsigned int n_wide_eff;        // wide items, which follow the narrow ones
   unsigned int n_outside;         // table mode: particles outside the box
   unsigned int n_units;           // table mode: the emission's work units
-  unsigned int pad[kLine - 15];
+  unsigned int ticket;            // workgroups of the call's last kernel that are done
+  unsigned int pad[kLine - 16];
+  unsigned long long clk[kLine / 2];   // device clock at the phase boundaries (kClk*)
   unsigned long long pool_fill[kPoolSubs * kLine / 2];   // sub-pool k at [k * kLine / 2]
   unsigned long long epool_fill[kPoolSubs * kLine / 2];  // emission lists, same layout
   unsigned int queue[kQueues * kLine];                   // queue q at [q * kLine]
@@ -148,6 +151,12 @@ struct Counters {
 
 static_assert(sizeof(unsigned long long) * 4 + sizeof(unsigned) * (kLine - 8) == kLine * 4,
               "the scalar counters fill one 128-byte line");
+// the part of the counters the host reads after a call: the scalars and the clock
+constexpr int kHostWords = 2 * kLine;
+// phase boundaries of a call binned through the base grid: its first kernel,
+// then the first kernel after the base binning, the deposit, the output cells,
+// the sums, and their end
+enum : int { kClkBegin, kClkBinned, kClkDeposit, kClkCombine, kClkSums, kClkEnd };
 
 // Work item of the persistent deposit: a chunk of one tile's entry list.
 struct Item {

@@ -477,12 +477,14 @@ __global__ void plan_count(const unsigned long long* start, int ntiles, int chun
 }
 
 __global__ void plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                           const unsigned long long* item_off, Item* items, const Counters* C) {
+                           const unsigned long long* item_off, Item* items, int* split_tiles, unsigned* n_split,
+                           const Counters* C) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ntiles || C->overflow) return;
   long long s0, s1, s2;
   int cn, cw;
   tile_chunks(start, t, chunk, chunk_wide, s0, s1, s2, cn, cw);
+  if (split_tiles && cn + cw > 1) split_tiles[atomicAdd(n_split, 1u)] = t;   // in any order
   long long k = (long long)item_off[t];
   for (int c = 0; c < cn; ++c, ++k) {
     const long long b = s0 + (long long)c * chunk;
@@ -755,6 +757,17 @@ __device__ __forceinline__ float base_centre(const Plan& P, int a, int i, int n)
   return r[i];
 }
 
+// tile-local coordinate of the centre cell of an entry in one of several tiles
+// its stencil touches: on the periodic base grid the image of the (wrapped)
+// centre that lies next to the tile
+__device__ __forceinline__ int centre_local(int c, int org, int ext, int n, bool periodic) {
+  if (!periodic) return c - org;
+  int l = wrap1(c, n) - org;
+  if (l > ext) l -= n;
+  if (l < -1) l += n;
+  return l;
+}
+
 // LDS layout of a deposit tile: cell (x, y, z), local coordinates from -1 (the
 // tile's halo) to T, at kTileFront + (x + 1) + HX * ((y + 1) + HY * (z + 2)).
 // Every entry's centre cell, clamped into its grid, lies in the tile, so a
@@ -796,6 +809,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
   __shared__ Acc acc[H];
   __shared__ unsigned s_item;
   const int tid = threadIdx.x, nthr = blockDim.x;
+  stamp(D.C, kClkDeposit);
   const float scale = (float)fixed_scale(D.C->mmax_bits);
   const unsigned n_items = D.C->n_items_eff;
   const float k0[3] = {P.ktab[P.kmax - 1], P.ktab[P.kmax], P.ktab[P.kmax + 1]};
@@ -875,9 +889,30 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
       }
       // in [-1, ext] by construction of the binning; clamped so the array
       // bounds never depend on that
-      const int lx = clampi((periodic ? wrap1(ci[0], G.n[0]) : ci[0]) - i0, -1, TX);
-      const int ly = clampi((periodic ? wrap1(ci[1], G.n[1]) : ci[1]) - j0, -1, TY);
-      const int lz = clampi((periodic ? wrap1(ci[2], G.n[2]) : ci[2]) - k0c, -1, TZ);
+      const int ext[3] = {min(TX, G.n[0] - i0 + 1), min(TY, G.n[1] - j0 + 1), min(TZ, G.n[2] - k0c + 1)};
+      const int org[3] = {i0, j0, k0c};
+      int lc[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        lc[a] = MODE == 1 && RED == 1 ? centre_local(ci[a], org[a], ext[a], G.n[a], periodic)
+                                      : (periodic ? wrap1(ci[a], G.n[a]) : ci[a]) - org[a];
+      if (MODE == 1 && RED == 1 && periodic && ok) {
+        // two tiles on an axis, the last one cell wide: a centre next to the
+        // wrap reaches the first tile on both sides, through two images
+        for (int k = 1; k < 8; ++k) {
+          int li[3];
+          bool img = true;
+          for (int a = 0; a < 3; ++a) {
+            li[a] = lc[a];
+            if (!((k >> a) & 1)) continue;
+            const bool below = lc[a] - G.n[a] >= -1;
+            li[a] += below ? -G.n[a] : G.n[a];
+            img = img && G.nt[a] > 1 && (below || li[a] <= ext[a]);
+          }
+          if (img) deposit27<RED, HX, HY>(acc + at(li[0] - 1, li[1] - 1, li[2] - 1), m, wx, wy, wz, scale);
+        }
+      }
+      const int lx = clampi(lc[0], -1, TX), ly = clampi(lc[1], -1, TY), lz = clampi(lc[2], -1, TZ);
       const int corner = at(lx - 1, ly - 1, lz - 1);
       if (MODE == 2 || P.merge_narrow)
         deposit27_merged<RED, HX, HY>(acc, corner, ok, m, wx, wy, wz, scale);
@@ -894,6 +929,23 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
       vb = at_j(o + 3 * nthr + tid);
     }
     __syncthreads();
+
+    // ---- entries in every tile they touch (P.per_tile): the halo is the other
+    // tiles' business and is cleared, after a tile spanning a whole periodic
+    // axis has folded it into its own cells (the reference's wrap) ----
+    if (MODE == 1 && RED == 1) {
+      const int ex = min(TX, G.n[0] - i0 + 1), ey = min(TY, G.n[1] - j0 + 1), ez = min(TZ, G.n[2] - k0c + 1);
+      const bool fold = periodic && (G.nt[0] == 1 || G.nt[1] == 1 || G.nt[2] == 1);
+      for (int c = tid; c < L::E; c += nthr) {
+        const int a = c % L::EX - 1, b = (c / L::EX) % L::EY - 1, cz = c / (L::EX * L::EY) - 1;
+        if (a >= 0 && a < ex && b >= 0 && b < ey && cz >= 0 && cz < ez) continue;
+        const int ga = wrap1(i0 + a, G.n[0]) - i0, gb = wrap1(j0 + b, G.n[1]) - j0, gc = wrap1(k0c + cz, G.n[2]) - k0c;
+        if (fold && ga >= 0 && ga < ex && gb >= 0 && gb < ey && gc >= 0 && gc < ez && acc[at(a, b, cz)] != 0)
+          lds_add(acc + at(ga, gb, gc), acc[at(a, b, cz)]);
+        acc[at(a, b, cz)] = 0;
+      }
+      __syncthreads();
+    }
 
     // ---- the tile and its halo to the exchange buffer: stored when the tile
     // has one item, added where several items share it (exact int64 adds, so
@@ -999,7 +1051,7 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
   constexpr int nthr = kWideThreads;
   static_assert(BX % 4 == 0 && BY % 4 == 0 && BZ % 4 == 0 && B / 4 <= nthr, "four outputs per thread and pass");
   __shared__ long long hist[kWideCells];
-  __shared__ long long acc[B];   // int64 sums (deterministic) or FP64 bits (atomic)
+  __shared__ Acc acc[B];
   __shared__ double s_k[kWideK];
   __shared__ unsigned s_item;
   __shared__ unsigned s_ccnt[kNLevels + 1];
@@ -1011,8 +1063,8 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
   const unsigned n_narrow = D.C->n_items_eff, n_wide = D.C->n_wide_eff;
   // a cell's FP64 sum into the block's accumulator (one thread per cell)
   auto put = [&](int c, double v) {
-    if (RED == 0) acc[c] += __double2ll_rn(v);
-    else reinterpret_cast<double*>(acc)[c] += v * inv_scale;
+    if (RED == 0) acc[c] += (Acc)__double2ll_rn(v);
+    else acc[c] += (Acc)(v * inv_scale);
   };
   const int q = blockIdx.x % D.n_queues;
   for (;;) {
@@ -1059,7 +1111,7 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
       const int oy = (sub % (TY / BY)) * BY, oz = (sub / (TY / BY)) * BZ;
       const int j0 = j0t + oy, k0 = k0t + oz;   // the block's first cell
       if (j0 > G.n[1] || k0 > G.n[2]) continue;  // past the grid: never read
-      for (int c = tid; c < B; c += nthr) acc[c] = 0;   // zero bits: 0 as FP64 too
+      for (int c = tid; c < B; c += nthr) acc[c] = 0;
       __syncthreads();
       for (int irk = 1; irk <= P.nl; ++irk) {
         const unsigned ncls = s_ccnt[irk];
@@ -1068,11 +1120,13 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
         const float* K = P.ktab + irk * P.kw + P.kmax;   // K[d], d in [-N, N]
         const WideShape w = wide_shape<BX, BY, BZ>(nk);
         const long long taps = 2 * nk + 1;
-        const long long box = (long long)min((int)taps, BX) * min((int)taps, BY) * min((int)taps, BZ);
+        // (atomic mode keeps the direct FP32 adds wherever it made them)
+        const long long box = RED == 0 ? (long long)min((int)taps, BX) * min((int)taps, BY) * min((int)taps, BZ)
+                                       : taps * taps * taps;
         const long long adds = w.form == 0 ? 1 : (w.form == 1 ? BZ : BY * BZ);
         const long long passes = taps * ((long long)BX * w.ny * w.nz + (w.form < 2 ? (long long)BX * BY * w.nz : 0) +
                                          (w.form < 1 ? B : 0));
-        if ((it.flags & 2) && w.form >= 0 && 4 * (long long)ncls * (box - adds) > passes) {
+        if ((it.flags & 2) && (RED == 0 ? w.form >= 0 : w.form == 0) && 4 * (long long)ncls * (box - adds) > passes) {
           // ---- the histogram
           if (tid < taps) s_k[tid] = (double)K[tid - nk];
           for (int c = tid; c < w.cells; c += nthr) hist[c] = 0;
@@ -1214,12 +1268,12 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
           const float* Kx = K + (xa - ci[0]);
           const float* Ky = K + (ya - ci[1]);
           const float* Kz = K + (za - ci[2]);
-          long long* base = acc + (xa - i0) + BX * ((ya - j0) + BY * (za - k0));
+          Acc* base = acc + (xa - i0) + BX * ((ya - j0) + BY * (za - k0));
           for (int q2 = lane; q2 < total; q2 += 64) {
             const float term = ((ms * Kx[a]) * Ky[b]) * Kz[c];
-            long long* cell = base + (a + BX * (b + BY * c));
-            if (RED == 0) lds_add(cell, (long long)__float2int_rn(term));
-            else atomicAdd(reinterpret_cast<double*>(cell), (double)term);
+            Acc* cell = base + (a + BX * (b + BY * c));
+            if (RED == 0) lds_add(reinterpret_cast<long long*>(cell), (long long)__float2int_rn(term));
+            else lds_add(reinterpret_cast<float*>(cell), term);
             a += da;
             const bool carry = a >= cx;
             if (carry) a -= cx;
@@ -1236,7 +1290,7 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
       // the block's cells to the tile's exchange cells, as the deposit's
       for (int c = tid; c < B; c += nthr) {
         Acc* cell = dst + (c % BX + 1) + L::EX * (((c / BX) % BY + oy + 1) + L::EY * (c / (BX * BY) + oz + 1));
-        const Acc v = RED == 0 ? (Acc)acc[c] : (Acc)reinterpret_cast<double*>(acc)[c];
+        const Acc v = acc[c];
         if (alone) *cell = v;
         else if (v != 0) glb_add(cell, v);
       }
@@ -1273,6 +1327,7 @@ __global__ void __launch_bounds__(256) combine_tiles(Plan P, DepArgs D) {
   __shared__ long long s_nb[27];   // first exchange cell of each neighbour, -1: none or empty
   __shared__ long long s_redi[4];
   __shared__ double s_redd[4];
+  stamp(D.C, kClkCombine);
   if (D.C->overflow) return;
   const double inv_scale = 1.0 / fixed_scale(D.C->mmax_bits);   // a power of two: exact
   const int tid = threadIdx.x;
@@ -1382,6 +1437,123 @@ __global__ void __launch_bounds__(256) grid_sums(Plan P, DepArgs D, double* grid
     s = block_sum(s, shd);
     if (threadIdx.x == 0) grid_mass[g] = s;
   }
+}
+
+// The first kernel of a call binned through the base grid: clears the
+// counters (the queue lengths to n_narrow and n_wide), the items' member
+// counts and the exchange cells of the tiles that several items add to, and
+// starts every tile's range empty.
+// One launch for what took six, and no events, memory copy or sums of their
+// own at the call's end (finish_call): a small call is bound by its launches
+// and the gaps between them.  13,824 particles 245 -> 189 us, 250,047 (kernel
+// table, graph) 247 -> 225, 2.1M (kernel table) 409 -> 352.
+__global__ void __launch_bounds__(256) begin_call(DepArgs D, unsigned n_narrow, unsigned n_wide, unsigned* item_pairs,
+                                                  long long n_items, unsigned long long* cursor, long long nkeys,
+                                                  const int* split_tiles, const unsigned* n_split, int words) {
+  const long long i0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, di = (long long)gridDim.x * blockDim.x;
+  Counters* C = D.C;
+  unsigned* c = reinterpret_cast<unsigned*>(C);
+  const long long eff = &C->n_items_eff - c, wide = &C->n_wide_eff - c;
+  const long long clk0 = reinterpret_cast<unsigned*>(C->clk) - c, clk1 = clk0 + kLine;
+  for (long long k = i0; k < (long long)(sizeof(Counters) / 4); k += di)
+    if (k < clk0 || k >= clk1) c[k] = k == eff ? n_narrow : (k == wide ? n_wide : 0u);
+  stamp(C, kClkBegin);
+  for (long long k = i0; k < n_items; k += di) item_pairs[k] = 0u;
+  for (long long k = i0; k < nkeys; k += di) cursor[k] = D.start[k];
+  const unsigned ns = *n_split;
+  for (unsigned k = blockIdx.x; k < ns; k += gridDim.x) {
+    unsigned* p = reinterpret_cast<unsigned*>(D.scratch) + (long long)split_tiles[k] * words;
+    for (int w = threadIdx.x; w < words; w += 256) p[w] = 0u;
+  }
+}
+
+// The last kernel of such a call: every grid's mass in a fixed order (a wave
+// per grid; a workgroup where the grid has many tiles), the call's members
+// (what the emission's items found; base members are in the counters already)
+// and entries (the filled part of every tile's range), and, by the last
+// workgroup to end, the counters written to the host.
+template <int RED>
+__global__ void __launch_bounds__(256) finish_call(Plan P, DepArgs D, double* grid_mass, const unsigned* item_pairs,
+                                                   long long n_items, long long nkeys, unsigned* host) {
+  __shared__ long long shi[4];
+  __shared__ double shd[4];
+  __shared__ unsigned long long sp[4], se[4];
+  __shared__ unsigned s_last;
+  constexpr int kWaveTiles = 1024;   // tiles up to which a wave sums a grid
+  Counters* C = D.C;
+  stamp(C, kClkSums);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const double scale = fixed_scale(C->mmax_bits);
+  auto tiles = [&](int g) {
+    const GridDesc& G = P.grids[g];
+    return G.level == 0 && g != 0 ? 0 : G.nt[0] * G.nt[1] * G.nt[2];
+  };
+  if (grid_mass) {
+    for (int g = blockIdx.x * 4 + (tid >> 6); g < P.ngrids; g += gridDim.x * 4) {
+      const int nt = tiles(g), t0 = P.grids[g].tile0;
+      if (nt > kWaveTiles) continue;
+      if (RED == 0) {
+        long long s = 0;
+        for (int k = lane; k < nt; k += 64) s += D.tile_mass_i[t0 + k];
+        s = wave_sum(s);
+        if (lane == 0) grid_mass[g] = (double)s / scale;
+      } else {
+        double s = 0;
+        for (int k = lane; k < nt; k += 64) s += D.tile_mass_d[t0 + k];
+        s = wave_sum(s);
+        if (lane == 0) grid_mass[g] = s;
+      }
+    }
+    for (int g = blockIdx.x; g < P.ngrids; g += gridDim.x) {
+      const int nt = tiles(g), t0 = P.grids[g].tile0;
+      if (nt <= kWaveTiles) continue;
+      long long si[8] = {};
+      double sd[8] = {};
+      for (int k0 = tid; k0 < nt; k0 += 8 * 256) {   // eight loads in flight
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int k = k0 + r * 256;
+          if (k < nt) {
+            if (RED == 0) si[r] += D.tile_mass_i[t0 + k];
+            else sd[r] += D.tile_mass_d[t0 + k];
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 1; r < 8; ++r) { si[0] += si[r]; sd[0] += sd[r]; }
+      if (RED == 0) {
+        const long long s = block_sum(si[0], shi);
+        if (tid == 0) grid_mass[g] = (double)s / scale;
+      } else {
+        const double s = block_sum(sd[0], shd);
+        if (tid == 0) grid_mass[g] = s;
+      }
+    }
+  }
+  unsigned long long p = 0, e = 0;
+  const long long i0 = blockIdx.x * (long long)blockDim.x + tid, di = (long long)gridDim.x * blockDim.x;
+  for (long long i = i0; i < n_items; i += di) p += item_pairs[i];
+  for (long long k = i0; k < nkeys; k += di) e += D.cursor[k] - D.start[k];
+  p = wave_sum(p);
+  e = wave_sum(e);
+  if (lane == 0) { sp[tid >> 6] = p; se[tid >> 6] = e; }
+  __syncthreads();
+  if (tid == 0) {
+    p = sp[0] + sp[1] + sp[2] + sp[3];
+    e = se[0] + se[1] + se[2] + se[3];
+    if (p) atomicAdd(&C->n_pairs, p);
+    if (e) atomicAdd(&C->n_entries, e);
+    __threadfence();
+    s_last = atomicAdd(&C->ticket, 1u) == gridDim.x - 1 ? 1u : 0u;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  if (tid == 0) C->clk[kClkEnd] = wall_clock64();
+  __syncthreads();
+  __threadfence();
+  if (tid < kHostWords)
+    host[tid] = __hip_atomic_load(reinterpret_cast<unsigned*>(C) + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __threadfence_system();
 }
 
 // ---------------------------------------------------------------------------
@@ -1814,8 +1986,10 @@ hipError_t launch_plan_count(const unsigned long long* start, int ntiles, int ch
 }
 
 hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                             const unsigned long long* item_off, Item* items, const Counters* C, hipStream_t s) {
-  plan_write<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, item_off, items, C);
+                             const unsigned long long* item_off, Item* items, int* split_tiles, unsigned* n_split,
+                             const Counters* C, hipStream_t s) {
+  plan_write<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, item_off, items,
+                                                           split_tiles, n_split, C);
   return hipGetLastError();
 }
 
@@ -1893,6 +2067,26 @@ hipError_t launch_grid_sums(const Plan& P, const DepArgs& D, int reduction, doub
   if (P.ngrids <= 0) return hipSuccess;
   if (reduction == 0) grid_sums<0><<<P.ngrids, 256, 0, s>>>(P, D, grid_mass);
   else grid_sums<1><<<P.ngrids, 256, 0, s>>>(P, D, grid_mass);
+  return hipGetLastError();
+}
+
+hipError_t launch_begin_call(const DepArgs& D, const int tile[3], int reduction, long long n_narrow, long long n_wide,
+                             unsigned* item_pairs, long long n_items, unsigned long long* cursor, long long nkeys,
+                             const int* split_tiles, const unsigned* n_split, int cus, hipStream_t s) {
+  const int words = (int)exchange_cells(tile) * (reduction == 0 ? 2 : 1);
+  const long long want = (std::max(std::max(n_items, nkeys), (long long)(sizeof(Counters) / 4)) + 255) / 256;
+  begin_call<<<(int)std::min<long long>(std::max<long long>(want, 64), (long long)std::max(cus, 1) * 8), 256, 0, s>>>(
+      D, (unsigned)n_narrow, (unsigned)n_wide, item_pairs, n_items, cursor, nkeys, split_tiles, n_split, words);
+  return hipGetLastError();
+}
+
+hipError_t launch_finish_call(const Plan& P, const DepArgs& D, int reduction, double* grid_mass,
+                              const unsigned* item_pairs, long long n_items, long long nkeys, unsigned* host, int cus,
+                              hipStream_t s) {
+  const long long want = std::max((std::max(n_items, nkeys) + 1023) / 1024, grid_mass ? (P.ngrids + 3ll) / 4 : 1ll);
+  const int grid = (int)std::min<long long>(std::max<long long>(want, 1), (long long)std::max(cus, 1) * 4);
+  if (reduction == 0) finish_call<0><<<grid, 256, 0, s>>>(P, D, grid_mass, item_pairs, n_items, nkeys, host);
+  else finish_call<1><<<grid, 256, 0, s>>>(P, D, grid_mass, item_pairs, n_items, nkeys, host);
   return hipGetLastError();
 }
 

@@ -27,7 +27,8 @@ hipError_t launch_reduce_blocks(const BlockTables& BT, long long nblk, Counters*
 hipError_t launch_plan_count(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
                              unsigned* cnt, unsigned* nitems_tile, hipStream_t s);
 hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
-                             const unsigned long long* item_off, Item* items, const Counters* C, hipStream_t s);
+                             const unsigned long long* item_off, Item* items, int* split_tiles, unsigned* n_split,
+                             const Counters* C, hipStream_t s);
 hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* item_off, int ntiles,
                        unsigned long long cap_entries, unsigned long long cap_items, Counters* C, hipStream_t s);
 bool tile_shape_supported(const int t[3]);
@@ -40,22 +41,27 @@ long long exchange_cells(const int tile[3]);
 hipError_t launch_combine(const Plan& P, const DepArgs& D, int reduction, int cus, hipStream_t s);
 hipError_t launch_grid_sums(const Plan& P, const DepArgs& D, int reduction, double* grid_mass, hipStream_t s);
 // binning through the base grid (hier.hip)
-hipError_t launch_cursor_reset(const unsigned long long* start, unsigned long long* cursor, long long nkeys,
-                               int cus, hipStream_t s);
 hipError_t launch_count_to_capacity(unsigned* cnt, long long nkeys, int cus, hipStream_t s);
 hipError_t launch_bin_base(const Plan& P, const Parts& A, unsigned long long* cursor,
                            const unsigned long long* start, int4* entries, Counters* C, const BlockTables& BT,
                            const TableBin& TB, int cus, hipStream_t s);
+hipError_t launch_after_bin(const Plan& P, const Parts& A, const BlockTables& BT, const Item* items,
+                            long long n_items, unsigned long long* cursor, const unsigned long long* start,
+                            int4* entries, Counters* C, const TableBin& TB, int cus, hipStream_t s);
 long long emit_pieces(int chunk);   // emission work units of an item of `chunk` entries
-hipError_t launch_emit_table(const Plan& P, const Parts& A, const Item* items, long long n_items, int chunk,
+hipError_t launch_emit_table(const Plan& P, const Item* items, long long n_items, int chunk,
                              unsigned long long* cursor, const unsigned long long* start, int4* entries,
                              unsigned* item_pairs, Counters* C, const TableBin& TB, int cus, hipStream_t s);
 hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, long long item_hi, int level,
                            unsigned long long* cursor, const unsigned long long* start, int4* entries,
                            unsigned* item_pairs, Counters* C, int cus, hipStream_t s);
-hipError_t launch_hier_stats(const unsigned* item_pairs, long long n_items, const unsigned long long* start,
-                             const unsigned long long* cursor, long long nkeys, Counters* C, int cus,
-                             hipStream_t s);
+// the first and the last kernel of a call binned through the base grid
+hipError_t launch_begin_call(const DepArgs& D, const int tile[3], int reduction, long long n_narrow, long long n_wide,
+                             unsigned* item_pairs, long long n_items, unsigned long long* cursor, long long nkeys,
+                             const int* split_tiles, const unsigned* n_split, int cus, hipStream_t s);
+hipError_t launch_finish_call(const Plan& P, const DepArgs& D, int reduction, double* grid_mass,
+                              const unsigned* item_pairs, long long n_items, long long nkeys, unsigned* host, int cus,
+                              hipStream_t s);
 hipError_t launch_adjoint(const Plan& P, const Parts& A, const float* g1, const float* g11, float* dm,
                           float* dx, float* dy, float* dz, const unsigned* order, int cus, hipStream_t s);
 hipError_t launch_cell_keys(const Plan& P, const Parts& A, unsigned* key, unsigned* idx, Counters* C, int cus,

@@ -82,3 +82,29 @@ def test_spilled_stencils_reach_their_cells(nx, sides, mode):
                     assert all(np.array_equal(u, v) for u, v in zip(got, first)), (tile, chunk)
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("mode", ["tsc", "table"])
+@pytest.mark.parametrize("nx,sides", CASES)
+def test_atomic_sums_reach_the_same_cells(nx, sides, mode):
+    """Atomic mode sums FP32 terms: table mode then keeps an entry in every tile
+    a stencil touches (two images of one tile where the last tile of a
+    two-tile axis is one cell wide)."""
+    import torch
+
+    from asohf_amd.density import DensityBuilder
+    snap = snapshot(nx, sides)
+    d = O.density64(snap, "A" if mode == "table" else "B")
+    rtol = (9 + snap.n) * 2.0 ** -24   # n FP32 sums
+    t = [torch.from_numpy(a).to("cuda:0") for a in (snap.x, snap.y, snap.z, snap.m)]
+    b = DensityBuilder(0)
+    try:
+        for tile in TILES:
+            b.set_tune(tile=tile)
+            r = b.density(snap.geom, *t, snap.npart_esp, mode=mode, reduction="atomic")
+            got = [r.u1.cpu().numpy(), r.u11[:int(snap.geom.patch_cells().sum())].cpu().numpy()]
+            for u, ref in [(u, ref) for u, ref in zip(got, d) if ref.size and u.size]:
+                # atol: the FP32 weights of a far corner cell keep few digits (1.5 - b cancels)
+                assert np.all(np.abs(u.ravel() - ref.ravel()) <= 2.0 ** -20 * ref.max() + rtol * ref.ravel()), tile
+    finally:
+        b.close()
