@@ -879,11 +879,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
         }
       } else {
         int irk;
-        if (D.cursor && g == 0)
-          unpack_table(table_base_entry(P, __int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z),
-                                        __int_as_float(v.w)), ci[0], ci[1], ci[2], irk, m);
-        else
-          unpack_table(v, ci[0], ci[1], ci[2], irk, m);
+        unpack_table(v, ci[0], ci[1], ci[2], irk, m);
 #pragma unroll
         for (int k = 0; k < 3; ++k) { wx[k] = k0[k]; wy[k] = k0[k]; wz[k] = k0[k]; }
       }
@@ -963,6 +959,124 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
   }
 }
 
+// Deterministic table mode's narrow entries (N = 1).  Every entry's 27 terms
+// are the kernel row's weights times its mass, rounded to the fixed-point unit,
+// and most snapshots hold one mass: the entries of the item's first mass are
+// counted at their centre cells, one LDS add per entry instead of 27, and the
+// cells' sums are counts times the 8 distinct terms (per axis an outer or the
+// centre weight; the centre keeps Q(m) minus the other 26).  Entries of another
+// mass deposit their 27 terms one by one.  Both are the sums of the same
+// integers, so the result depends on neither the item's first entry nor how
+// entries fall into items.
+// Bound by reading the entries and the 27 counts per cell.  Against 27 LDS adds
+// per entry with neighbouring lanes merged: 16.8M particles, 4 levels 762 ->
+// 371 us; 134M particles, 6 levels 6.2 -> 1.9 ms; 2.1M, 3 levels 111 -> 45 us.
+template <int TX, int TY, int TZ>
+__global__ void __launch_bounds__(1024) deposit_counts(Plan P, DepArgs D) {
+  using L = TileLds<TX, TY, TZ>;
+  // counts at local cells -1..T of the tile, with a ring of zeros around them
+  constexpr int CX = TX + 4, CY = TY + 4, CZ = TZ + 4;
+  __shared__ long long acc[L::H];
+  __shared__ unsigned cnt[CX * CY * CZ];
+  __shared__ unsigned s_item;
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  stamp(D.C, kClkDeposit);
+  const float scale = (float)fixed_scale(D.C->mmax_bits);
+  const unsigned n_items = D.C->n_items_eff;
+  const float k0[3] = {P.ktab[P.kmax - 1], P.ktab[P.kmax], P.ktab[P.kmax + 1]};
+  const int q = blockIdx.x % D.n_queues;
+  for (;;) {
+    if (tid == 0) s_item = atomicAdd(&D.C->queue[q * kLine], 1u) * D.n_queues + q;
+    __syncthreads();
+    const unsigned idx = __builtin_amdgcn_readfirstlane(s_item);
+    if (idx >= n_items) break;
+    const Item it = D.items[idx];
+    const int t = __builtin_amdgcn_readfirstlane(it.tile);
+    const int g = __builtin_amdgcn_readfirstlane(P.tile_grid[t]);
+    const GridDesc& G = P.grids[g];
+    const int n[3] = {G.n[0], G.n[1], G.n[2]}, nt0 = G.nt[0], nt1 = G.nt[1];
+    const int local = t - G.tile0;
+    const int org[3] = {(local % nt0) * TX + 1, ((local / nt0) % nt1) * TY + 1, (local / (nt0 * nt1)) * TZ + 1};
+    long long len = it.end - it.begin;
+    if (D.cursor) len = min(it.end, (long long)D.cursor[2 * t]) - it.begin;
+    len = uniform64(len);
+    if (len <= 0) {
+      __syncthreads();   // every wave has read s_item before thread 0 takes the next item
+      continue;
+    }
+    const int4* const eb = D.entries + uniform64(it.begin);
+    const bool positions = D.cursor && g == 0;
+    const int m_bits = __builtin_amdgcn_readfirstlane(positions ? eb[0].w : eb[0].z);   // the item's first mass
+    for (int c = tid; c < L::H; c += nthr) acc[c] = 0;
+    for (int c = tid; c < CX * CY * CZ; c += nthr) cnt[c] = 0u;
+    __syncthreads();
+    bool others = false;   // the wave met another mass
+    for (long long o = 0; o < len; o += 4 * nthr) {   // four loads in flight
+      int4 v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = eb[min(o + r * nthr + tid, len - 1)];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool ok = o + r * nthr + tid < len;
+        int ci[3], irk;
+        float m;
+        const int4 e = positions ? table_base_entry(P, __int_as_float(v[r].x), __int_as_float(v[r].y),
+                                                    __int_as_float(v[r].z), __int_as_float(v[r].w))
+                                 : v[r];
+        unpack_table(e, ci[0], ci[1], ci[2], irk, m);
+        int lc[3];
+        constexpr int T[3] = {TX, TY, TZ};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) lc[a] = clampi((g == 0 ? wrap1(ci[a], n[a]) : ci[a]) - org[a], -1, T[a]);
+        const bool same = __float_as_int(m) == m_bits;
+        if (ok && same) {
+          atomicAdd(&cnt[(lc[0] + 2) + CX * ((lc[1] + 2) + CY * (lc[2] + 2))], 1u);
+        } else if (ok) {
+          others = true;
+          deposit27<0, L::HX, L::HY>(acc + L::at(lc[0] - 1, lc[1] - 1, lc[2] - 1), m, k0, k0, k0, scale);
+        }
+      }
+    }
+    const bool any_other = __syncthreads_or(others);
+    // the terms of the first mass, as deposit27 forms them: index bit a set
+    // where the cell is the centre's neighbour along axis a
+    unsigned term[8];
+    {
+      const float ms = __int_as_float(m_bits) * scale;
+      unsigned rest = 0;
+#pragma unroll
+      for (int k = 1; k < 8; ++k) {
+        term[k] = term_u32((ms * k0[k & 1 ? 0 : 1]) * k0[k & 2 ? 0 : 1], k0[k & 4 ? 0 : 1]);
+        rest += term[k] << __popc(k);   // 2, 4 or 8 cells
+      }
+      term[0] = rest;   // what the centre gives away
+    }
+    const unsigned whole = __float2uint_rn(__int_as_float(m_bits) * scale);
+    const long long centre = (long long)whole - (long long)term[0];
+    long long* dst = reinterpret_cast<long long*>(D.scratch) + (long long)t * L::E;
+    const bool alone = D.nitems_tile[t] == 1;
+    for (int c = tid; c < L::E; c += nthr) {
+      // counts around exchange cell c, from the corner (-1, -1, -1)
+      const unsigned* N = cnt + c % L::EX + CX * ((c / L::EX) % L::EY + CY * (c / (L::EX * L::EY)));
+      unsigned sum[8] = {};
+#pragma unroll
+      for (int z = 0; z < 3; ++z)
+#pragma unroll
+        for (int y = 0; y < 3; ++y)
+#pragma unroll
+          for (int x = 0; x < 3; ++x)
+            sum[(x != 1 ? 1 : 0) + (y != 1 ? 2 : 0) + (z != 1 ? 4 : 0)] += N[x + CX * (y + CY * z)];
+      long long v = any_other ? acc[L::of_exchange(c)] : 0ll;
+      v += (long long)sum[0] * centre;
+#pragma unroll
+      for (int k = 1; k < 8; ++k) v += (long long)((unsigned long long)sum[k] * term[k]);
+      if (alone) dst[c] = v;
+      else if (v != 0) glb_add(dst + c, v);
+    }
+    __syncthreads();
+  }
+}
+
 // ---------------------------------------------------------------------------
 // wide table-mode entries (kernel level irk >= 1, half-width N = 2^irk)
 // ---------------------------------------------------------------------------
@@ -1000,31 +1114,31 @@ __host__ __device__ __forceinline__ WideShape wide_shape(int nk) {
 }
 
 // Four outputs o..o+3 of a kernel row of half-width nk applied to a line of
-// stride st: s[i] = sum_j line[i + j] K[j - nk], j ascending.
+// stride st: s[i] = sum_j line[i + j] K[j - nk], j from 2 nk down to 0.
 __device__ __forceinline__ void conv4(const double* line, int st, int nk, const double* K, double s[4]) {
-  double a = line[0], b = line[st], c = line[2 * st], d = line[3 * st];
-  const double* p = line + 4 * st;
+  const double* p = line + 2 * nk * st;
+  double a = p[0], b = p[st], c = p[2 * st], d = p[3 * st];
   s[0] = s[1] = s[2] = s[3] = 0.0;
   auto tap = [&](double k, double w, double x, double y, double z) {
-    s[0] = __fma_rn(w, k, s[0]);
-    s[1] = __fma_rn(x, k, s[1]);
-    s[2] = __fma_rn(y, k, s[2]);
-    s[3] = __fma_rn(z, k, s[3]);
+    s[0] += w * k;
+    s[1] += x * k;
+    s[2] += y * k;
+    s[3] += z * k;
   };
   // 2 nk + 1 taps, nk even: four at a time, the window's registers in rotation
 #pragma unroll 1
-  for (int j = 0; j < 2 * nk; j += 4) {
+  for (int j = 2 * nk; j > 0; j -= 4) {
     tap(K[j], a, b, c, d);
-    a = p[0];
-    tap(K[j + 1], b, c, d, a);
-    b = p[st];
-    tap(K[j + 2], c, d, a, b);
-    c = p[2 * st];
-    tap(K[j + 3], d, a, b, c);
-    d = p[3 * st];
-    p += 4 * st;
+    d = p[-st];
+    tap(K[j - 1], d, a, b, c);
+    c = p[-2 * st];
+    tap(K[j - 2], c, d, a, b);
+    b = p[-3 * st];
+    tap(K[j - 3], b, c, d, a);
+    a = p[-4 * st];
+    p -= 4 * st;
   }
-  tap(K[2 * nk], a, b, c, d);
+  tap(K[0], a, b, c, d);
 }
 
 // The wide items, persistent over 8 queues like the deposit.  A tile is taken
@@ -1039,8 +1153,8 @@ __device__ __forceinline__ void conv4(const double* line, int st, int nk, const 
 // Bound by reading the entries once per class and by the LDS reads of the
 // convolution.  As part of the narrow kernel the histogram had one layout, so
 // N = 8 and more walked every entry's box (29 G adds at 512^3, 6 levels), and
-// its LDS left one narrow workgroup per CU: 113 ms, now 10.8 here and 6.2 ms
-// in the narrow kernel; 256^3, 4 levels 1,094 -> 68 + 762 us.  256 threads or
+// its LDS left one narrow workgroup per CU: 113 ms, now 12.2 here and 1.9 ms
+// in the narrow kernel; 256^3, 4 levels 1,094 -> 85 + 371 us.  256 threads or
 // a 41 KB histogram (three workgroups per CU) were slower: 19.2 and 17.5 ms
 // when this took 14.7.
 template <int RED, int TX, int TY, int TZ>
@@ -1120,13 +1234,24 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
         const float* K = P.ktab + irk * P.kw + P.kmax;   // K[d], d in [-N, N]
         const WideShape w = wide_shape<BX, BY, BZ>(nk);
         const long long taps = 2 * nk + 1;
-        // (atomic mode keeps the direct FP32 adds wherever it made them)
-        const long long box = RED == 0 ? (long long)min((int)taps, BX) * min((int)taps, BY) * min((int)taps, BZ)
-                                       : taps * taps * taps;
-        const long long adds = w.form == 0 ? 1 : (w.form == 1 ? BZ : BY * BZ);
-        const long long passes = taps * ((long long)BX * w.ny * w.nz + (w.form < 2 ? (long long)BX * BY * w.nz : 0) +
-                                         (w.form < 1 ? B : 0));
-        if ((it.flags & 2) && (RED == 0 ? w.form >= 0 : w.form == 0) && 4 * (long long)ncls * (box - adds) > passes) {
+        // The histogram of masses (form 0) when its passes cost less than the
+        // entries' direct adds.  The other forms trade the direct adds for 8 or
+        // 64 of their own and give the cells another rounding, so a class takes
+        // them from four times its passes' cost on (N = 8: 69 entries of a
+        // 16 x 8 x 8 tile; with one, two, four and eight times this kernel takes
+        // 10.8, 11.4, 12.2 and 15.2 ms at 512^3, 6 levels, and 113 without
+        // these forms, the narrow entries included).
+        bool use = false;
+        if (w.form == 0) {
+          const long long bx = TX + 2 * nk, by = TY + 2 * nk, bz = TZ + 2 * nk;
+          use = 4 * (long long)ncls * taps * taps * taps > taps * (bx * by * TX + TX * bz * TY + TX * TY * TZ);
+        } else if (w.form > 0 && RED == 0) {   // (atomic mode keeps its direct FP32 adds)
+          const long long box = (long long)min((int)taps, BX) * min((int)taps, BY) * min((int)taps, BZ);
+          const long long adds = w.form == 1 ? BZ : BY * BZ;
+          const long long passes = taps * ((long long)BX * w.ny * w.nz + (w.form < 2 ? (long long)BX * BY * w.nz : 0));
+          use = 4 * (long long)ncls * (box - adds) > 4 * passes;
+        }
+        if ((it.flags & 2) && use) {
           // ---- the histogram
           if (tid < taps) s_k[tid] = (double)K[tid - nk];
           for (int c = tid; c < w.cells; c += nthr) hist[c] = 0;
@@ -1999,15 +2124,13 @@ hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned lon
   return hipGetLastError();
 }
 
-template <int MODE, int RED>
-static hipError_t dep_shape(const Plan& P, const DepArgs& D, int grid, int block, hipStream_t s) {
-  const int* t = P.tile;
-  if (t[0] == 8 && t[1] == 8 && t[2] == 8) deposit_kernel<MODE, RED, 8, 8, 8><<<grid, block, 0, s>>>(P, D);
-  else if (t[0] == 16 && t[1] == 8 && t[2] == 8) deposit_kernel<MODE, RED, 16, 8, 8><<<grid, block, 0, s>>>(P, D);
-  else if (t[0] == 16 && t[1] == 16 && t[2] == 8) deposit_kernel<MODE, RED, 16, 16, 8><<<grid, block, 0, s>>>(P, D);
-  else if (t[0] == 16 && t[1] == 16 && t[2] == 16) deposit_kernel<MODE, RED, 16, 16, 16><<<grid, block, 0, s>>>(P, D);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+// the narrow items' kernel on tiles of TX x TY x TZ cells
+template <int TX, int TY, int TZ>
+static void narrow_tile(const Plan& P, const DepArgs& D, int red, int grid, int block, hipStream_t s) {
+  if (P.mode == 1 && red == 0) deposit_counts<TX, TY, TZ><<<grid, block, 0, s>>>(P, D);
+  else if (P.mode == 1) deposit_kernel<1, 1, TX, TY, TZ><<<grid, block, 0, s>>>(P, D);
+  else if (red == 0) deposit_kernel<2, 0, TX, TY, TZ><<<grid, block, 0, s>>>(P, D);
+  else deposit_kernel<2, 1, TX, TY, TZ><<<grid, block, 0, s>>>(P, D);
 }
 
 template <int RED>
@@ -2059,8 +2182,13 @@ hipError_t launch_combine(const Plan& P, const DepArgs& D, int reduction, int cu
 }
 
 hipError_t launch_deposit(const Plan& P, const DepArgs& D, int reduction, int grid, int block, hipStream_t s) {
-  if (P.mode == 2) return reduction == 0 ? dep_shape<2, 0>(P, D, grid, block, s) : dep_shape<2, 1>(P, D, grid, block, s);
-  return reduction == 0 ? dep_shape<1, 0>(P, D, grid, block, s) : dep_shape<1, 1>(P, D, grid, block, s);
+  const int* t = P.tile;
+  if (t[0] == 8 && t[1] == 8 && t[2] == 8) narrow_tile<8, 8, 8>(P, D, reduction, grid, block, s);
+  else if (t[0] == 16 && t[1] == 8 && t[2] == 8) narrow_tile<16, 8, 8>(P, D, reduction, grid, block, s);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 8) narrow_tile<16, 16, 8>(P, D, reduction, grid, block, s);
+  else if (t[0] == 16 && t[1] == 16 && t[2] == 16) narrow_tile<16, 16, 16>(P, D, reduction, grid, block, s);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
 }
 
 hipError_t launch_grid_sums(const Plan& P, const DepArgs& D, int reduction, double* grid_mass, hipStream_t s) {

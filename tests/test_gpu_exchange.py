@@ -108,3 +108,35 @@ def test_atomic_sums_reach_the_same_cells(nx, sides, mode):
                 assert np.all(np.abs(u.ravel() - ref.ravel()) <= 2.0 ** -20 * ref.max() + rtol * ref.ravel()), tile
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("masses", [(1.0,), (1.0, 0.25), (3e-7, 1.0, 0.1, 0.7)])
+def test_counted_masses_equal_single_deposits(masses):
+    """Table mode counts the entries of an item's first mass per cell and
+    deposits the others one by one: the same integers whichever mass comes
+    first, so the fields do not depend on the particle order or the item size,
+    and the base grid keeps the quantised mass exactly."""
+    import torch
+
+    from asohf_amd.density import DensityBuilder
+    snap = snapshot(17, ((18, 16, 8), (7, 1, 33)))
+    rng = np.random.default_rng(len(masses))
+    m = rng.choice(np.array(masses, np.float32), snap.n)
+    half = int(snap.npart_esp[0])
+    q = np.rint(m.astype(np.float64) * 2.0 ** (30 - int(np.frexp(np.float32(m.max()))[1])))
+    b = DensityBuilder(0)
+    first = None
+    try:
+        for k in range(3):
+            # another order within each species block
+            o = np.concatenate([rng.permutation(half), half + rng.permutation(snap.n - half)]) if k else np.arange(snap.n)
+            t = [torch.from_numpy(a[o]).to("cuda:0") for a in (snap.x, snap.y, snap.z, m)]
+            for chunk in (64, 4096):
+                b.set_tune(chunk=chunk)
+                r = b.density(snap.geom, *t, snap.npart_esp, mode="table")
+                got = [v.cpu().numpy() for v in (r.u1, r.u11, r.grid_mass)]
+                assert got[2][0] == q.sum() / 2.0 ** (30 - int(np.frexp(np.float32(m.max()))[1]))
+                first = first or got
+                assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1])
+    finally:
+        b.close()
