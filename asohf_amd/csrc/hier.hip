@@ -467,23 +467,20 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
 // ---------------------------------------------------------------------------
 constexpr int kEtThreads = 256;
 constexpr int kEtPiece = 1024;     // entries of a work unit (a collected member keeps 10 bits of it)
+constexpr int kEtRows = kEtPiece / kEtThreads;   // rows of 64 entries per wave
 constexpr int kEtTargets = 32;     // target records staged in LDS at once
 constexpr int kEtCap = 1024;       // LDS key slots
 constexpr int kEtWList = 128;      // emissions a wave lists before it works through them
 constexpr int kEtPend = 128;       // members a wave collects before it works through them
 constexpr unsigned long long kEtFull = ~0ull;   // a key's reservation past its capacity
 
-// A target patch in LDS: its strict membership box, its first cell's corner,
-// its sides, the largest cell side (with 1/64 of slack) and its ratio to the x
-// side for the tests; the cell and tile fields for the members.
+// A target patch in LDS, for its members: the cell and tile fields (padded so
+// that the records of several targets start in different banks).
 struct EtTarget {
-  float lo[3], hi[3], org[3], nd[3];
-  float dl, ratio;
-  int level, tile0;
-  float d[3], inv_d[3];
-  int n[3], nt0, nt1, pad[5];
+  float org[3], d[3], inv_d[3];
+  int n[3], level, tile0, nt0, nt1, pad[4];
 };
-static_assert(sizeof(EtTarget) == 128, "four 16-byte LDS reads for the tests");
+static_assert(sizeof(EtTarget) == 80, "16-byte LDS reads");
 
 // slot of key k in the table, -1 when it is not there (slot_insert found its
 // probe path full)
@@ -498,6 +495,15 @@ __device__ __forceinline__ int slot_find(const int* keys, int k) {
     h = (h + 1) & (CAP - 1);
   }
   return -1;
+}
+
+__device__ __forceinline__ float readlanef(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ unsigned long long readlane64(unsigned long long v, int lane) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), lane);
+  return ((unsigned long long)hi << 32) | lo;
 }
 
 // exclusive prefix over the wave's lanes of v >= 0, and the total
@@ -515,28 +521,34 @@ __device__ __forceinline__ int wave_exclusive(int v, int& total) {
 // The kernel-table members of every patch from the base-grid entries.  A work
 // unit is kEtPiece entries of a base tile's work item; workgroups take units
 // from the list in turn, the next one's number on its way while this one is
-// worked through; up to kEtTargets target patches at a time are staged
-// in LDS and worked through in two passes over the unit's entries:
-//   count  every wave tests its 64 entries against each target (the
-//          reference's strict box, counted as members), keeps as a bit mask
-//          those whose 2N+1 cells can meet the patch (the distance to the patch
-//          against N cells) and adds up their emissions per tile key in the
+// worked through; up to kEtTargets target patches at a time are worked through
+// in three steps over the unit's entries:
+//   test   every wave holds its kEtRows rows of entries in registers, and the
+//          targets' boxes one per lane: a target's box is read from its lane
+//          into scalars once for all rows.  Members are counted (the
+//          reference's strict box); those whose 2N+1 cells can meet the patch
+//          (the distance to the patch against N cells) are kept as a bit mask
+//   count  the emissions of the masks' members are added up per tile key in the
 //          LDS table: one for the tile of the centre cell where N = 1, one per
 //          tile the clipped box touches otherwise
 //   write  after one global add per key reserved the unit's ranges, the same
-//          members again from the masks, every emission written at the next
-//          slot of its key's range
-// Both passes collect members over the wave's entries and work through 64 at a
-// time, one per lane (their entries read again), and spread the emissions of
+//          members again, every emission written at the next slot of its key's
+//          range
+// The last two collect members over the wave's entries and work through 64 at
+// a time, one per lane (their entries read again), and spread the emissions of
 // wide members densely over the lanes.
-// Bound by VALU work (9.4 G instructions at 512^3: 54 targets per entry on
-// average, 4.1 members, 1.8 tiles each).  The count and scatter passes over
-// the patch hash this replaces, and what it takes with bin_base<1>: 512^3, 6
-// levels 70.1 -> 23.3 ms; 256^3, 4 levels 2,235 -> 1,206 us; 128^3, 3 levels
-// 175 -> 127 us.  One pass that listed the emissions for a reservation per
+// Bound by VALU work (54 targets per entry at 512^3, 4.1 members, 1.8 tiles
+// each).  With the boxes read from LDS for every row, and the tests inside the
+// count: 512^3, 6 levels 20.7 -> 16.7 ms (2.2 of them the box tests); 256^3, 4
+// levels 788 -> 640 us; 128^3, 3 levels 69 us either way.  Five workgroups per
+// CU spill 48 bytes a lane; with four and no spill 18.8 ms, 684 and 78 us, with
+// six 16.0 ms, 676 and 78 us.  The count and scatter passes over the patch hash
+// that this replaced, against this and bin_base<1>: 70.1 -> 19.2 ms; 2,235 ->
+// 1,040 us; 175 -> 127 us.  A slot per tile of the staged targets instead of
+// the hash table took 36 ms: the tiles of a few targets fill the slots.  One pass that listed the emissions for a reservation per
 // round of 256 entries took 35.6 ms, and 97 ms with lists short enough for six
 // workgroups per CU: what overflowed them reserved one by one.
-__global__ void __launch_bounds__(kEtThreads) emit_table(Plan P, const Item* items, const unsigned long long* units,
+__global__ void __launch_bounds__(kEtThreads, 5) emit_table(Plan P, const Item* items, const unsigned long long* units,
                                                          unsigned long long* cursor, const unsigned long long* start,
                                                          int4* entries, unsigned* item_pairs, Counters* C,
                                                          TableBin TB) {
@@ -570,26 +582,77 @@ __global__ void __launch_bounds__(kEtThreads) emit_table(Plan P, const Item* ite
     for (unsigned q = q0; q < q1; q += kEtTargets) {
       const int nq = (int)min((unsigned)kEtTargets, q1 - q);
       for (int k = tid; k < kEtCap; k += kEtThreads) { keys[k] = -1; slots[k] = 0ull; }
-      if (tid < nq) {
-        const BoxRec& R = P.grec[P.tgt[q + tid]];
-        EtTarget& T = targets[tid];
+      {
+        // every wave holds the targets' boxes, one per lane, and tests its rows
+        // of entries against one target at a time
+        const BoxRec& R = P.grec[P.tgt[q + min(lane, nq - 1)]];
         const float dm = fmaxf(R.d[0], fmaxf(R.d[1], R.d[2]));
+        float blo[3], bhi[3], borg[3], bnd[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-          T.lo[a] = R.lo[a];
-          T.hi[a] = R.hi[a];
-          T.org[a] = R.org[a];
-          T.nd[a] = (float)R.n[a] * R.d[a];
-          T.d[a] = R.d[a];
-          T.inv_d[a] = R.inv_d[a];
-          T.n[a] = R.n[a];
+          blo[a] = R.lo[a];
+          bhi[a] = R.hi[a];
+          borg[a] = R.org[a];
+          bnd[a] = (float)R.n[a] * R.d[a];
         }
-        T.dl = 1.015625f * dm;
-        T.ratio = dm / R.d[0];
-        T.level = R.level;
-        T.tile0 = R.tile0;
-        T.nt0 = R.nt0;
-        T.nt1 = R.nt1;
+        const float bdl = 1.015625f * dm, bratio = dm / R.d[0];
+        if (tid < nq) {
+          EtTarget& T = targets[tid];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            T.org[a] = R.org[a];
+            T.d[a] = R.d[a];
+            T.inv_d[a] = R.inv_d[a];
+            T.n[a] = R.n[a];
+          }
+          T.level = R.level;
+          T.tile0 = R.tile0;
+          T.nt0 = R.nt0;
+          T.nt1 = R.nt1;
+        }
+        float p[kEtRows][3], reach[kEtRows];
+#pragma unroll
+        for (int i = 0; i < kEtRows; ++i) {
+          const int k = 64 * (i * (kEtThreads / 64) + (tid >> 6)) + lane;
+          const int4 v = ent[min(k, ne - 1)];
+          const int sp = k < ne ? (int)spc[k] : kSpOutside;
+          // NaN is in no box: past the end, and a particle outside the box,
+          // which is enumerated by itself
+          p[i][0] = sp != kSpOutside ? __int_as_float(v.x) : __int_as_float(0x7fc00000);
+          p[i][1] = __int_as_float(v.y);
+          p[i][2] = __int_as_float(v.z);
+          reach[i] = ldexpf(dx, -sp);   // N cells of any level >= the species
+          if (lane < nq) mask[i * (kEtThreads / 64) + (tid >> 6)][lane] = 0ull;
+        }
+#pragma unroll 1
+        for (int j = 0; j < nq; ++j) {
+          const float l0 = readlanef(blo[0], j), l1 = readlanef(blo[1], j), l2 = readlanef(blo[2], j);
+          const float h0 = readlanef(bhi[0], j), h1 = readlanef(bhi[1], j), h2 = readlanef(bhi[2], j);
+          unsigned long long mb[kEtRows], any = 0;
+#pragma unroll
+          for (int i = 0; i < kEtRows; ++i) {
+            mb[i] = __ballot(l0 < p[i][0]) & __ballot(p[i][0] < h0) & __ballot(l1 < p[i][1]) &
+                    __ballot(p[i][1] < h1) & __ballot(l2 < p[i][2]) & __ballot(p[i][2] < h2);
+            any |= mb[i];
+          }
+          if (!any) continue;
+          // distance past the patch's cells [org, org + n d] against N cells
+          // (at least one); 1/64 of a cell of slack covers the rounding of the
+          // cell index (16,512 cells of 2^-22) and of this test
+          const float o0 = readlanef(borg[0], j), o1 = readlanef(borg[1], j), o2 = readlanef(borg[2], j);
+          const float n0 = readlanef(bnd[0], j), n1 = readlanef(bnd[1], j), n2 = readlanef(bnd[2], j);
+          const float dl = readlanef(bdl, j), ratio = readlanef(bratio, j);
+#pragma unroll
+          for (int i = 0; i < kEtRows; ++i) {
+            if (!mb[i]) continue;
+            pairs += (unsigned)__popcll(mb[i]);
+            const float lim = fmaxf(reach[i] * ratio + dl * 0.015625f, dl);
+            const float f0 = p[i][0] - o0, f1 = p[i][1] - o1, f2 = p[i][2] - o2;
+            const float far = fmaxf(fmaxf(fmaxf(-f0, f0 - n0), fmaxf(-f1, f1 - n1)), fmaxf(-f2, f2 - n2));
+            const unsigned long long tb = mb[i] & __ballot(far <= lim);
+            if (lane == j) mask[i * (kEtThreads / 64) + (tid >> 6)][j] = tb;
+          }
+        }
       }
       __syncthreads();
       auto work = [&](auto pass_c) {
@@ -670,46 +733,10 @@ __global__ void __launch_bounds__(kEtThreads) emit_table(Plan P, const Item* ite
         };
 #pragma unroll 1
         for (int r = tid >> 6; 64 * r < ne; r += kEtThreads / 64) {
-          const bool in = 64 * r + lane < ne;
-          float p[3] = {0.f, 0.f, 0.f}, reach = 0.f;
-          bool ok = false;
-          if (pass == 0) {
-            const int4 v = in ? ent[64 * r + lane] : make_int4(0, 0, 0, 0);
-            const int sp = in ? (int)spc[64 * r + lane] : kSpOutside;
-            ok = sp != kSpOutside;   // a particle outside the box is enumerated by itself
-            p[0] = __int_as_float(v.x);
-            p[1] = __int_as_float(v.y);
-            p[2] = __int_as_float(v.z);
-            reach = ldexpf(dx, -sp);   // N cells of any level >= the species
-          }
-#pragma unroll 1
-          for (int j = 0; j < nq; ++j) {
-            unsigned long long tb = 0;
-            if (pass == 0) {
-              const EtTarget& T = targets[j];
-              const unsigned long long mb =
-                  __ballot(ok && T.lo[0] < p[0] && p[0] < T.hi[0] && T.lo[1] < p[1] && p[1] < T.hi[1] &&
-                           T.lo[2] < p[2] && p[2] < T.hi[2]);
-              if (mb) {
-                pairs += (unsigned)__popcll(mb);
-                // distance past the patch's cells [org, org + n d] against
-                // N cells (at least one); 1/64 of a cell of slack covers the
-                // rounding of the cell index (16,512 cells of 2^-22) and of
-                // this test
-                const float lim = fmaxf(reach * T.ratio + T.dl * 0.015625f, T.dl);
-                float far = 0.f;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                  const float f = p[a] - T.org[a];
-                  far = fmaxf(far, fmaxf(-f, f - T.nd[a]));
-                }
-                tb = mb & __ballot(far <= lim);
-              }
-              if (lane == 0) mask[r][j] = tb;
-            } else {
-              tb = mask[r][j];
-            }
-            if (!tb) continue;
+          const unsigned long long mine = lane < nq ? mask[r][lane] : 0ull;
+          for (unsigned long long js = __ballot(mine != 0ull); js; js &= js - 1) {
+            const int j = __ffsll((long long)js) - 1;
+            const unsigned long long tb = readlane64(mine, j);
             if ((tb >> lane) & 1ull)
               pd[np + __popcll(tb & ((1ull << lane) - 1ull))] = (unsigned)(64 * r + lane) | ((unsigned)j << 10);
             np += __popcll(tb);
