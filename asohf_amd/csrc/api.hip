@@ -208,6 +208,7 @@ struct asohf_ctx {
   PipeArgs gkey;
   DBuf h_in[4], h_out[2], h_mass;    // device copies for the host entry point
   DBuf ord[4], ord_tmp;              // adjoint gather order: keys and indices (in, out), sort scratch
+  DBuf ord_rec;                      // its packed particles
   Counters* hcount = nullptr;          // pinned
   unsigned long long* hscalar = nullptr;
   hipEvent_t ev[9] = {};   // 0 start, 1 count pass, 2 scatter start, 3 scatter end, 4 deposit start,
@@ -225,8 +226,15 @@ constexpr unsigned kTableTargets = 1024;
 // takes the count and scatter passes
 constexpr long long kOutsideMax = 1ll << 20;
 
-// particles from which the adjoint gathers in base-cell order
-constexpr long long kAdjointSortMin = 1ll << 20;
+// particles from which the adjoint gathers in the order of their positions: the
+// sort costs more than scattered rows below it, whatever the input's order
+// (1M particles: 261 us sorted, 131 unsorted with the input ordered by halo and
+// 220 shuffled; 2.1M: 351 against 262 and 451; 4.2M: 594 against 614 and 1,107)
+constexpr long long kAdjointSortMin = 3ll << 19;
+// sub-cells per axis of that order, as a power of two: particles of a cell lie
+// in different cells of its patches.  Adjoint of 16.8M particles: 2,500 us with
+// 0, 2,455 with 1, 2,436 with 2 (2.1M: 359, 354, 354)
+constexpr int kAdjointSub = 2;
 
 static asohf_status fail(asohf_ctx* c, asohf_status st, const std::string& msg) {
   if (c) c->err = msg;
@@ -1382,7 +1390,7 @@ void asohf_hip_destroy(asohf_ctx* ctx) {
                   &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->split, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries, &ctx->items,
                   &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1], &ctx->h_in[2],
                   &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0], &ctx->ord[1],
-                  &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount, &ctx->sp_k[0],
+                  &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->ord_rec, &ctx->elist, &ctx->eoff, &ctx->ecount, &ctx->sp_k[0],
                   &ctx->sp_k[1], &ctx->sp_k[2], &ctx->sp_k[3], &ctx->sp_dens, &ctx->sp_cnt, &ctx->sp_tmp,
                   &ctx->pk_r[0], &ctx->pk_r[1], &ctx->pk_k[0], &ctx->pk_k[1], &ctx->pk_tmp, &ctx->pk_cnt,
                   &ctx->pk_geo, &ctx->mk_geo, &ctx->mk_err, &ctx->vg_cnt, &ctx->vg_start, &ctx->vg_pairs};
@@ -1497,16 +1505,23 @@ asohf_status asohf_hip_density_adjoint(asohf_ctx* ctx, const asohf_geom* geom, i
   // the forward's input checks (non-finite values, negative masses,
   // positions outside the TSC base range), read back after the gather
   HIPCHK(launch_fill_u32((unsigned*)C, 0u, sizeof(Counters) / 4, s), "clearing counters");
-  // Large inputs are gathered in base-cell order (a radix sort of (cell,
-  // index) pairs): neighbouring lanes then read the same gradient rows.  The
+  // Large inputs are gathered in the order of their base cells (a radix sort
+  // of (key, index) pairs): neighbouring lanes then read the same gradient rows.  The
   // key pass makes the input checks; smaller inputs get the validation pass.
   const bool sorted = n >= kAdjointSortMin && n < (1ll << 32);
   if (n > 0 && !sorted) HIPCHK(launch_plain_validate(ctx->plan.dev, A, C, ctx->cus, s), "validation");
   const unsigned* order = nullptr;
+  float4* rec = nullptr;
   if (sorted) {
-    const long long nc = (long long)geom->nx * geom->ny * geom->nz;
-    int bits = 1;
-    while (bits < 32 && (1ll << bits) < nc) ++bits;
+    const long long na[3] = {geom->nx, geom->ny, geom->nz};
+    KeyBits B{{0, 0, 0}, (float)(1 << kAdjointSub)};
+    for (int a = 0; a < 3; ++a)
+      while ((1ll << B.b[a]) < na[a] << kAdjointSub) ++B.b[a];
+    while (B.b[0] + B.b[1] + B.b[2] > 32) {   // a coarser grid on every axis
+      for (int a = 0; a < 3; ++a) B.b[a] = std::max(B.b[a] - 1, 0);
+      B.scale *= 0.5f;
+    }
+    const int bits = B.b[0] + B.b[1] + B.b[2];
     const size_t b4 = sizeof(unsigned) * (size_t)n;
     HIPCHK(ctx->ord[0].ensure(b4), "allocating the gather order");
     HIPCHK(ctx->ord[1].ensure(b4), "allocating the gather order");
@@ -1516,14 +1531,19 @@ asohf_status asohf_hip_density_adjoint(asohf_ctx* ctx, const asohf_geom* geom, i
     HIPCHK(sort_cell_pairs(nullptr, tb, nullptr, nullptr, nullptr, nullptr, (unsigned long long)n, bits, s),
            "sizing the sort");
     HIPCHK(ctx->ord_tmp.ensure(std::max<size_t>(tb, 1)), "allocating the sort");
-    HIPCHK(launch_cell_keys(ctx->plan.dev, A, ctx->ord[0].as<unsigned>(), ctx->ord[1].as<unsigned>(), C, ctx->cus, s),
+    // the packed records, where memory allows (the gather does without them)
+    if (ctx->ord_rec.ensure(sizeof(float4) * (size_t)n) == hipSuccess) rec = ctx->ord_rec.as<float4>();
+    else (void)hipGetLastError();
+    HIPCHK(launch_cell_keys(ctx->plan.dev, A, B, ctx->ord[0].as<unsigned>(), ctx->ord[1].as<unsigned>(), rec, C,
+                            ctx->cus, s),
            "cell keys");
     HIPCHK(sort_cell_pairs(ctx->ord_tmp.p, tb, ctx->ord[0].as<unsigned>(), ctx->ord[2].as<unsigned>(),
                            ctx->ord[1].as<unsigned>(), ctx->ord[3].as<unsigned>(), (unsigned long long)n, bits, s),
            "sorting by cell");
     order = ctx->ord[3].as<unsigned>();
   }
-  if (n > 0) HIPCHK(launch_adjoint(ctx->plan.dev, A, g1, g11, dm, dxp, dyp, dzp, order, ctx->cus, s), "adjoint kernel");
+  if (n > 0) HIPCHK(launch_adjoint(ctx->plan.dev, A, g1, g11, dm, dxp, dyp, dzp, order, rec, ctx->cus, s),
+                    "adjoint kernel");
   HIPCHK(hipEventRecord(ctx->ev[6], s), "event");
   HIPCHK(hipMemcpyAsync(ctx->hcount, C, sizeof(Counters), hipMemcpyDeviceToHost, s), "reading counters");
   HIPCHK(hipStreamSynchronize(s), "adjoint");
@@ -2337,7 +2357,7 @@ asohf_status asohf_hip_release_workspaces(asohf_ctx* ctx) {
                   &ctx->nitems, &ctx->icnt, &ctx->ipairs, &ctx->split, &ctx->spc, &ctx->outside, &ctx->units, &ctx->tmass, &ctx->entries,
                   &ctx->items, &ctx->scratch, &ctx->flags, &ctx->idx, &ctx->h_in[0], &ctx->h_in[1],
                   &ctx->h_in[2], &ctx->h_in[3], &ctx->h_out[0], &ctx->h_out[1], &ctx->h_mass, &ctx->ord[0],
-                  &ctx->ord[1], &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->elist, &ctx->eoff, &ctx->ecount,
+                  &ctx->ord[1], &ctx->ord[2], &ctx->ord[3], &ctx->ord_tmp, &ctx->ord_rec, &ctx->elist, &ctx->eoff, &ctx->ecount,
                   &ctx->sp_k[0], &ctx->sp_k[1], &ctx->sp_k[2], &ctx->sp_k[3], &ctx->sp_dens, &ctx->sp_cnt,
                   &ctx->sp_tmp, &ctx->pk_r[0], &ctx->pk_r[1], &ctx->pk_k[0], &ctx->pk_k[1], &ctx->pk_tmp,
                   &ctx->pk_cnt, &ctx->pk_geo, &ctx->mk_geo, &ctx->mk_err, &ctx->vg_cnt, &ctx->vg_start,

@@ -65,6 +65,13 @@ struct BoxRec {
 };
 static_assert(sizeof(BoxRec) == 128, "eight 16-byte loads");
 
+// The adjoint's gather key: bits per axis of a position in units of
+// 1/scale base cells.
+struct KeyBits {
+  int b[3];
+  float scale;
+};
+
 // Per-level spatial hash of patch membership boxes.
 struct LevelHash {
   float x0, inv_bs;  // bucket b = clamp(floor((x - x0) * inv_bs), 0, nb-1)

@@ -1696,12 +1696,15 @@ __device__ __forceinline__ void load_row3(const float* p, float out[3]) {
   out[2] = r.v[2];
 }
 
-// Base-cell key (x fastest) of every particle, for the gather order of the
-// adjoint: lanes of a wave that take particles of one cell read the same
-// rows of the upstream gradient.  The pass also makes the TSC input checks
-// (non-finite values, negative masses, positions outside the base range:
-// the flags of the forward's validation), as it reads the positions anyway.
-__global__ void __launch_bounds__(256) cell_keys(Plan P, Parts A, unsigned* key, unsigned* idx, Counters* C) {
+// Gather key of every particle for the adjoint: the bits of its position in
+// base cells of 2^-sub, interleaved, so that neighbours in the order are
+// neighbours in space and their gradient rows are cached together.  The pass
+// also packs the particles, (x, y, z, m) in one 16-byte record each (rec NULL:
+// not), and makes the TSC input checks (non-finite values, negative masses,
+// positions outside the base range: the flags of the forward's validation), as
+// it reads the positions anyway.
+__global__ void __launch_bounds__(256) cell_keys(Plan P, Parts A, KeyBits B, unsigned* key, unsigned* idx,
+                                                 float4* rec, Counters* C) {
   const GridDesc& G = P.grids[0];
   unsigned err = 0;
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < A.n;
@@ -1716,10 +1719,20 @@ __global__ void __launch_bounds__(256) cell_keys(Plan P, Parts A, unsigned* key,
       for (int a = 0; a < 3; ++a)
         if (!tsc_base_in_range(p[a], P.xl, G.inv_d[a], G.n[a])) err |= kErrWrap;
     }
-    int c[3];
+    unsigned c[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) c[a] = clampi(tsc_base_index(p[a], P.xl, G.d[a], G.inv_d[a], G.n[a]), 1, G.n[a]) - 1;
-    key[i] = (unsigned)c[0] + (unsigned)G.n[0] * ((unsigned)c[1] + (unsigned)G.n[1] * (unsigned)c[2]);
+    for (int a = 0; a < 3; ++a) {
+      const float t = (p[a] - P.xl) * G.inv_d[a] * B.scale;
+      c[a] = t > 0.f ? min((unsigned)fminf(t, 2.0e9f), (1u << B.b[a]) - 1u) : 0u;
+    }
+    // highest bits first; an axis out of bits drops out
+    unsigned k = 0u;
+    for (int b = max(max(B.b[0], B.b[1]), B.b[2]); b-- > 0;)
+#pragma unroll
+      for (int a = 2; a >= 0; --a)
+        if (b < B.b[a]) k = (k << 1) | ((c[a] >> b) & 1u);
+    key[i] = k;
+    if (rec) rec[i] = make_float4(p[0], p[1], p[2], m);
     idx[i] = (unsigned)i;
   }
   err = wave_or(err);
@@ -1745,18 +1758,27 @@ struct AdjAcc {
 };
 
 // One thread per particle, in the given order (NULL: index order).  The
-// result of a particle does not depend on the order.  Eight workgroups per
-// CU (at most 64 VGPRs, a few of them spilled): the gather waits on memory,
-// and the extra waves in flight gain more than the spills cost.
+// result of a particle does not depend on the order.  With packed records the
+// particle is read from its record and its results replace it there (dm, dx,
+// dy, dz; adjoint_unpack moves them to their arrays): in another order than the
+// arrays', every access to one costs a 64-byte sector, and a record is one
+// sector instead of four in and four out.  Eight workgroups per CU (at most 64
+// VGPRs, a few of them spilled): the gather waits on memory, and the extra waves
+// in flight gain more than the spills cost.
+// 16.8M particles, 4 levels: 2,909 us in x-fastest order of the cells without
+// records; with both 1,720 and 89 to unpack, the whole adjoint 3,290 -> 2,440
+// us; 2.1M 370 -> 354 us.  A contiguous part of the order per XCD was slower by
+// 1 to 5 percent (the parts' costs differ).
 __global__ void __launch_bounds__(256, 8) adjoint_gather(Plan P, Parts A, const float* g1, const float* g11,
                                                       float* dm, float* dxo, float* dyo, float* dzo,
-                                                      const unsigned* order) {
+                                                      const unsigned* order, float4* rec) {
   for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < A.n;
        t += (long long)gridDim.x * blockDim.x) {
     const long long i = order ? (long long)order[t] : t;
     if (i >= A.n) continue;   // the order is a permutation of [0, n); checked so a bad one cannot read out of range
-    const float p[3] = {A.x[i], A.y[i], A.z[i]};
-    const float m = A.m[i];
+    const float4 r = rec ? rec[i] : make_float4(A.x[i], A.y[i], A.z[i], A.m[i]);
+    const float p[3] = {r.x, r.y, r.z};
+    const float m = r.w;
     AdjAcc acc;
     // the first level's hash slot is loaded while the base grid is handled
     Probe nxt;
@@ -1840,10 +1862,26 @@ __global__ void __launch_bounds__(256, 8) adjoint_gather(Plan P, Parts A, const 
       }
       if (!any && P.nested) break;
     }
-    dm[i] = acc.am;
-    dxo[i] = m * acc.ax;
-    dyo[i] = m * acc.ay;
-    dzo[i] = m * acc.az;
+    if (rec) {
+      rec[i] = make_float4(acc.am, m * acc.ax, m * acc.ay, m * acc.az);
+    } else {
+      dm[i] = acc.am;
+      dxo[i] = m * acc.ax;
+      dyo[i] = m * acc.ay;
+      dzo[i] = m * acc.az;
+    }
+  }
+}
+
+// the adjoint's results from their records to the caller's arrays
+__global__ void __launch_bounds__(256) adjoint_unpack(long long n, const float4* rec, float* dm, float* dx, float* dy,
+                                                      float* dz) {
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const float4 r = rec[i];
+    dm[i] = r.x;
+    dx[i] = r.y;
+    dy[i] = r.z;
+    dz[i] = r.w;
   }
 }
 
@@ -2218,15 +2256,16 @@ hipError_t launch_finish_call(const Plan& P, const DepArgs& D, int reduction, do
   return hipGetLastError();
 }
 
-hipError_t launch_cell_keys(const Plan& P, const Parts& A, unsigned* key, unsigned* idx, Counters* C, int cus,
-                            hipStream_t s) {
-  cell_keys<<<grid_for(A.n, 256, cus * 16), 256, 0, s>>>(P, A, key, idx, C);
+hipError_t launch_cell_keys(const Plan& P, const Parts& A, const KeyBits& B, unsigned* key, unsigned* idx,
+                            float4* rec, Counters* C, int cus, hipStream_t s) {
+  cell_keys<<<grid_for(A.n, 256, cus * 16), 256, 0, s>>>(P, A, B, key, idx, rec, C);
   return hipGetLastError();
 }
 
 hipError_t launch_adjoint(const Plan& P, const Parts& A, const float* g1, const float* g11, float* dm,
-                          float* dx, float* dy, float* dz, const unsigned* order, int cus, hipStream_t s) {
-  adjoint_gather<<<grid_for(A.n, 256, cus * 16), 256, 0, s>>>(P, A, g1, g11, dm, dx, dy, dz, order);
+                          float* dx, float* dy, float* dz, const unsigned* order, float4* rec, int cus, hipStream_t s) {
+  adjoint_gather<<<grid_for(A.n, 256, cus * 16), 256, 0, s>>>(P, A, g1, g11, dm, dx, dy, dz, order, rec);
+  if (rec) adjoint_unpack<<<grid_for(A.n, 256, cus * 16), 256, 0, s>>>(A.n, rec, dm, dx, dy, dz);
   return hipGetLastError();
 }
 

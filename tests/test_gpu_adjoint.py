@@ -186,3 +186,26 @@ def test_adjoint_rejects_invalid_input_in_gather_order(bld):
     outs = bld.adjoint(g, *dev(x0, y0, z0, m0), w + 1.0, None)
     for t in outs:
         assert torch.isfinite(t).all()
+
+
+@pytest.mark.parametrize("n", [(3 << 19) - 1, 3 << 19, (3 << 19) + 77])
+def test_adjoint_of_a_call_equals_its_parts(bld, n):
+    """From 3 * 2^19 particles on, the gather takes them in the order of their
+    positions, packed in records; a particle's result is the same bits as in a
+    smaller call, which takes them as they come."""
+    snap, _ = load_fixture("seeded_12")
+    g = snap.geom
+    rng = np.random.default_rng(n)
+    pick = rng.integers(0, snap.n, n)
+    h = np.abs(np.concatenate([snap.x, snap.y, snap.z])).max()
+    p = [np.clip(v[pick] + rng.normal(0, 0.01 * h, n).astype(np.float32), -h, h).astype(np.float32)
+         for v in (snap.x, snap.y, snap.z)]
+    x, y, z, m = dev(*p, snap.m[pick])
+    t1, t11 = dev(rng.standard_normal((g.nz, g.ny, g.nx)).astype(np.float32),
+                  rng.standard_normal(max(int(g.patch_cells().sum()), 1)).astype(np.float32))
+    whole = bld.adjoint(g, x, y, z, m, t1, t11)
+    half = n // 2
+    parts = [bld.adjoint(g, *[v[s].contiguous() for v in (x, y, z, m)], t1, t11)
+             for s in (slice(0, half), slice(half, n))]
+    for k, nm in enumerate(("dm", "dx", "dy", "dz")):
+        assert torch.equal(whole[k], torch.cat([parts[0][k], parts[1][k]])), nm
