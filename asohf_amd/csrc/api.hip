@@ -2233,13 +2233,38 @@ asohf_status asohf_hip_create_mesh(asohf_ctx* ctx, const asohf_geom* base, int64
   if (n > 0)
     HIPCHK(launch_mesh_count_base(A, nx, ny, nz, base->dx, base->dy, base->dz, pr.refine_thr, dcount, ctx->cus, s),
            "base-grid counts");
-  std::vector<int> conta((size_t)nc);
-  HIPCHK(hipMemcpyAsync(conta.data(), dcount, sizeof(int) * (size_t)nc, hipMemcpyDeviceToHost, s),
-         "reading the base counts");
-  HIPCHK(hipStreamSynchronize(s), "base-grid counts");
   std::vector<MeshPatchHost> all;
-  std::string e = mesh_first_level(nx, ny, nz, rad[0].data(), rad[1].data(), rad[2].data(), conta, pr, all);
-  if (!e.empty()) return fail(ctx, ASOHF_ERR_INVALID, e);
+  std::string e;
+  if (pr.refine_thr >= 1) {
+    // the cells that reach the threshold: every one holds a particle
+    const size_t cap_seeds = (size_t)std::max(std::min<long long>(nc, n), 1ll);
+    HIPCHK(ctx->vg_cnt.ensure((size_t)nc), "allocating the cell flags");
+    HIPCHK(ctx->vg_pairs.ensure(sizeof(MeshSeed) * cap_seeds), "allocating the seed cells");
+    HIPCHK(ctx->vg_start.ensure(sizeof(unsigned long long)), "allocating the seed count");
+    HIPCHK(launch_mesh_seeds(dcount, nx, ny, nz, pr.bor, pr.refine_thr, ctx->vg_cnt.as<unsigned char>(),
+                             ctx->vg_pairs.as<MeshSeed>(), ctx->vg_start.as<unsigned long long>(), ctx->cus, s),
+           "seed cells");
+    std::vector<unsigned char> flags((size_t)nc);
+    unsigned long long n_seeds = 0;
+    HIPCHK(hipMemcpyAsync(&n_seeds, ctx->vg_start.p, sizeof(n_seeds), hipMemcpyDeviceToHost, s),
+           "reading the seed count");
+    HIPCHK(hipMemcpyAsync(flags.data(), ctx->vg_cnt.p, (size_t)nc, hipMemcpyDeviceToHost, s), "reading the cell flags");
+    HIPCHK(hipStreamSynchronize(s), "seed cells");
+    if (n_seeds > cap_seeds) return fail(ctx, ASOHF_ERR_HIP, "more seed cells than particles");
+    std::vector<MeshSeed> seeds((size_t)n_seeds);
+    if (n_seeds > 0) {
+      HIPCHK(hipMemcpyAsync(seeds.data(), ctx->vg_pairs.p, sizeof(MeshSeed) * seeds.size(), hipMemcpyDeviceToHost, s),
+             "reading the seed cells");
+      HIPCHK(hipStreamSynchronize(s), "seed cells");
+    }
+    mesh_first_level(nx, ny, nz, rad[0].data(), rad[1].data(), rad[2].data(), flags, seeds, pr, all);
+  } else {
+    std::vector<int> conta((size_t)nc);
+    HIPCHK(hipMemcpyAsync(conta.data(), dcount, sizeof(int) * (size_t)nc, hipMemcpyDeviceToHost, s),
+           "reading the base counts");
+    HIPCHK(hipStreamSynchronize(s), "base-grid counts");
+    mesh_first_level(nx, ny, nz, rad[0].data(), rad[1].data(), rad[2].data(), conta, pr, all);
+  }
   std::vector<int> npatch(kNLevels + 1, 0);
   npatch[1] = (int)all.size();
   const float rad1[3] = {rad[0][1], rad[1][1], rad[2][1]};

@@ -150,8 +150,19 @@ hipError_t launch_mesh_count_base(const Parts& A, int nx, int ny, int nz, float 
                                   int* conta, int cus, hipStream_t s);
 hipError_t launch_mesh_count_level(const Plan& P, const Parts& A, int l, const MeshPatchDev* mp, float dxpa,
                                    float dypa, float dzpa, int thr, int* conta, int cus, hipStream_t s);
-std::string mesh_first_level(int nx, int ny, int nz, const float* radx, const float* rady, const float* radz,
-                             std::vector<int>& conta1, const MeshParams& pr, std::vector<MeshPatchHost>& out);
+// a base cell that reaches the refinement threshold
+struct MeshSeed {
+  long long cell;   // x fastest
+  int count;
+  float key;        // 1 / count, when sorted
+};
+hipError_t launch_mesh_seeds(const int* conta, int nx, int ny, int nz, int bor, int thr, unsigned char* flags,
+                             MeshSeed* seeds, unsigned long long* count, int cus, hipStream_t s);
+void mesh_first_level(int nx, int ny, int nz, const float* radx, const float* rady, const float* radz,
+                      std::vector<unsigned char>& flags, std::vector<MeshSeed>& seeds, const MeshParams& pr,
+                      std::vector<MeshPatchHost>& out);
+void mesh_first_level(int nx, int ny, int nz, const float* radx, const float* rady, const float* radz,
+                      std::vector<int>& conta, const MeshParams& pr, std::vector<MeshPatchHost>& out);
 std::string mesh_next_level(int irpa, const std::vector<MeshPatchHost>& all, int first, int np,
                             std::vector<int>& conta, const std::vector<long long>& off, float dx, float dy, float dz,
                             const float rad1[3], const MeshParams& pr, int total_before,
