@@ -1075,6 +1075,8 @@ static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
   for (int l = 0; l <= kNLevels + 1; ++l) a.lvl_items[l] = ctx->hier_items[std::min(l, a.P.nl + 1)];
   a.emit_levels = ctx->plan.emit_levels;
   a.nl = a.P.nl;
+  // fewer items than CUs fit at this workgroup size: larger workgroups
+  while (a.block <= 512 && a.n_narrow * a.block * 2 <= a.cus * 1024ll) a.block *= 2;
   a.grid = (int)std::min<long long>(a.grid, std::max<long long>(a.n_items, 1));
   a.D.n_queues = std::min(kQueues, a.grid);
 }
@@ -1096,7 +1098,7 @@ static asohf_status enqueue_hier(asohf_ctx* ctx, const PipeArgs& a, hipStream_t 
            "emission pass");
   for (int l = 0; a.P.mode == 2 && l < a.nl; ++l) {
     if (!(a.emit_levels & (1u << l))) continue;
-    HIPCHK(launch_emit_tsc(a.P, a.D.items, a.lvl_items[l], a.lvl_items[l + 1], l, a.cursor, a.start, entries,
+    HIPCHK(launch_emit_tsc(a.P, a.D.items, a.lvl_items[l], a.lvl_items[l + 1], a.chunk, l, a.cursor, a.start, entries,
                            a.item_pairs, a.C, a.cus, s),
            "emission pass");
   }

@@ -170,7 +170,7 @@ __device__ __forceinline__ long long reserved_slot(unsigned long long b, unsigne
 // entries are written: 16.8M particles on 256^3 cells (16x8x8 tiles) 1,431 ->
 // 356 us, 134M particles 6.57 -> 2.11 ms.
 template <int MODE>
-__global__ void __launch_bounds__(kHbThreads) bin_base(Plan P, Parts A, unsigned long long* cursor,
+__global__ void __launch_bounds__(kHbThreads, 7) bin_base(Plan P, Parts A, unsigned long long* cursor,
                                                        const unsigned long long* start, int4* entries,
                                                        Counters* C, BlockTables BT, TableBin TB) {
   __shared__ int keys[kHbCap];
@@ -306,11 +306,12 @@ __global__ void __launch_bounds__(kHbThreads) bin_base(Plan P, Parts A, unsigned
 }
 
 // The emission pass of one level: items [item_lo, item_hi) are the work items
-// (chunks of one tile's entry range) of the level's tiles.  A workgroup takes
-// `batch` consecutive items at a time from the level's queue counter and
-// works through those whose tile has targets (the others' member counts stay
-// 0).  Per item the target records are staged in LDS (kEmTargets at a time);
-// the item's entries are taken kEmPer per thread per round (one per round
+// (chunks of one tile's entry range) of the level's tiles, each in `pieces`
+// pieces of plen entries where there are fewer items than workgroups fit.  A
+// workgroup takes `batch` consecutive pieces at a time from the level's queue
+// counter and works through those whose tile has targets (the others' member
+// counts stay 0).  Per piece the target records are staged in LDS (kEmTargets at a time);
+// the piece's entries are taken kEmPer per thread per round (one per round
 // where overlapping patches make the lists long).  In a
 // round every wave tests its entries against the targets and collects the
 // members; 64 of them at a time, one per lane, get their tile in the patch, a
@@ -321,8 +322,8 @@ __global__ void __launch_bounds__(kHbThreads) bin_base(Plan P, Parts A, unsigned
 // over the tiles of a stencil: 256^3 particles, 4 levels 1,111 -> 762 us;
 // 512^3, 6 levels 9.23 -> 6.06 ms.
 __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* items, long long item_lo,
-                                                       long long item_hi, int level, int batch,
-                                                       unsigned long long* cursor,
+                                                       long long n_pieces, int pieces, int plen, int level,
+                                                       int batch, unsigned long long* cursor,
                                                        const unsigned long long* start, int4* entries,
                                                        unsigned* item_pairs, Counters* C) {
   __shared__ int keys[kEmCap];
@@ -343,21 +344,21 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
   unsigned* ml = mlist_all + (tid >> 6) * 128;
   unsigned* queue = &C->equeue[level * kLine];
   for (;;) {
-    if (tid == 0) s_i0 = item_lo + (long long)atomicAdd(queue, (unsigned)batch);
+    if (tid == 0) s_i0 = (long long)atomicAdd(queue, (unsigned)batch);
     __syncthreads();
     const long long i0 = s_i0;
     __syncthreads();   // every wave has read s_i0 before thread 0 takes the next batch
-    if (i0 >= item_hi) break;
-    const int nb = (int)min((long long)batch, item_hi - i0);
+    if (i0 >= n_pieces) break;
+    const int nb = (int)min((long long)batch, n_pieces - i0);
     for (int bi = 0; bi < nb; ++bi) {
-      const long long ii = i0 + bi;
+      const long long ii = item_lo + (i0 + bi) / pieces;
       const Item it = items[ii];
       const int t = it.tile;
       const unsigned q0 = P.tgt_off[t], q1 = P.tgt_off[t + 1];
       if (q0 == q1) continue;
-      // the item's filled entries
-      const long long e0 = it.begin;
-      const long long e1 = min(it.end, (long long)cursor[2 * t]);
+      // the piece's filled entries
+      const long long e0 = it.begin + (i0 + bi) % pieces * plen;
+      const long long e1 = min(min(it.end, e0 + plen), (long long)cursor[2 * t]);
       if (e1 <= e0) continue;
       for (int k = tid; k < kEmCap; k += kEmThreads) { keys[k] = -1; vals[k] = 0u; }
       if (tid < 2) s_nwmax[tid] = 0;
@@ -448,14 +449,14 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
           }
         }
       }
-      // members found by this item
+      // members found in this piece
       const unsigned sw = wave_sum(pairs);
       if ((tid & 63) == 0) s_red[tid >> 6] = sw;
       __syncthreads();
       if (tid == 0) {
         unsigned tot = 0;
         for (int w = 0; w < kEmThreads / 64; ++w) tot += s_red[w];
-        item_pairs[ii] = tot;
+        if (tot) atomicAdd(&item_pairs[ii], tot);
       }
       __syncthreads();
     }
@@ -902,7 +903,7 @@ hipError_t launch_emit_table(const Plan& P, const Item* items, long long n_items
   return hipGetLastError();
 }
 
-hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, long long item_hi, int level,
+hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, long long item_hi, int chunk, int level,
                            unsigned long long* cursor, const unsigned long long* start, int4* entries,
                            unsigned* item_pairs, Counters* C, int cus, hipStream_t s) {
   if (item_hi <= item_lo) return hipSuccess;
@@ -915,11 +916,16 @@ hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, 
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, emit_tsc, kEmThreads, 0) != hipSuccess || nb <= 0) nb = 4;
     per_cu = nb;
   }
-  const long long n = item_hi - item_lo;
-  const int grid = (int)std::min<long long>(n, (long long)cus * per_cu);
+  const long long items_n = item_hi - item_lo, room = (long long)cus * per_cu;
+  // pieces of at least one round, as many as workgroups fit
+  const int rounds = (chunk + kEmRound - 1) / kEmRound;
+  const int pieces = (int)std::max<long long>(1, std::min<long long>(rounds, room / items_n));
+  const int plen = (rounds + pieces - 1) / pieces * kEmRound;
+  const long long n = items_n * pieces;
+  const int grid = (int)std::min<long long>(n, room);
   const int batch = (int)std::max<long long>(1, std::min<long long>(8, n / ((long long)grid * 16)));
-  emit_tsc<<<grid, kEmThreads, 0, s>>>(P, items, item_lo, item_hi, level, batch, cursor, start, entries, item_pairs,
-                                       C);
+  emit_tsc<<<grid, kEmThreads, 0, s>>>(P, items, item_lo, n, pieces, plen, level, batch, cursor, start, entries,
+                                       item_pairs, C);
   return hipGetLastError();
 }
 

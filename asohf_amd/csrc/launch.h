@@ -52,7 +52,7 @@ long long emit_pieces(int chunk);   // emission work units of an item of `chunk`
 hipError_t launch_emit_table(const Plan& P, const Item* items, long long n_items, int chunk,
                              unsigned long long* cursor, const unsigned long long* start, int4* entries,
                              unsigned* item_pairs, Counters* C, const TableBin& TB, int cus, hipStream_t s);
-hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, long long item_hi, int level,
+hipError_t launch_emit_tsc(const Plan& P, const Item* items, long long item_lo, long long item_hi, int chunk, int level,
                            unsigned long long* cursor, const unsigned long long* start, int4* entries,
                            unsigned* item_pairs, Counters* C, int cus, hipStream_t s);
 // the first and the last kernel of a call binned through the base grid
