@@ -1438,12 +1438,15 @@ __global__ void __launch_bounds__(kWideThreads, 4) deposit_wide(Plan P, DepArgs 
 // divided by DENBAS then FDM (FP32, the reference's two divisions) and stored
 // row by row.  The exact int64 (FP64 in atomic mode) tile mass is the sum of
 // the cells before the divisions.
-// Exchanging halo sums costs 14 B written and read per cell of a 16x8x8 tile
-// (179 us on 18.1M cells, 1.18 ms on 93.9M), less than the entries it saves:
-// a stencil crossing tile borders used to be binned, emitted and deposited
-// once per tile it touched, 1.5 to 1.8 entries per member (the whole build on
-// 256^3 particles and 4 levels 4.01 -> 2.22 ms, 512^3 and 6 levels 28.9 ->
-// 18.0 ms).
+// Exchanging halo sums costs 14 B written and read per cell of a 16x8x8 tile,
+// less than the entries it saves: a stencil crossing tile borders used to be
+// binned, emitted and deposited once per tile it touched, 1.5 to 1.8 entries
+// per member (the whole build on 256^3 particles and 4 levels 4.01 -> 2.22 ms,
+// 512^3 and 6 levels 28.9 -> 18.0 ms).
+// Bound by latency in small builds and by the strided halo reads in large ones.
+// A thread's four cells are loaded together, their neighbours' terms too: one
+// after the other they took 13 us on 38,000 cells (now 6.4), 180 on 18.1M (157)
+// and 1,184 on 93.9M (1,016).
 template <int RED, int TX, int TY, int TZ>
 __global__ void __launch_bounds__(256) combine_tiles(Plan P, DepArgs D) {
   using Acc = typename AccT<RED>::T;
@@ -1488,39 +1491,95 @@ __global__ void __launch_bounds__(256) combine_tiles(Plan P, DepArgs D) {
     float* out = (g == 0 ? D.u1 : D.u11) + G.off;
     long long msi = 0;
     double msd = 0.0;
-    for (int c = tid; c < T; c += 256) {
-      const int l[3] = {c % TX, (c / TX) % TY, c / (TX * TY)};
-      if (l[0] >= ext[0] || l[1] >= ext[1] || l[2] >= ext[2]) continue;
-      Acc v = 0;
-      if (s_nb[13] >= 0) v = S[s_nb[13] + (l[0] + 1) + L::EX * ((l[1] + 1) + L::EY * (l[2] + 1))];
-      int lo[3], hi[3];
-      bool edge = false;
+    const long long own = s_nb[13];
+    const bool thin = ext[0] == 1 || ext[1] == 1 || ext[2] == 1;
+    constexpr int U = T / 256 < 4 ? T / 256 : 4;   // cells of a thread in flight
+    for (int c0 = tid; c0 < T; c0 += 256 * U) {
+      Acc v[U];
+      if (!thin) {
+        // a cell has a neighbour on at most one side per axis: up to 7 terms,
+        // all loads issued before the first is used
+        Acc term[U][8];
 #pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        lo[a] = l[a] == 0 ? -1 : 0;
-        hi[a] = l[a] == ext[a] - 1 ? 1 : 0;
-        edge = edge || lo[a] < 0 || hi[a] > 0;
-      }
-      if (edge) {
-        for (int dz = lo[2]; dz <= hi[2]; ++dz)
-          for (int dy = lo[1]; dy <= hi[1]; ++dy)
-            for (int dx = lo[0]; dx <= hi[0]; ++dx) {
-              const long long nb = s_nb[(dx + 1) + 3 * ((dy + 1) + 3 * (dz + 1))];
-              if ((dx | dy | dz) == 0 || nb < 0) continue;
-              // this cell in the neighbour's coordinates: past the last cell
-              // of the tile before, or the halo below the tile after
-              const int x = dx == 0 ? l[0] : (dx < 0 ? prev[0] : -1);
-              const int y = dy == 0 ? l[1] : (dy < 0 ? prev[1] : -1);
-              const int z = dz == 0 ? l[2] : (dz < 0 ? prev[2] : -1);
-              v += S[nb + (x + 1) + L::EX * ((y + 1) + L::EY * (z + 1))];
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + 256 * u;
+          const int l[3] = {c % TX, (c / TX) % TY, c / (TX * TY)};
+          const bool on = l[0] < ext[0] && l[1] < ext[1] && l[2] < ext[2];
+          constexpr int pitch[3] = {1, L::EX, L::EX * L::EY}, step[3] = {1, 3, 9};
+          int self[3], side[3], nbr[3];   // the cell's offset, as seen from its side's tile, and that tile's slot
+          bool has[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) {
+            const bool low = l[a] == 0, high = l[a] == ext[a] - 1;
+            has[a] = on && (low || high);
+            self[a] = (l[a] + 1) * pitch[a];
+            side[a] = (low ? prev[a] + 1 : 0) * pitch[a];
+            nbr[a] = low ? -step[a] : step[a];
+          }
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            term[u][k] = 0;
+            const bool need = k == 0 ? on && own >= 0
+                                     : (!(k & 1) || has[0]) && (!(k & 2) || has[1]) && (!(k & 4) || has[2]);
+            if (need) {
+              const long long nb =
+                  k == 0 ? own : s_nb[13 + (k & 1 ? nbr[0] : 0) + (k & 2 ? nbr[1] : 0) + (k & 4 ? nbr[2] : 0)];
+              if (nb >= 0)
+                term[u][k] = S[nb + (k & 1 ? side[0] : self[0]) + (k & 2 ? side[1] : self[1]) +
+                               (k & 4 ? side[2] : self[2])];
             }
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          v[u] = term[u][0];
+#pragma unroll
+          for (int k = 1; k < 8; ++k) v[u] += term[u][k];
+        }
+      } else {
+        // a tile one cell wide: neighbours on both sides of a cell
+#pragma unroll 1
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + 256 * u;
+          const int l[3] = {c % TX, (c / TX) % TY, c / (TX * TY)};
+          Acc w = 0;
+          if (l[0] < ext[0] && l[1] < ext[1] && l[2] < ext[2]) {
+            int lo[3], hi[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+              lo[a] = l[a] == 0 ? -1 : 0;
+              hi[a] = l[a] == ext[a] - 1 ? 1 : 0;
+            }
+            for (int dz = lo[2]; dz <= hi[2]; ++dz)
+              for (int dy = lo[1]; dy <= hi[1]; ++dy)
+                for (int dx = lo[0]; dx <= hi[0]; ++dx) {
+                  const long long nb = s_nb[(dx + 1) + 3 * ((dy + 1) + 3 * (dz + 1))];
+                  if (nb < 0) continue;
+                  // this cell in the neighbour's coordinates: past the last cell
+                  // of the tile before, or the halo below the tile after
+                  const int x = dx == 0 ? l[0] : (dx < 0 ? prev[0] : -1);
+                  const int y = dy == 0 ? l[1] : (dy < 0 ? prev[1] : -1);
+                  const int z = dz == 0 ? l[2] : (dz < 0 ? prev[2] : -1);
+                  w += S[nb + (x + 1) + L::EX * ((y + 1) + L::EY * (z + 1))];
+                }
+          }
+#pragma unroll
+          for (int q = 0; q < U; ++q)
+            if (q == u) v[q] = w;
+        }
       }
-      if (RED == 0) msi += (long long)v;
-      else msd += (double)v;
-      float f = RED == 0 ? (float)((double)v * inv_scale) : (float)v;
-      f = f / G.den;
-      f = f / P.fdm;
-      out[(long long)(o[0] + l[0]) + (long long)G.ld1 * (o[1] + l[1]) + (long long)G.ld2 * (o[2] + l[2])] = f;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = c0 + 256 * u;
+        const int l[3] = {c % TX, (c / TX) % TY, c / (TX * TY)};
+        if (l[0] >= ext[0] || l[1] >= ext[1] || l[2] >= ext[2]) continue;
+        if (RED == 0) msi += (long long)v[u];
+        else msd += (double)v[u];
+        float f = RED == 0 ? (float)((double)v[u] * inv_scale) : (float)v[u];
+        f = f / G.den;
+        f = f / P.fdm;
+        out[(long long)(o[0] + l[0]) + (long long)G.ld1 * (o[1] + l[1]) + (long long)G.ld2 * (o[2] + l[2])] = f;
+      }
     }
     if (RED == 0) {
       msi = block_sum(msi, s_redi);
