@@ -49,11 +49,14 @@ constexpr int kHbCap = 1024;                     // LDS key slots (power of two,
 constexpr int kHbProbe = 32;
 constexpr int kEmThreads = 256;
 constexpr int kEmPer = 2;                        // entries per thread and round
-constexpr int kEmRound = kEmPer * kEmThreads;    // entries per round (< 2^16: a list word's position)
-constexpr int kEmCap = 512;                      // LDS key slots of an item (< 2^16)
+constexpr int kEmRound = kEmPer * kEmThreads;    // entries per round
+constexpr int kEmCap = 512;                      // LDS key slots of an item
 constexpr int kEmWList = 384;                    // list words per wave and round
-constexpr unsigned long long kEmSkip = ~0ull;    // list word of an emission written directly
-static_assert(kEmRound <= 65536 && kEmCap <= 65536, "a list word holds (entry, slot, position)");
+constexpr unsigned kEmSkip = ~0u;                // list word of an emission written directly
+// a list word: the key's slot | position in the key's range of the round << 9 |
+// entry of the round << 19 (an entry is in a patch's tile at most once, so a
+// position is below kEmRound)
+static_assert(kEmPer == 2 && kEmRound <= 512 && kEmCap <= 512, "the fields of a list word");
 constexpr int kEmTargets = 32;                   // target records staged in LDS at once
 
 __device__ __forceinline__ unsigned slot_hash(unsigned k, unsigned mask) {
@@ -310,17 +313,21 @@ __global__ void __launch_bounds__(kHbThreads, 7) bin_base(Plan P, Parts A, unsig
 // pieces of plen entries where there are fewer items than workgroups fit.  A
 // workgroup takes `batch` consecutive pieces at a time from the level's queue
 // counter and works through those whose tile has targets (the others' member
-// counts stay 0).  Per piece the target records are staged in LDS (kEmTargets at a time);
-// the piece's entries are taken kEmPer per thread per round (one per round
-// where overlapping patches make the lists long).  In a
-// round every wave tests its entries against the targets and collects the
-// members; 64 of them at a time, one per lane, get their tile in the patch, a
-// position in the tile key's range of the round and a word in the wave's
-// list; one global add per key reserves the round's ranges and every wave
-// writes its listed entries, reading each again from its source tile.
-// Bound by VALU work and latency.  With one entry per member no lane loops
-// over the tiles of a stencil: 256^3 particles, 4 levels 1,111 -> 762 us;
-// 512^3, 6 levels 9.23 -> 6.06 ms.
+// counts stay 0).  Per piece the target records are staged in LDS (kEmTargets
+// at a time); the piece's entries are taken kEmPer per thread per round (one
+// per round where overlapping patches make the lists long), loaded a round
+// ahead and kept in LDS.  In a round every wave tests its entries against the
+// targets and collects the members; 64 of them at a time, one per lane, get
+// their tile in the patch, a position in the tile key's range of the round and
+// a word in the wave's list; one global add per key reserves the round's ranges
+// and every wave writes its listed entries from LDS.
+// Bound by latency (the waves wait 80 percent of their time, VALU 35 percent
+// busy): the reservation's round trip and the barriers of a round.  With one
+// entry per member instead of one per tile, rounds loaded ahead, and entries
+// written from LDS instead of read again: 256^3 particles, 4 levels 1,111 ->
+// 762 -> 704 us; 512^3, 6 levels 9.23 -> 6.06 -> 5.52 ms.  Six workgroups per CU
+// (48 bytes a lane spilled) take 705 us and 5.30 ms, but 158 instead of 138 us
+// on 2.1M particles.  Pieces: 13,824 particles, 3 levels 75 -> 25 us.
 __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* items, long long item_lo,
                                                        long long n_pieces, int pieces, int plen, int level,
                                                        int batch, unsigned long long* cursor,
@@ -329,14 +336,15 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
   __shared__ int keys[kEmCap];
   __shared__ unsigned vals[kEmCap];
   __shared__ unsigned long long base[kEmCap];
-  __shared__ unsigned long long wlist_all[(kEmThreads / 64) * kEmWList];
+  __shared__ unsigned wlist_all[(kEmThreads / 64) * kEmWList];
+  __shared__ int4 stage[kEmRound];   // the round's entries; a wave reads its own
   __shared__ unsigned mlist_all[(kEmThreads / 64) * 128];
   __shared__ BoxRec recs[kEmTargets];
   __shared__ long long s_i0;
   __shared__ unsigned s_red[kEmThreads / 64];
   __shared__ int s_nwmax[2];   // the waves' longest list of a round, by round parity
   const int tid = threadIdx.x, lane = (int)__lane_id();
-  unsigned long long* wl = wlist_all + (tid >> 6) * kEmWList;
+  unsigned* wl = wlist_all + (tid >> 6) * kEmWList;
   // wave-steps per round: kEmPer, or 1 after a round whose lists would have
   // overflowed with kEmPer (members of overlapping patches emit several
   // entries each); kept from one item to the next
@@ -369,16 +377,26 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
         for (int k = tid; k < nq * 8; k += kEmThreads)
           reinterpret_cast<int4*>(recs)[k] = reinterpret_cast<const int4*>(P.grec + P.tgt[q + (k >> 3)])[k & 7];
         __syncthreads();
+        // the next round's entries, on their way while this one is worked through
+        int4 nxt0, nxt1;
+        auto fetch = [&](long long r) {
+          nxt0 = entries[min(r + tid, e1 - 1)];
+          nxt1 = entries[min(r + kEmThreads + tid, e1 - 1)];
+        };
+        fetch(e0);
         for (long long r0 = e0, rn = 0; r0 < e1; r0 += rn) {
           const int nsteps = steps;
           rn = (long long)nsteps * kEmThreads;
+          const int4 cur0 = nxt0, cur1 = nxt1;
+          fetch(r0 + rn);
           // ---- list the wave's member emissions
           int nw = 0;   // the wave's list length (uniform)
 #pragma unroll 1
           for (int i = 0; i < nsteps; ++i) {
             const int k = i * kEmThreads + tid;
             const bool ok = r0 + k < e1;
-            const int4 v = ok ? entries[r0 + k] : make_int4(0, 0, 0, 0);
+            const int4 v = i == 0 ? cur0 : cur1;
+            stage[k] = v;
             const float p[3] = {__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z)};
             // the item's targets, one per pass: the box tests, with the
             // members listed (lane, target) in the wave's member list; every
@@ -413,7 +431,7 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
                 const int h = off < kEmWList ? count_key<kEmCap>(keys, vals, key, at) : -1;
                 if (h < 0) emit_direct(cursor, start, entries, C, key, u);
                 if (off < kEmWList)
-                  wl[off] = h < 0 ? kEmSkip : ((unsigned long long)ks << 32) | ((unsigned long long)h << 16) | at;
+                  wl[off] = h < 0 ? kEmSkip : ((unsigned)ks << 19) | (at << 9) | (unsigned)h;
               }
               nw = min(nw + __popcll(mb), kEmWList);
             };
@@ -442,10 +460,10 @@ __global__ void __launch_bounds__(kEmThreads, 5) emit_tsc(Plan P, const Item* it
           __syncthreads();
           // ---- write the listed entries
           for (int idx = lane; idx < nw; idx += 64) {
-            const unsigned long long w = wl[idx];
+            const unsigned w = wl[idx];
             if (w == kEmSkip) continue;
-            const long long pos = reserved_slot(base[(w >> 16) & 0xffffu], (unsigned)(w & 0xffffu));
-            if (pos >= 0) entries[pos] = entries[r0 + (long long)(w >> 32)];
+            const long long pos = reserved_slot(base[w & 0x1ffu], (w >> 9) & 0x3ffu);
+            if (pos >= 0) entries[pos] = stage[w >> 19];
           }
         }
       }
