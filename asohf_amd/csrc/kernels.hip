@@ -832,6 +832,9 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     const int tx = local % G.nt[0], ty = (local / G.nt[0]) % G.nt[1], tz = local / (G.nt[0] * G.nt[1]);
     const int i0 = tx * TX + 1, j0 = ty * TY + 1, k0c = tz * TZ + 1;
     const bool periodic = g == 0;
+    // two tiles on a periodic axis, the last one cell wide
+    const bool images = periodic && ((G.nt[0] == 2 && G.n[0] == TX + 1) || (G.nt[1] == 2 && G.n[1] == TY + 1) ||
+                                     (G.nt[2] == 2 && G.n[2] == TZ + 1));
 
     // the item's filled entries
     long long len = it.end - it.begin;
@@ -892,9 +895,9 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
       for (int a = 0; a < 3; ++a)
         lc[a] = MODE == 1 && RED == 1 ? centre_local(ci[a], org[a], ext[a], G.n[a], periodic)
                                       : (periodic ? wrap1(ci[a], G.n[a]) : ci[a]) - org[a];
-      if (MODE == 1 && RED == 1 && periodic && ok) {
-        // two tiles on an axis, the last one cell wide: a centre next to the
-        // wrap reaches the first tile on both sides, through two images
+      if (MODE == 1 && RED == 1 && images && ok) {
+        // a centre next to the wrap reaches the first tile on both sides,
+        // through two images
         for (int k = 1; k < 8; ++k) {
           int li[3];
           bool img = true;
@@ -927,18 +930,20 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     __syncthreads();
 
     // ---- entries in every tile they touch (P.per_tile): the halo is the other
-    // tiles' business and is cleared, after a tile spanning a whole periodic
-    // axis has folded it into its own cells (the reference's wrap) ----
-    if (MODE == 1 && RED == 1) {
-      const int ex = min(TX, G.n[0] - i0 + 1), ey = min(TY, G.n[1] - j0 + 1), ez = min(TZ, G.n[2] - k0c + 1);
-      const bool fold = periodic && (G.nt[0] == 1 || G.nt[1] == 1 || G.nt[2] == 1);
+    // tiles' business, once a tile spanning a whole periodic axis has folded it
+    // into its own cells (the reference's wrap) ----
+    const int ex = min(TX, G.n[0] - i0 + 1), ey = min(TY, G.n[1] - j0 + 1), ez = min(TZ, G.n[2] - k0c + 1);
+    auto inside = [&](int c) {
+      const int a = c % L::EX - 1, b = (c / L::EX) % L::EY - 1, cz = c / (L::EX * L::EY) - 1;
+      return a >= 0 && a < ex && b >= 0 && b < ey && cz >= 0 && cz < ez;
+    };
+    if (MODE == 1 && RED == 1 && periodic && (G.nt[0] == 1 || G.nt[1] == 1 || G.nt[2] == 1)) {
       for (int c = tid; c < L::E; c += nthr) {
+        if (inside(c)) continue;
         const int a = c % L::EX - 1, b = (c / L::EX) % L::EY - 1, cz = c / (L::EX * L::EY) - 1;
-        if (a >= 0 && a < ex && b >= 0 && b < ey && cz >= 0 && cz < ez) continue;
         const int ga = wrap1(i0 + a, G.n[0]) - i0, gb = wrap1(j0 + b, G.n[1]) - j0, gc = wrap1(k0c + cz, G.n[2]) - k0c;
-        if (fold && ga >= 0 && ga < ex && gb >= 0 && gb < ey && gc >= 0 && gc < ez && acc[at(a, b, cz)] != 0)
+        if (ga >= 0 && ga < ex && gb >= 0 && gb < ey && gc >= 0 && gc < ez && acc[at(a, b, cz)] != 0)
           lds_add(acc + at(ga, gb, gc), acc[at(a, b, cz)]);
-        acc[at(a, b, cz)] = 0;
       }
       __syncthreads();
     }
@@ -947,11 +952,12 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     // has one item, added where several items share it (exact int64 adds, so
     // the sum does not depend on their order; the cells were cleared) ----
     Acc* dst = reinterpret_cast<Acc*>(D.scratch) + (long long)t * L::E;
+    auto cell = [&](int c) -> Acc { return MODE == 1 && RED == 1 && !inside(c) ? (Acc)0 : acc[L::of_exchange(c)]; };
     if (D.nitems_tile[t] == 1) {
-      for (int c = tid; c < L::E; c += nthr) dst[c] = acc[L::of_exchange(c)];
+      for (int c = tid; c < L::E; c += nthr) dst[c] = cell(c);
     } else {
       for (int c = tid; c < L::E; c += nthr) {
-        const Acc v = acc[L::of_exchange(c)];
+        const Acc v = cell(c);
         if (v != 0) glb_add(dst + c, v);
       }
     }
