@@ -890,8 +890,9 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
 static void bind_sized(asohf_ctx* ctx, PipeArgs& a) {
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
+  a.D.work = a.D.items + ctx->items.cap / (2 * sizeof(Item));
   a.cap_entries = ctx->entries.cap / sizeof(int4);
-  a.cap_items = ctx->items.cap / sizeof(Item);
+  a.cap_items = ctx->items.cap / (2 * sizeof(Item));   // the work queue is the second half
 }
 
 // count pass: per-(tile, kind) counts, block sums, offsets and the item plan
@@ -917,6 +918,8 @@ static asohf_status enqueue_deposit(asohf_ctx* ctx, const PipeArgs& a, hipStream
   HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.chunk_wide, a.item_off, const_cast<Item*>(a.D.items), nullptr,
                            nullptr, a.C, s),
          "writing items");
+  HIPCHK(launch_order_items(a.D.items, const_cast<Item*>(a.D.work), -1, (long long)a.cap_items, a.C, a.cus, s),
+         "work queue");
   HIPCHK(launch_zero_split(a.P, a.D, a.red, a.cus, s), "clearing split tiles");
   if (events) HIPCHK(hipEventRecord(ctx->ev[4], s), "event");
   HIPCHK(launch_deposit(a.P, a.D, a.red, a.grid, a.block, s), "deposit kernel");
@@ -975,7 +978,7 @@ static asohf_status run_exact(asohf_ctx* ctx, const asohf_opts& o, const Parts& 
   if (hc.n_items >= (1ull << 31)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^31 work items");
   note_pool(ctx, hc);
   HIPCHK(ctx->entries.ensure(sizeof(int4) * std::max<unsigned long long>(hc.n_entries, 1)), "allocating entries");
-  HIPCHK(ctx->items.ensure(sizeof(Item) * std::max<unsigned long long>(hc.n_items, 1)), "allocating work items");
+  HIPCHK(ctx->items.ensure(2 * sizeof(Item) * std::max<unsigned long long>(hc.n_items, 1)), "allocating work items");
   bind_sized(ctx, a);
   a.grid = (int)std::min<long long>(a.grid, std::max<unsigned long long>(hc.n_items, 1));
   a.D.n_queues = std::min(kQueues, a.grid);
@@ -1031,7 +1034,7 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   if (cap_entries >= (1ull << 40)) return fail(ctx, ASOHF_ERR_CAPACITY, "more than 2^40 tile entries");
   for (int l = 0; l <= nl + 1; ++l) ctx->hier_items[l] = (long long)ctx->hscalar[1 + l];
   HIPCHK(ctx->entries.ensure(sizeof(int4) * std::max<unsigned long long>(cap_entries, 1)), "allocating entries");
-  HIPCHK(ctx->items.ensure(sizeof(Item) * std::max<long long>(n_items, 1)), "allocating work items");
+  HIPCHK(ctx->items.ensure(2 * sizeof(Item) * std::max<long long>(n_items, 1)), "allocating work items");
   HIPCHK(ctx->ipairs.ensure(sizeof(unsigned) * std::max<long long>(n_items, 1)), "allocating item sums");
   if (a.P.mode == 1) {
     HIPCHK(ctx->spc.ensure(std::max<unsigned long long>(ctx->hscalar[nl + 3], 1)), "allocating species");
@@ -1043,6 +1046,7 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   }
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
+  a.D.work = a.D.items + ctx->items.cap / (2 * sizeof(Item));
   HIPCHK(ctx->split.ensure(sizeof(int) * (a.ntiles + 1ll)), "allocating the split tiles");
   a.split_n = ctx->split.as<unsigned>();
   a.split_tiles = ctx->split.as<int>() + 1;
@@ -1050,6 +1054,8 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
   HIPCHK(launch_plan_write(a.start, a.ntiles, a.chunk, a.P.mode == 2 ? 0 : a.chunk_wide, a.item_off,
                            const_cast<Item*>(a.D.items), a.split_tiles, a.split_n, a.C, s),
          "writing items");
+  HIPCHK(launch_order_items(a.D.items, const_cast<Item*>(a.D.work), ctx->hier_items[nl + 1], n_items, a.C, a.cus, s),
+         "work queue");
   ctx->hier_nitems = n_items;
   ctx->hier_nnarrow = ctx->hier_items[nl + 1];
   return ASOHF_OK;
@@ -1059,6 +1065,7 @@ static asohf_status hier_plan(asohf_ctx* ctx, PipeArgs& a, hipStream_t s) {
 static void hier_bind(asohf_ctx* ctx, PipeArgs& a) {
   a.D.entries = ctx->entries.as<int4>();
   a.D.items = ctx->items.as<Item>();
+  a.D.work = a.D.items + ctx->items.cap / (2 * sizeof(Item));
   a.D.cursor = a.cursor;
   a.item_pairs = ctx->ipairs.as<unsigned>();
   a.split_n = ctx->split.as<unsigned>();

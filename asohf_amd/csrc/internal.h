@@ -206,7 +206,8 @@ struct TableBin {
 // Arguments of the persistent deposit.
 struct DepArgs {
   const int4* entries;       // binned entries, grouped by tile
-  const Item* items;         // work queue
+  const Item* items;         // work items, tile by tile, the narrow ones before the wide ones
+  const Item* work;          // the narrow items again, long ones first: the deposit's work queue
   const int* nitems_tile;    // items per tile
   void* scratch;             // exchange cells: int64 (deterministic) or FP32 (atomic), a tile with its
                              // one-cell halo per tile

@@ -500,6 +500,51 @@ __global__ void plan_write(const unsigned long long* start, int ntiles, int chun
   }
 }
 
+// The narrow items once more, long ones first (by half powers of two of their
+// length, in any order within one): a workgroup that takes a long item last
+// keeps the deposit waiting for it.  The classes' counts and then their fill
+// lie in the emission's queue words, which are 0 here.  Atomic TSC deposit of
+// 2.1M particles, whose CUs worked 496 us of it on average: 789 -> 623 us; the
+// shorter items of deterministic sums gain 1 to 4 percent.
+constexpr int kItemClasses = 64;
+__device__ __forceinline__ int item_class(const Item& it) {   // 0: longest
+  const unsigned long long len = (unsigned long long)max(it.end - it.begin, 1ll);
+  const int e = 63 - __clzll((long long)len);
+  const int c = 2 * e + (e > 0 ? (int)((len >> (e - 1)) & 1ull) : 0);
+  return kItemClasses - 1 - min(c, kItemClasses - 1);
+}
+__global__ void __launch_bounds__(256) order_items(const Item* items, Item* work, long long n_given, Counters* C,
+                                                   int pass) {
+  __shared__ unsigned cnt[kItemClasses], base[kItemClasses];
+  unsigned* const total = C->equeue;
+  unsigned* const fill = C->equeue + kItemClasses;
+  const unsigned n = n_given >= 0 ? (unsigned)n_given : C->n_items_eff;   // narrow items
+  // a contiguous part of the items per workgroup
+  const unsigned per = (n + gridDim.x - 1) / gridDim.x;
+  const unsigned i0 = min(blockIdx.x * per, n), i1 = min(i0 + per, n);
+  if (threadIdx.x < kItemClasses) cnt[threadIdx.x] = 0u;
+  __syncthreads();
+  for (unsigned i = i0 + threadIdx.x; i < i1; i += blockDim.x) atomicAdd(&cnt[item_class(items[i])], 1u);
+  __syncthreads();
+  if (threadIdx.x < kItemClasses) {
+    const unsigned c = cnt[threadIdx.x];
+    if (pass == 0) {
+      if (c) atomicAdd(&total[threadIdx.x], c);
+    } else {
+      unsigned b = 0;
+      for (int k = 0; k < (int)threadIdx.x; ++k) b += total[k];
+      base[threadIdx.x] = b + (c ? atomicAdd(&fill[threadIdx.x], c) : 0u);
+    }
+  }
+  if (pass == 0) return;
+  __syncthreads();
+  for (unsigned i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
+    const Item it = items[i];
+    const unsigned at = atomicAdd(&base[item_class(it)], 1u);
+    if (at < n) work[at] = it;
+  }
+}
+
 // The totals of the planning scans against the workspaces of this call.  A
 // call whose buffers were sized by an earlier call finds out here, on the
 // device, whether they still suffice; if not, every later kernel of the call
@@ -824,7 +869,7 @@ __global__ void __launch_bounds__(1024) deposit_kernel(Plan P, DepArgs D) {
     __syncthreads();
     const unsigned idx = __builtin_amdgcn_readfirstlane(s_item);
     if (idx >= n_items) break;
-    const Item it = D.items[idx];
+    const Item it = D.work[idx];
     const int t = __builtin_amdgcn_readfirstlane(it.tile);
     const int g = __builtin_amdgcn_readfirstlane(P.tile_grid[t]);
     const GridDesc G = P.grids[g];
@@ -996,7 +1041,7 @@ __global__ void __launch_bounds__(1024) deposit_counts(Plan P, DepArgs D) {
     __syncthreads();
     const unsigned idx = __builtin_amdgcn_readfirstlane(s_item);
     if (idx >= n_items) break;
-    const Item it = D.items[idx];
+    const Item it = D.work[idx];
     const int t = __builtin_amdgcn_readfirstlane(it.tile);
     const int g = __builtin_amdgcn_readfirstlane(P.tile_grid[t]);
     const GridDesc& G = P.grids[g];
@@ -2218,6 +2263,15 @@ hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int ch
                              const Counters* C, hipStream_t s) {
   plan_write<<<grid_for(ntiles, 256, 1 << 30), 256, 0, s>>>(start, ntiles, chunk, chunk_wide, item_off, items,
                                                            split_tiles, n_split, C);
+  return hipGetLastError();
+}
+
+// n < 0: the items that the gate admitted, at most n_max
+hipError_t launch_order_items(const Item* items, Item* work, long long n, long long n_max, Counters* C, int cus,
+                              hipStream_t s) {
+  const int grid = grid_for(std::max(n_max, 1ll), 1024, cus);
+  order_items<<<grid, 256, 0, s>>>(items, work, n, C, 0);
+  order_items<<<grid, 256, 0, s>>>(items, work, n, C, 1);
   return hipGetLastError();
 }
 

@@ -29,6 +29,8 @@ hipError_t launch_plan_count(const unsigned long long* start, int ntiles, int ch
 hipError_t launch_plan_write(const unsigned long long* start, int ntiles, int chunk, int chunk_wide,
                              const unsigned long long* item_off, Item* items, int* split_tiles, unsigned* n_split,
                              const Counters* C, hipStream_t s);
+hipError_t launch_order_items(const Item* items, Item* work, long long n, long long n_max, Counters* C, int cus,
+                              hipStream_t s);
 hipError_t launch_gate(const unsigned long long* tot_entries, const unsigned long long* item_off, int ntiles,
                        unsigned long long cap_entries, unsigned long long cap_items, Counters* C, hipStream_t s);
 bool tile_shape_supported(const int t[3]);
