@@ -172,13 +172,13 @@ def roofline_block(spec, args, st, n, P, avg, med, ms_step):
     return {
         "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-        "kernel": "the whole build step (binning, deposit, split tiles, grid sums), device time",
+        "kernel": "the whole build step (binning, deposit, tile exchange, grid sums), device time",
         "algorithmic_bytes": b_fwd, "avg_ms": t_step, "median_ms": med["ms_total"],
         "wall_ms_per_step": ms_step,
         "b_min": b_min, "b_min_frac": b_min / (t_step * 1e-3) / 1e9 / HBM_PEAK_GBS,
         "n_pairs": int(n_pairs), "n_entries": int(n_entries), "n_cells": int(n_cells),
         "phase_ms": avg, "phase_ms_median": med,
-        "deposit_phase": {"kernels": "deposit kernels + split_reduce", "algorithmic_bytes": b_dep,
+        "deposit_phase": {"kernels": "deposit kernels", "algorithmic_bytes": b_dep,
                           "avg_ms": dep_ms, "achieved": b_dep / (dep_ms * 1e-3) / 1e9,
                           "frac": b_dep / (dep_ms * 1e-3) / 1e9 / HBM_PEAK_GBS},
     }
