@@ -863,6 +863,11 @@ static asohf_status prepare_args(asohf_ctx* ctx, const asohf_opts& o, const Part
   a.item_off = ctx->item_off.as<unsigned long long>();
   a.grid_mass = grid_mass;
   a.chunk = std::max(ctx->tune.chunk, 64);
+  // a small TSC build has few items: shorter ones occupy more of the chip (exact
+  // sums only, which may split anywhere).  13,824 particles 134 -> 118 us, 60,000
+  // 158 -> 124, 250,000 197 -> 164, 500,000 261 -> 222; from a million on nothing,
+  // and nothing in table mode, whose emission has units of its own
+  while (a.P.mode == 2 && a.red == 0 && a.chunk > 1024 && A.n * 2 < (long long)ctx->cus * a.chunk) a.chunk /= 2;
   // wide table-mode entries: a tile's classes are deposited in the
   // histogram form (a fixed cost per tile and class) when one work item
   // holds all of the tile's wide entries, otherwise (and for the widest
